@@ -51,7 +51,7 @@ def build_reference() -> bool:
     are present), and of the reference program with its compresid replaced
     by this library (needs the library built first).  Returns False when
     there is nothing to build."""
-    if not os.path.isdir("/root/reference"):
+    if not os.path.isdir("/root/reference") or not os.listdir("/root/reference"):
         return False
     subprocess.run(["make", "-s", "-f", os.path.join(REPO, "oracle", "ref.mk"), "all", "dropin"],
                    check=True, cwd=REPO, stdout=subprocess.DEVNULL)

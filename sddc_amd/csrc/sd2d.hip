@@ -401,14 +401,15 @@ static hipError_t launch_vis_n(sd2d_ctx *c, const double *qin) {
   va.qin = qin; va.ftab = c->ftab; va.met = c->met; va.metw = c->metw;
   va.gq = c->gq; va.dei = c->dei; va.visres = c->visres;
   va.mu = c->p.mu; va.eta0 = c->p.eta0;
-  va.ncell = c->ncell; va.ntile = c->ntile; va.walls = c->dei != nullptr; va.s2c = c->s2c;
-  constexpr size_t lds = vis_lds_bytes<N>();
-  static_assert(lds <= 65536, "viscous kernel LDS above 64 KiB");
-  hipLaunchKernelGGL(vis_grad_kernel<N>, dim3(c->ntile), dim3(STAGE_THREADS), lds, c->stream,
+  va.ntile = c->ntile; va.walls = c->dei != nullptr; va.tinfo = c->tinfo; va.sfam = c->sfam;
+  constexpr size_t lg = vis_grad_lds_bytes<N>(), lf = vis_flux_lds_bytes<N>();
+  static_assert(lg <= 65536 && lf <= 65536, "viscous kernel LDS above 64 KiB");
+  hipLaunchKernelGGL(vis_grad_kernel<N>, dim3(c->ntile), dim3(STAGE_THREADS), lg, c->stream,
                      va, c->ops, c->ph);
   hipError_t r = hipGetLastError();
   if (r != hipSuccess) return r;
-  hipLaunchKernelGGL(vis_flux_kernel<N>, dim3(c->ntile), dim3(STAGE_THREADS), lds, c->stream,
+  va.rev = 1;   // start on the tiles the gradient kernel wrote last
+  hipLaunchKernelGGL(vis_flux_kernel<N>, dim3(c->ntile), dim3(STAGE_THREADS), lf, c->stream,
                      va, c->ops, c->ph);
   return hipGetLastError();
 }

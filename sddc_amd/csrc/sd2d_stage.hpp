@@ -347,8 +347,10 @@ __device__ __forceinline__ void neighbour_line(int kn, int nfp, int &p0, int &st
 // the same tile, nothing is read here: lci returns its index in the tile
 // and the trace is formed from the staged tile by face_trace_lds.
 // The face-table words (neighbour base, info) of end face `rfp` of a line.
-template <int N>
-__device__ __forceinline__ void face_words(const StageArgs &a, int tile, int ci, int fam, int line,
+// (A is StageArgs, or another kernel's arguments with the same ftab and, for
+// the gathers, qin.)
+template <int N, typename A>
+__device__ __forceinline__ void face_words(const A &a, int tile, int ci, int fam, int line,
                                            int rfp, int &nbase, int &info) {
   constexpr int T = Geo<N>::CPW;
   int k, nfp;
@@ -358,33 +360,6 @@ __device__ __forceinline__ void face_words(const StageArgs &a, int tile, int ci,
   info = ft[T];
 }
 
-// The gather of face_gather from already loaded face-table words.
-template <int N, typename R, typename OP>
-__device__ __forceinline__ void face_gather_w(const StageArgs &a, const OP &ops, int tile, int fam,
-                                              int line, int rfp, int nbase, int info, R *Qn,
-                                              int &lci) {
-  constexpr int T = Geo<N>::CPW, N2 = Geo<N>::N2, QT = Geo<N>::QT;
-  int k, nfp;
-  end_face<N>(fam, line, rfp, k, nfp);
-  lci = -1;
-  if (((info >> 3) & 7) == FT_INTERIOR) {
-    const int ntile = nbase / QT;
-    if (ntile == tile) {
-      lci = nbase - tile * QT;
-    } else {
-      const int nci = nbase - ntile * QT;
-      int p0, stride;
-      bool endN;
-      neighbour_line<N>(info & 3, nfp, p0, stride, endN);
-      R Lr[N];
-#pragma unroll
-      for (int s = 0; s < N; ++s) Lr[s] = endN ? ops.L[N][s] : ops.L[0][s];
-      line_vals<N, R>(a.qin + (size_t)ntile * QT, p0, stride, nci,
-                      [&](int v, const R *vals) { Qn[v] = line_trace<N, R>(vals, Lr); });
-    }
-  }
-}
-
 // The gathers of both end faces of a line from loaded face-table words, in
 // as few passes as the wave needs: pass 1 gathers, in every lane, the first
 // end face whose neighbour lies in another tile; pass 2 the N end of the
@@ -392,8 +367,8 @@ __device__ __forceinline__ void face_gather_w(const StageArgs &a, const OP &ops,
 // (a line family whose neighbours are mostly in the tile: only the lanes of
 // the strip's end cells gather) pass 2 is skipped, which halves its gather
 // loads.  Each face's trace is formed exactly as by face_gather_w.
-template <int N, typename R, typename OP>
-__device__ __forceinline__ void face_gather_pair(const StageArgs &a, const OP &ops, int tile,
+template <int N, typename R, typename A, typename OP>
+__device__ __forceinline__ void face_gather_pair(const A &a, const OP &ops, int tile,
                                                  int fam, int line, int nb0, int info0, int nbN,
                                                  int infoN, R *qn0, R *qnN, int &lci0,
                                                  int &lciN) {
@@ -425,21 +400,6 @@ __device__ __forceinline__ void face_gather_pair(const StageArgs &a, const OP &o
     }
   }
   if (g0 && gN) gather(N, nbN, infoN, qnN);
-}
-
-// Gather for an end face: the face-table info word and, for an interior or
-// periodic face, the neighbour's trace Qn at the shared face point (its
-// line through that point, interpolated with the same arithmetic as the
-// own trace: interfaceflux_all.f90:59-76).  When the neighbour cell is in
-// the same tile, nothing is read here: lci returns its index in the tile
-// and the trace is formed from the staged tile by face_trace_lds.
-template <int N, typename R, typename OP>
-__device__ __forceinline__ int face_gather(const StageArgs &a, const OP &ops, int tile, int ci,
-                                           int fam, int line, int rfp, R *Qn, int &lci) {
-  int nbase, info;
-  face_words<N>(a, tile, ci, fam, line, rfp, nbase, info);
-  face_gather_w<N, R>(a, ops, tile, fam, line, rfp, nbase, info, Qn, lci);
-  return info;
 }
 
 // The neighbour's trace for a neighbour in the same tile, from the staged
@@ -792,12 +752,18 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
       // the energy and psi only their own update
       load_vars<N, 0, 8>(qs, p, ci, q);
       if (V1 == 9) q[8] = qs[qo<N>(8, p, ci)];
+      // the viscous divergence (of variables 0-7; psi has none)
+      double vr[9];
+      if (VIS) {
+        load_vars<N, V0, (V1 < 8 ? V1 : 8)>(a.visres + (size_t)tile * G::QT, p, ci, vr + V0);
+        vr[8] = 0.0;
+      }
 #pragma unroll
       for (int v = V0; v < V1; ++v) {
         // resid = -(dF/dxi + dG/deta) / J   (compresid.f90:41,56), with the
         // viscous divergence added before the scaling (compresid.f90:43-46)
         if (VIS)
-          R[v] = (a.visres[(size_t)tile * G::QT + qo<N>(v, p, ci)] - D[s][v]) * ji;
+          R[v] = (vr[v] - D[s][v]) * ji;
         else
           R[v] = -D[s][v] * ji;
       }

@@ -7,25 +7,24 @@
 // and a cotangent Rbar, the kernels accumulate
 //   Qbar += (dR/dQ)^T Rbar,  and the partial sums of
 //   c_hbar = (dR/dc_h)^T Rbar and pbar = (dR/d free stream)^T Rbar.
-// Reverse sweep, written by hand over the structure of the forward kernel:
-//   adj_point_kernel  per solution point: resid = -(dF/dxi + dG/deta)/J -
-//                     Powell(divB) - alpha psi, reversed: the cotangent of
-//                     the flux derivatives Dbar = -Rbar/J and of the divB
-//                     weight wbar = (dR/d divB)^T Rbar / J, and the direct
-//                     (pointwise) part of Qbar;
-//   adj_line_kernel   per grid line and flux point: the cotangent of the
-//                     flux there (Mmat^T Dbar along the line) goes through
-//                     the transposed Jacobian of the interior flux, of the
-//                     Rusanov flux at faces (with the neighbour's own
-//                     cotangent of the same face flux, gathered from its
-//                     line, so each cell updates only its own Qbar) or of
-//                     the boundary flux with its ghost state; the divB
-//                     weights of the averaged face states likewise; the
-//                     trace cotangents go back to the solution points
-//                     through Lmat^T.
-// The local Jacobians come from the same physics templates instantiated
-// with dual numbers (sd2d_dual.hpp), one input direction per evaluation.
-// The AV sensor does not act on the state and has no adjoint.
+// adj_stage_kernel does the whole reverse sweep of one evaluation in one pass
+// over the tiles, written by hand over the structure of the forward kernel:
+//   - per solution point, resid = -(dF/dxi + dG/deta)/J - Powell(divB) -
+//     alpha psi reversed: the cotangent of the flux derivatives
+//     Dbar = -Rbar/J, that of the divB weight wbar = (dR/d divB)^T Rbar / J,
+//     and the direct (pointwise) part of Qbar;
+//   - per grid line and flux point, the cotangent of the flux there
+//     (Mmat^T Dbar along the line) through the transposed Jacobian of the
+//     interior flux, of the Rusanov flux at faces (with the neighbour's own
+//     cotangent of the same face flux, formed from its line, so each cell
+//     updates only its own Qbar) or of the boundary flux with its ghost
+//     state; the divB weights of the averaged face states likewise; the
+//     trace cotangents go back to the line's points through Lmat^T.
+// With Rbar = rscale * (cotangent of the stage's output) it is also the
+// reverse of the Runge-Kutta stage Qout = cin Qin + ca Qaux + b dt R(Qin).
+// The running maxima behind c_h are differentiated by adj_tail_kernel with
+// the forward's physics on dual numbers (sd2d_dual.hpp), one input direction
+// per lane.  The AV sensor does not act on the state and has no adjoint.
 #pragma once
 #include "sd2d_dual.hpp"
 #include "sd2d_stage.hpp"
@@ -34,32 +33,33 @@ namespace sd2d {
 
 struct AdjArgs {
   const double *q;         // state the residual is taken of (tile layout)
-  const double *rbar;      // cotangent of the residual (tile layout)
-  double rscale;           // the cotangent used is rscale * rbar
+  const double *rbar;      // cotangent of the stage's output (tile layout)
+  double rscale;           // that of the residual is rscale * rbar
+  double cin, ca;          // qbar gets cin * rbar besides, abar ca * rbar
   const double *divb;      // divB of q per solution point [tile][p][ci]
   const double *met;
   const int *ftab;
-  const int *s2c;
+  const int *tinfo;        // per tile: member << 6 | valid cells
   const Phys *phm;         // free stream
   const double *gm;        // eigvmax_g, umax_g that the evaluation's c_h came from
-  double *g;               // [tile][k*N2 + p][ci]: k < 9 Dbar, k = 9 wbar
-  double *qbar;            // accumulated (tile layout)
+  double *qbar, *abar;     // cotangents of Qin and Qaux (abar may be null)
+  int qadd, aadd;          // add to what they hold (else overwrite it)
   double *part;            // per tile: c_hbar, pbar[6] (rinf pinf uinf vinf bx by)
   double alpha;
-  int ncell, ntile;
+  int ntile;
 };
 
 constexpr int ADJ_NPART = 7;
 
+// LDS (in doubles): the tile's state and Rbar (qo layout), after the line
+// sweeps the cotangents the families hand each other (variables 0-3 for the
+// xi-lines, 4-8 for the eta-lines), and the reduction slots.
 template <int N> struct AdjLds {
-  static constexpr int T = Geo<N>::CPW, NF = N + 1;
-  // trace cotangents [fam][line][rfp][v][ci], then the reduction slots
-  static __device__ __forceinline__ int at(int fam, int line, int r, int v, int ci) {
-    return (((fam * N + line) * NF + r) * 9 + v) * T + ci;
-  }
-  static constexpr int RED = 2 * N * NF * 9 * T;
-  static constexpr int OPS = RED + ADJ_NPART * (STAGE_THREADS / 64);
-  static constexpr int TOTAL = OPS + (int)(sizeof(Ops) / sizeof(double));
+  static constexpr int T = Geo<N>::CPW, N2 = N * N;
+  static constexpr int Q0 = 0, R0 = 9 * N2 * T;
+  static constexpr int XA = 0, XB = 5 * N2 * T;
+  static constexpr int RED = 18 * N2 * T;
+  static constexpr int TOTAL = RED + ADJ_NPART * (STAGE_THREADS / 64);
 };
 
 // The operators copied to LDS, where the reverse sweeps index their rows
@@ -76,74 +76,6 @@ __device__ __forceinline__ const Ops &ops_to_lds(double *lds, const Ops &ops) {
 
 template <int N>
 constexpr size_t adj_lds_bytes() { return sizeof(double) * AdjLds<N>::TOTAL; }
-
-// ---- per solution point ------------------------------------------------------
-// Forward (stage kernel, points step): R = -D/J, then
-//   R1..3 -= divB*B, R4 -= divB*(u.B), R5..7 -= divB*u, R8 -= alpha*psi,
-// divB = db/J with db the summed divB-weight derivatives.
-template <int N>
-__global__ __launch_bounds__(STAGE_THREADS) void adj_point_kernel(AdjArgs a) {
-  using G = Geo<N>;
-  constexpr int T = G::CPW, N2 = G::N2;
-  const int tile = blockIdx.x;
-  const double *mt = a.met + (size_t)tile * G::NM * T;
-  for (int i = threadIdx.x; i < N2 * T; i += STAGE_THREADS) {
-    const int p = i / T, ci = i % T;
-    const int slot = tile * T + ci;
-    const int cell = a.s2c[slot];
-    if (cell < 0) continue;   // padding slot
-    const int is = p % N, js = p / N;
-    const double ji = mt[(G::JI + js + N * is) * T + ci];
-    const size_t off = (size_t)tile * G::QT;
-    double q[9], rb[9];
-#pragma unroll
-    for (int v = 0; v < 9; ++v) {
-      q[v] = a.q[off + qo<N>(v, p, ci)];
-      rb[v] = a.rscale * a.rbar[off + qo<N>(v, p, ci)];
-    }
-    const double divB = a.divb[(size_t)tile * N2 * T + (size_t)p * T + ci];
-    const double ri = 1.0 / q[0];
-    const double ux = q[1] * ri, uy = q[2] * ri, uz = q[3] * ri;
-    // cotangent of divB
-    const double dd = -(rb[1] * q[5] + rb[2] * q[6] + rb[3] * q[7] +
-                        rb[4] * (ux * q[5] + uy * q[6] + uz * q[7]) + rb[5] * ux + rb[6] * uy +
-                        rb[7] * uz);
-    double *gp = a.g + (size_t)tile * 10 * N2 * T + ci;
-#pragma unroll
-    for (int v = 0; v < 9; ++v) gp[(size_t)(v * N2 + p) * T] = -ji * rb[v];
-    gp[(size_t)(9 * N2 + p) * T] = ji * dd;
-    // direct part: Powell source and GLM damping at the point
-    double qb[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    qb[5] = -divB * (rb[1] + rb[4] * ux);
-    qb[6] = -divB * (rb[2] + rb[4] * uy);
-    qb[7] = -divB * (rb[3] + rb[4] * uz);
-    const double ubx = -divB * (rb[4] * q[5] + rb[5]);
-    const double uby = -divB * (rb[4] * q[6] + rb[6]);
-    const double ubz = -divB * (rb[4] * q[7] + rb[7]);
-    qb[1] = ubx * ri;
-    qb[2] = uby * ri;
-    qb[3] = ubz * ri;
-    qb[0] = -(ubx * ux + uby * uy + ubz * uz) * ri;
-    qb[8] = -a.alpha * rb[8];
-#pragma unroll
-    for (int v = 0; v < 9; ++v) a.qbar[off + qo<N>(v, p, ci)] += qb[v];
-  }
-}
-
-// Cotangent of the flux and of the divB weight at flux point r of a line:
-// Mmat^T applied to the line's Dbar / wbar (g at the cell `gb`).
-template <int N>
-__device__ __forceinline__ void adj_flux_cot(const double *gb, int p0, int ps, int r,
-                                             const Ops &ops, double *Fb, double &Wb) {
-  constexpr int T = Geo<N>::CPW, N2 = Geo<N>::N2;
-#pragma unroll
-  for (int v = 0; v < 10; ++v) {
-    double acc = 0.0;
-#pragma unroll
-    for (int s = 0; s < N; ++s) acc += ops.M[r][s] * gb[(size_t)(v * N2 + p0 + ps * s) * T];
-    if (v < 9) Fb[v] = acc; else Wb = acc;
-  }
-}
 
 // Trace of the 9 variables along the line through point p0 (stride ps) of
 // the slot `base` = tile * QT + ci (the face-table encoding) of the
@@ -168,7 +100,7 @@ __device__ __forceinline__ void adj_trace(const double *q, int base, int p0, int
 // (dF/dc_h)^T Fb, the forward values being formed as iflux_n / rusanov
 // form them.  Derivatives of |x| take the sign of x (+1 at 0), of sqrt(x)
 // 1/(2 sqrt(x)), as the dual numbers of sd2d_dual.hpp do; the running
-// maxima outputs are not differentiated here (adj_argmax_kernel).
+// maxima outputs are not differentiated here (adj_tail_kernel).
 
 // iflux_n (getrusanov.f90:127-193 contracted with (sx, sy))
 __device__ __forceinline__ void iflux_n_vjp(const double *q, double c_h, double sx, double sy,
@@ -268,27 +200,32 @@ __device__ __forceinline__ void rusanov_side_vjp(const double *Q, double ux, dou
 }
 
 // rusanov (getrusanov.f90:1-125): Fn = sc (Fl + Fr - ev (QR - QL)) with the
-// fast magneto-acoustic speed ev of the averaged state; QLb, QRb are set
-__device__ __forceinline__ void rusanov_vjp(const double *QL, const double *QR, double nx,
-                                            double ny, int sign_l, double c_h, const double *Fnb,
-                                            double *QLb, double *QRb, double &chb) {
+// fast magneto-acoustic speed ev of the averaged state.  The cotangent of
+// one side, or with BOTH of both: Qa is the side wanted (the left state when
+// aleft), Qb the other; Fnb is the cotangent of Fn.  chb receives the c_h
+// part of the sides that are formed.
+template <bool BOTH>
+__device__ __forceinline__ void rusanov_vjp(const double *Qa, const double *Qb, bool aleft,
+                                            double nx, double ny, int sign_l, double c_h,
+                                            const double *Fnb, double *Qab, double *Qbb,
+                                            double &chb) {
   constexpr double g1 = GAM - 1.0;
   const double mag = sqrt(nx * nx + ny * ny);
   const double im = double(sign_l) * rcp(mag);
   const double ux = nx * im, uy = ny * im;
-  const double ril = rcp(QL[0]), rir = rcp(QR[0]);
-  const double ul = ril * QL[1], vl = ril * QL[2], wl = ril * QL[3];
-  const double ur = rir * QR[1], vr = rir * QR[2], wr = rir * QR[3];
-  const double B2l = QL[5] * QL[5] + QL[6] * QL[6] + QL[7] * QL[7];
-  const double B2r = QR[5] * QR[5] + QR[6] * QR[6] + QR[7] * QR[7];
-  const double pgl = g1 * (QL[4] - 0.5 * QL[0] * (ul * ul + vl * vl + wl * wl) - B2l * 0.5 -
-                           0.5 * QL[8] * QL[8]);
-  const double pgr = g1 * (QR[4] - 0.5 * QR[0] * (ur * ur + vr * vr + wr * wr) - B2r * 0.5 -
-                           0.5 * QR[8] * QR[8]);
-  const double Vnl = ul * ux + vl * uy, Vnr = ur * ux + vr * uy;
-  const double bx = 0.5 * (QL[5] + QR[5]), by = 0.5 * (QL[6] + QR[6]), bz = 0.5 * (QL[7] + QR[7]);
-  const double irs = rcp(QL[0] + QR[0]);
-  const double ca = GAM * (pgl + pgr) * irs;
+  const double ria = rcp(Qa[0]), rib = rcp(Qb[0]);
+  const double ua = ria * Qa[1], va = ria * Qa[2], wa = ria * Qa[3];
+  const double ub = rib * Qb[1], vb = rib * Qb[2], wb = rib * Qb[3];
+  const double B2a = Qa[5] * Qa[5] + Qa[6] * Qa[6] + Qa[7] * Qa[7];
+  const double B2b = Qb[5] * Qb[5] + Qb[6] * Qb[6] + Qb[7] * Qb[7];
+  const double pga = g1 * (Qa[4] - 0.5 * Qa[0] * (ua * ua + va * va + wa * wa) - B2a * 0.5 -
+                           0.5 * Qa[8] * Qa[8]);
+  const double pgb = g1 * (Qb[4] - 0.5 * Qb[0] * (ub * ub + vb * vb + wb * wb) - B2b * 0.5 -
+                           0.5 * Qb[8] * Qb[8]);
+  const double sV = (ua * ux + va * uy) + (ub * ux + vb * uy);
+  const double bx = 0.5 * (Qa[5] + Qb[5]), by = 0.5 * (Qa[6] + Qb[6]), bz = 0.5 * (Qa[7] + Qb[7]);
+  const double irs = rcp(Qa[0] + Qb[0]);
+  const double ca = GAM * (pga + pgb) * irs;
   const double bb = bx * bx + by * by + bz * bz;
   const double cd = 2.0 * bb * irs;
   const double bn = bx * ux + by * uy;
@@ -296,20 +233,22 @@ __device__ __forceinline__ void rusanov_vjp(const double *QL, const double *QR, 
   const double cad = ca + cd;
   const double ct = sqrt(cad * cad - 4.0 * ca * cn);
   const double cf = sqrt(0.5 * (cad + ct));
-  const double sV = Vnl + Vnr;
   const double ev = 0.5 * fabs(sV) + cf;
   const double sc = 0.5 * mag * double(sign_l);
+  // QR - QL is sg (Qb - Qa)
+  const double sg = aleft ? 1.0 : -1.0;
   double G[9], evb = 0.0;
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
     G[k] = sc * Fnb[k];
-    evb -= G[k] * (QR[k] - QL[k]);
-    QLb[k] = G[k] * ev;
-    QRb[k] = -G[k] * ev;
+    evb -= G[k] * (Qb[k] - Qa[k]);
+    Qab[k] = sg * G[k] * ev;
+    if (BOTH) Qbb[k] = -sg * G[k] * ev;
   }
-  // ev = |Vnl + Vnr|/2 + cf, cf = sqrt((cad + ct)/2), ct = sqrt(cad^2 - 4 ca cn)
+  evb *= sg;
+  // ev = |Vn_l + Vn_r|/2 + cf, cf = sqrt((cad + ct)/2), ct = sqrt(cad^2 - 4 ca cn)
   const double sb = 0.5 * (sV < 0.0 ? -evb : evb);
-  const double yb = evb / (2.0 * cf);
+  const double yb = 0.5 * evb * rcp(cf);
   double cadb = 0.5 * yb;
   const double ctb = 0.5 * yb;
   const double zb = ctb / (2.0 * ct);
@@ -318,174 +257,388 @@ __device__ __forceinline__ void rusanov_vjp(const double *QL, const double *QR, 
   const double cnb = -4.0 * ca * zb;
   const double cdb = cadb;
   const double bnb = 4.0 * bn * irs * cnb;
-  double irsb = 2.0 * bn * bn * cnb + 2.0 * bb * cdb + GAM * (pgl + pgr) * cab;
-  const double bxb = bnb * ux + 4.0 * bx * irs * cdb;
-  const double byb = bnb * uy + 4.0 * by * irs * cdb;
-  const double bzb = 4.0 * bz * irs * cdb;
-  const double pgb = GAM * irs * cab;
+  const double irsb = 2.0 * bn * bn * cnb + 2.0 * bb * cdb + GAM * (pga + pgb) * cab;
+  const double h5 = 0.5 * (bnb * ux + 4.0 * bx * irs * cdb);
+  const double h6 = 0.5 * (bnb * uy + 4.0 * by * irs * cdb);
+  const double h7 = 0.5 * (4.0 * bz * irs * cdb);
+  const double pb = GAM * irs * cab;
   const double d0 = -irs * irs * irsb;
-  QLb[0] += d0; QRb[0] += d0;
-  QLb[5] += 0.5 * bxb; QRb[5] += 0.5 * bxb;
-  QLb[6] += 0.5 * byb; QRb[6] += 0.5 * byb;
-  QLb[7] += 0.5 * bzb; QRb[7] += 0.5 * bzb;
-  rusanov_side_vjp(QL, ux, uy, c_h, G, pgb, sb, QLb, chb);
-  rusanov_side_vjp(QR, ux, uy, c_h, G, pgb, sb, QRb, chb);
+  Qab[0] += d0; Qab[5] += h5; Qab[6] += h6; Qab[7] += h7;
+  rusanov_side_vjp(Qa, ux, uy, c_h, G, pb, sb, Qab, chb);
+  if (BOTH) {
+    Qbb[0] += d0; Qbb[5] += h5; Qbb[6] += h6; Qbb[7] += h7;
+    rusanov_side_vjp(Qb, ux, uy, c_h, G, pb, sb, Qbb, chb);
+  }
 }
 
-// The trace cotangent of flux point r of a line (own side only), and the
-// c_h / free-stream partial sums of the points this cell owns.
-template <int N>
-__device__ void adj_point_flux(const AdjArgs &a, const Ops &ops, double c_h, int tile, int ci,
-                               int fam, int line, int r, double *Qt, double &chb, double *pb) {
-  using G = Geo<N>;
-  constexpr int T = G::CPW, N2 = G::N2, NF = N + 1, QT = G::QT;
-  const int p0 = fam ? line : N * line, ps = fam ? N : 1;
-  const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;
-  const double *mt = a.met + (size_t)tile * G::NM * T + ci;
-  const double sx = mt[(mx + r + NF * line) * T], sy = mt[(my + r + NF * line) * T];
-  double Lr[N];
+// The ghost state of a boundary face (bc_ghost_p with vismode 1) backwards:
+// the ghost's cotangent gb goes to the own trace t (added to ob) and to the
+// free stream pb[6] (rinf pinf uinf vinf bx by).
+__device__ __forceinline__ void bc_ghost_vjp(int bc, const double *t, double nx, double ny,
+                                             const Phys &ph, const double *gb, double *ob,
+                                             double *pb) {
+  constexpr double ig1 = 1.0 / (GAM - 1.0);
+  const double ri = rcp(t[0]);
+  const double uw = t[1] * ri, vw = t[2] * ri, ww = t[3] * ri;
+  if (bc == FT_INLE) {
+    pb[0] += gb[0] + gb[1] * ph.uinf + gb[2] * ph.vinf +
+             gb[4] * 0.5 * (ph.uinf * ph.uinf + ph.vinf * ph.vinf);
+    pb[2] += ph.rinf * (gb[1] + gb[4] * ph.uinf);
+    pb[3] += ph.rinf * (gb[2] + gb[4] * ph.vinf);
+    ob[8] += gb[8] + gb[4] * t[8];
+  } else if (bc == FT_OUTL) {
+    ob[0] += gb[0] - gb[4] * 0.5 * (uw * uw + vw * vw);
+    ob[1] += gb[1] + gb[4] * uw;
+    ob[2] += gb[2] + gb[4] * vw;
+    ob[8] += gb[4] * t[8];
+  } else if (bc == FT_WALL) {
+    ob[0] += gb[0]; ob[1] -= gb[1]; ob[2] -= gb[2]; ob[3] -= gb[3]; ob[4] += gb[4];
+    ob[5] -= gb[5]; ob[6] -= gb[6]; ob[7] -= gb[7]; ob[8] += gb[8];
+  } else if (bc == FT_SYMP) {
+    const double im = rcp(sqrt(nx * nx + ny * ny)), ex = nx * im, ey = ny * im;
+    const double vn = uw * ex + vw * ey;
+    const double ur = uw - 2.0 * vn * ex, vr = vw - 2.0 * vn * ey;
+    const double rs = 2.0 * ph.rinf - t[0];
+    // ghost momenta rs (ur, vr, -ww) and energy with |m|^2 / (2 rs)
+    const double m1 = gb[1] + gb[4] * ur, m2 = gb[2] + gb[4] * vr, m3 = gb[3] - gb[4] * ww;
+    const double rsb = gb[0] - 0.5 * gb[4] * (ur * ur + vr * vr + ww * ww) + m1 * ur + m2 * vr -
+                       m3 * ww;
+    const double urb = m1 * rs, vrb = m2 * rs, wwb = -m3 * rs;
+    const double nb = 2.0 * (urb * ex + vrb * ey);   // the reflection is symmetric
+    const double uwb = urb - nb * ex, vwb = vrb - nb * ey;
+    ob[0] += -rsb - (uwb * uw + vwb * vw + wwb * ww) * ri;
+    ob[1] += uwb * ri;
+    ob[2] += vwb * ri;
+    ob[3] += wwb * ri;
+    ob[7] += gb[4] * t[7] - gb[7];
+    ob[8] += gb[8] + gb[4] * t[8];
+    pb[0] += 2.0 * rsb;
+  } else {   // FREE
 #pragma unroll
-  for (int s = 0; s < N; ++s) Lr[s] = ops.L[r][s];
-  double t[9], Fb[9], Wb;
-  adj_trace<N>(a.q, tile * QT + ci, p0, ps, Lr, t);
-  adj_flux_cot<N>(a.g + (size_t)tile * 10 * N2 * T + ci, p0, ps, r, ops, Fb, Wb);
-  if (r != 0 && r != N) {
-    // interior flux point (compflux.f90:53-104) and the divB weight of the trace
-    iflux_n_vjp(t, c_h, sx, sy, Fb, Qt, chb);
-    Qt[5] += Wb * sx;
-    Qt[6] += Wb * sy;
-    return;
+    for (int v = 0; v < 9; ++v) ob[v] += gb[v];
   }
-  int k, nfp;
-  end_face<N>(fam, line, r, k, nfp);
-  const int *ft = a.ftab + ((size_t)tile * 8 + k * 2) * T + ci;
-  const int nbase = ft[0], info = ft[T];
-  const int bc = (info >> 3) & 7;
-  const int own_sl = (k == 0 || k == 3) ? -1 : 1;
-  if (bc == FT_INTERIOR) {
-    // the face as interfaceflux / CYCLOCFLUX evaluate it, and the
-    // neighbour's cotangent of its own copy of the face flux
-    const int kn = info & 3, left = (info >> 2) & 1, sneg = (info >> 6) & 1;
-    const int nt = nbase / QT, nci = nbase - nt * QT;
-    int np0, nst;
-    bool endN;
-    neighbour_line<N>(kn, nfp, np0, nst, endN);
-    double Ln[N];
+  if (bc == FT_INLE || bc == FT_OUTL || bc == FT_SYMP) {
+    pb[1] += gb[4] * ig1;
+    pb[4] += gb[5] + gb[4] * ph.bxinf;
+    pb[5] += gb[6] + gb[4] * ph.byinf;
+  }
+}
+
+// Cotangent of divB at a point, (dR/d divB)^T rb: the Powell source backwards.
+__device__ __forceinline__ double adj_divb_cot(const double *q, const double *rb) {
+  const double ri = rcp(q[0]);
+  const double ux = q[1] * ri, uy = q[2] * ri, uz = q[3] * ri;
+  return -(rb[1] * q[5] + rb[2] * q[6] + rb[3] * q[7] +
+           rb[4] * (ux * q[5] + uy * q[6] + uz * q[7]) + rb[5] * ux + rb[6] * uy + rb[7] * uz);
+}
+
+// From the line of another cell through a shared face point (points p0 + ps*s
+// of slot ci, state q and cotangent r in qo layout, 1/J at ji): the state's
+// trace t with row Lr, and the cotangents of that cell's flux and divB weight
+// there, Mr^T Dbar and Mr^T wbar.
+// (is, js) of a solution point
+template <int N> __device__ __forceinline__ int pt_is(int p) { return p % N; }
+template <int N> __device__ __forceinline__ int pt_js(int p) { return p / N; }
+
+template <int N>
+__device__ __forceinline__ void adj_far_line(const double *q, const double *r, const double *ji,
+                                             int p0, int ps, int ci, const double *Lr,
+                                             const double *Mr, double rscale, double *t,
+                                             double *Fb, double &Wb) {
+  constexpr int T = Geo<N>::CPW;
 #pragma unroll
-    for (int s = 0; s < N; ++s) Ln[s] = endN ? ops.L[N][s] : ops.L[0][s];
-    double qn[9], Fnb[9], Wnb;
-    adj_trace<N>(a.q, nbase, np0, nst, Ln, qn);
-    adj_flux_cot<N>(a.g + (size_t)nt * 10 * N2 * T + nci, np0, nst, endN ? N : 0, ops, Fnb, Wnb);
-    const int sl = left ? own_sl : ((kn == 0 || kn == 3) ? -1 : 1);
-    const int sr = left ? ((kn == 1 || kn == 2) ? -1 : 1) : ((k == 1 || k == 2) ? -1 : 1);
-    const double nsg = (left || !sneg) ? 1.0 : -1.0;
-    const double fo = left ? 1.0 : double(sl * sr), fn = left ? double(sl * sr) : 1.0;
-    // the neighbour's own metric at the point is sig times this cell's
-    int sgn_nb = sneg;
-    if (left) sgn_nb = (a.ftab[((size_t)nt * 8 + kn * 2 + 1) * T + nci] >> 6) & 1;
-    const double sig = sgn_nb ? -1.0 : 1.0;
-    double Gb[9];
+  for (int v = 0; v < 9; ++v) t[v] = Fb[v] = 0.0;
+  Wb = 0.0;
 #pragma unroll
-    for (int v = 0; v < 9; ++v) Gb[v] = fo * Fb[v] + fn * Fnb[v];
-    {
-      // the face flux backwards; this cell keeps its own side's cotangent,
-      // and the left cell also takes the c_h part
-      double QLb[9], QRb[9], chf = 0.0;
-      rusanov_vjp(left ? t : qn, left ? qn : t, nsg * sx, nsg * sy, sl, c_h, Gb, QLb, QRb, chf);
+  for (int s = 0; s < N; ++s) {
+    const int p = p0 + ps * s;
+    double a[9], b[9];
+    load_vars<N, 0, 9>(q, p, ci, a);
+    load_vars<N, 0, 9>(r, p, ci, b);
+    const double c = rscale * ji[(pt_js<N>(p) + N * pt_is<N>(p)) * T] * Mr[s];
+    Wb = fma(c, adj_divb_cot(a, b), Wb);
 #pragma unroll
-      for (int v = 0; v < 9; ++v) Qt[v] = left ? QLb[v] : QRb[v];
-      if (left) chb += chf;
+    for (int v = 0; v < 9; ++v) {
+      t[v] = fma(a[v], Lr[s], t[v]);
+      Fb[v] = fma(-c, b[v], Fb[v]);
     }
-    // divB weights of the averaged state Qv = (QL + QR)/2 seen by both cells
-    const double wq = 0.5 * (Wb + sig * Wnb);
-    Qt[5] += wq * sx;
-    Qt[6] += wq * sy;
-    return;
-  }
-  // boundary face: Rusanov with the ghost state of the own trace (bcflux.f90)
-  const Phys &ph = a.phm[0];
-  const double par[6] = {ph.rinf, ph.pinf, ph.uinf, ph.vinf, ph.bxinf, ph.byinf};
-#pragma unroll 1
-  for (int kk = 0; kk < 16; ++kk) {   // 9 state, c_h, 6 free-stream directions
-    Dual Qo[9], QR[9], F[9], eig(0.0), um(0.0), pd[6];
-#pragma unroll
-    for (int v = 0; v < 9; ++v) Qo[v] = Dual(t[v], v == kk ? 1.0 : 0.0);
-#pragma unroll
-    for (int j = 0; j < 6; ++j) pd[j] = Dual(par[j], kk == 10 + j ? 1.0 : 0.0);
-    bc_ghost_p<Dual>(bc, Qo, Dual(sx), Dual(sy), pd[0], pd[1], pd[2], pd[3], pd[4], pd[5],
-                     ph.vismode, QR);
-    rusanov<Dual>(Qo, QR, Dual(sx), Dual(sy), own_sl, Dual(c_h, kk == 9 ? 1.0 : 0.0), F, eig,
-                  um);
-    double acc = 0.0;
-#pragma unroll
-    for (int v = 0; v < 9; ++v) acc += Fb[v] * F[v].d;
-    // divB weight of Qv = (Qo + ghost)/2
-    acc += Wb * 0.5 * ((Qo[5].d + QR[5].d) * sx + (Qo[6].d + QR[6].d) * sy);
-    if (kk < 9) Qt[kk] = acc;
-    else if (kk == 9) chb += acc;
-    else pb[kk - 10] += acc;
   }
 }
 
-// ---- per grid line -------------------------------------------------------------
-// Every line thread forms the trace cotangents of its N+1 flux points into
-// LDS; the xi-line threads then send both families' trace cotangents back
-// to their points through Lmat^T and add them to Qbar.
+// ---- one evaluation backwards ------------------------------------------------
+// One 128-thread workgroup per tile, one thread per grid line, one family per
+// wavefront, as in the stage kernel.  The state and Rbar of the tile are staged
+// in LDS (one wave each); the first end face of a line whose neighbour lies in
+// another tile is gathered meanwhile.  Every flux point's trace cotangent is
+// folded straight into the line's Qbar accumulators through Lmat^T; then the
+// pointwise parts and the Runge-Kutta terms are added (xi-lines variables 0-3,
+// eta-lines 4-8) and the families exchange their halves through the staging
+// area.
+// 256 VGPRs and 26-62 AGPRs (the 9 N accumulators beside the Rusanov sweep),
+// so one wave per SIMD; bound by the latency of its loads, then by FP64 issue.
+// 128 x 256 cells, N = 4: 79 us.  It replaces a point kernel, a line kernel
+// that read every flux point's lines from memory and the RK combinations
+// (31 + 150 + 2 x 19 us and a clear of the cotangent).  Held to two waves per
+// SIMD it spills (108-284 bytes a lane): 89 us at N = 4, 50 against 47 us at
+// N = 5 (64 x 128 cells), 22 against 17 us at N = 3.
 template <int N>
-__global__ __launch_bounds__(STAGE_THREADS) void adj_line_kernel(AdjArgs a, Ops ops_arg) {
+__global__ __launch_bounds__(STAGE_THREADS, 1) void adj_stage_kernel(AdjArgs a, Ops ops) {
   using G = Geo<N>;
   using LD = AdjLds<N>;
-  constexpr int T = G::CPW, N2 = G::N2, NF = N + 1, NT = 2 * N * T;
+  constexpr int T = G::CPW, N2 = G::N2, NF = N + 1, QT = G::QT;
+  static_assert(N * T <= 64 && STAGE_THREADS == 128, "one wavefront per line family");
   extern __shared__ double lds[];
-  const int tid = threadIdx.x, tile = blockIdx.x;
-  const int ci = tid % T, fl = tid / T;
-  const int fam = fl >= N ? 1 : 0, line = fl - fam * N;
-  const bool valid = tid < NT && a.s2c[tile * T + ci] >= 0;
-  const Ops &ops = ops_to_lds<LD::OPS>(lds, ops_arg);
-  const double ge = a.gm[0], gu = a.gm[1];
-  const double c_h = sqrt(ge * (ge - gu));   // as the forward forms it (compflux.f90:6)
-  double chb = 0.0, pb[6] = {0, 0, 0, 0, 0, 0};
-  if (valid) {
-#pragma unroll 1
-    for (int r = 0; r < NF; ++r) {
-      double Qt[9];
-      adj_point_flux<N>(a, ops, c_h, tile, ci, fam, line, r, Qt, chb, pb);
+  const int tid = threadIdx.x;
+  const int tile = tile_of_block(blockIdx.x, a.ntile, 0);
+  const int fam = tid >> 6, line = (tid & 63) / T, ci = (tid & 63) % T;
+  int nb0, nbN, info0, infoN;
+  face_words<N>(a, tile, ci, fam, line, 0, nb0, info0);
+  face_words<N>(a, tile, ci, fam, line, N, nbN, infoN);
+  const int ti = a.tinfo[tile];
+  {   // the xi wave stages the state, the eta wave Rbar
+    constexpr int NV2 = QT / 2, NSW = (NV2 + 63) / 64;
+    const double2 *src = reinterpret_cast<const double2 *>((fam ? a.rbar : a.q) + (size_t)tile * QT);
+    double2 *dst = reinterpret_cast<double2 *>(lds + (fam ? LD::R0 : LD::Q0));
+    const int l = tid & 63;
+    double2 st[NSW];
 #pragma unroll
-      for (int v = 0; v < 9; ++v) lds[LD::at(fam, line, r, v, ci)] = Qt[v];
+    for (int k = 0; k < NSW; ++k) {
+      const int i = l + k * 64;
+      st[k] = src[(k < NSW - 1 || i < NV2) ? i : 0];
+    }
+#pragma unroll
+    for (int k = 0; k < NSW - 1; ++k) dst[l + k * 64] = st[k];
+    if (l + (NSW - 1) * 64 < NV2) dst[l + (NSW - 1) * 64] = st[NSW - 1];
+  }
+  const bool valid = line < N && ci < (ti & 63);
+  const double *mt = a.met + (size_t)tile * G::NM * T + ci;
+  const int p0 = fam ? line : N * line, ps = fam ? N : 1;
+  const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;
+  const bool i0 = ((info0 >> 3) & 7) == FT_INTERIOR, iN = ((infoN >> 3) & 7) == FT_INTERIOR;
+  const bool far0 = i0 && nb0 / QT != tile, farN = iN && nbN / QT != tile;
+  const bool nfirst = farN && !far0;   // the end whose traces are gathered first
+  double tn[9], Fn[9], Wn = 0.0;       // neighbour's trace and cotangents at an end
+  int sgn = 0;                         // whether its stored normal is the negative
+  auto other_side = [&](bool atN, bool staged) __attribute__((always_inline)) {
+    const int rfp = atN ? N : 0, nb = atN ? nbN : nb0, info = atN ? infoN : info0;
+    const int nt = nb / QT, nci = nb - nt * QT, kn = info & 3;
+    int k, nfp, np0, nst;
+    bool endN;
+    end_face<N>(fam, line, rfp, k, nfp);
+    neighbour_line<N>(kn, nfp, np0, nst, endN);
+    double Lr[N], Mr[N];
+#pragma unroll
+    for (int s = 0; s < N; ++s) {
+      Lr[s] = endN ? ops.L[N][s] : ops.L[0][s];
+      Mr[s] = endN ? ops.M[N][s] : ops.M[0][s];
+    }
+    const double *ji = a.met + ((size_t)nt * G::NM + G::JI) * T + nci;
+    sgn = a.ftab[((size_t)nt * 8 + kn * 2 + 1) * T + nci];
+    if (staged)
+      adj_far_line<N>(lds + LD::Q0, lds + LD::R0, ji, np0, nst, nci, Lr, Mr, a.rscale, tn, Fn, Wn);
+    else
+      adj_far_line<N>(a.q + (size_t)nt * QT, a.rbar + (size_t)nt * QT, ji, np0, nst, nci, Lr, Mr,
+                      a.rscale, tn, Fn, Wn);
+  };
+  double ji[N], msx[NF], msy[NF];
+  if (valid) {
+    if (far0 || farN) other_side(nfirst, false);
+#pragma unroll
+    for (int s = 0; s < N; ++s) ji[s] = mt[(G::JI + (fam ? s : line) + N * (fam ? line : s)) * T];
+#pragma unroll
+    for (int r = 0; r < NF; ++r) {
+      msx[r] = mt[(mx + r + NF * line) * T];
+      msy[r] = mt[(my + r + NF * line) * T];
     }
   }
-  // partial sums of the block
-  {
-    constexpr int NW = STAGE_THREADS / 64;
+  const double ge = a.gm[0], gu = a.gm[1];
+  const double c_h = sqrt(ge * (ge - gu));   // as the forward forms it (compflux.f90:6)
+  const Phys &ph = a.phm[0];
+  double chb = 0.0, pb[6] = {0, 0, 0, 0, 0, 0};
+  __syncthreads();
+  double A[N][9];   // the line's part of Qbar at its points
+  const double *qs = lds + LD::Q0, *rs = lds + LD::R0;
+  if (valid) {
+    double c[N], wb[N];   // Dbar = c * rbar and wbar at the line's points
+#pragma unroll
+    for (int s = 0; s < N; ++s) {
+      double q[9], b[9];
+      load_vars<N, 0, 9>(qs, p0 + ps * s, ci, q);
+      load_vars<N, 0, 9>(rs, p0 + ps * s, ci, b);
+      c[s] = -a.rscale * ji[s];
+      wb[s] = -c[s] * adj_divb_cot(q, b);
+    }
+    // trace, flux cotangent and divB-weight cotangent at a flux point
+    auto point = [&](const double *Lr, const double *Mr, double *t, double *Fb, double &Wb) __attribute__((always_inline)) {
+      double m[N];
+      Wb = 0.0;
+#pragma unroll
+      for (int s = 0; s < N; ++s) {
+        m[s] = Mr[s] * c[s];
+        Wb = fma(Mr[s], wb[s], Wb);
+      }
+      line_vals<N, double>(qs, p0, ps, ci, [&](int v, const double *x) {
+        t[v] = line_trace<N, double>(x, Lr);
+      });
+      line_vals<N, double>(rs, p0, ps, ci, [&](int v, const double *x) {
+        Fb[v] = line_trace<N, double>(x, m);
+      });
+    };
+    auto end_point = [&](bool atN, bool gathered, double *Qt) __attribute__((always_inline)) {
+      const int rfp = atN ? N : 0, info = atN ? infoN : info0;
+      const int k = fam == 0 ? (atN ? 1 : 3) : (atN ? 2 : 0);
+      const bool inter = atN ? iN : i0, far = atN ? farN : far0;
+      const double sx = atN ? msx[N] : msx[0], sy = atN ? msy[N] : msy[0];
+      if (inter && !far) other_side(atN, true);
+      else if (far && !gathered) other_side(atN, false);
+      (void)rfp;
+      double Lo[N], Mo[N], t[9], Fb[9], Wb;
+#pragma unroll
+      for (int s = 0; s < N; ++s) {
+        Lo[s] = atN ? ops.L[N][s] : ops.L[0][s];
+        Mo[s] = atN ? ops.M[N][s] : ops.M[0][s];
+      }
+      point(Lo, Mo, t, Fb, Wb);
+      const int own_sl = (k == 0 || k == 3) ? -1 : 1;
+      if (inter) {
+        // the face as interfaceflux / CYCLOCFLUX evaluate it, with the
+        // neighbour's cotangent of its own copy of the face flux
+        const int kn = info & 3, left = (info >> 2) & 1, sneg = (info >> 6) & 1;
+        const int sl = left ? own_sl : ((kn == 0 || kn == 3) ? -1 : 1);
+        const int sr = left ? ((kn == 1 || kn == 2) ? -1 : 1) : ((k == 1 || k == 2) ? -1 : 1);
+        const double nsg = (left || !sneg) ? 1.0 : -1.0;
+        const double fo = left ? 1.0 : double(sl * sr), fn = left ? double(sl * sr) : 1.0;
+        // the neighbour's own metric at the point is sig times this cell's
+        const double sig = (left ? (sgn >> 6) & 1 : sneg) ? -1.0 : 1.0;
+        const double wq = 0.5 * (Wb + sig * Wn);
+#pragma unroll
+        for (int v = 0; v < 9; ++v) Fb[v] = fo * Fb[v] + fn * Fn[v];
+        rusanov_vjp<false>(t, tn, left, nsg * sx, nsg * sy, sl, c_h, Fb, Qt, nullptr, chb);
+        // divB weights of the averaged state (QL + QR)/2 seen by both cells
+        Qt[5] += wq * sx;
+        Qt[6] += wq * sy;
+      } else {
+        const int bc = (info >> 3) & 7;
+        double g[9], gb[9];
+        bc_ghost<double>(bc, t, sx, sy, ph, g);
+        rusanov_vjp<true>(t, g, true, sx, sy, own_sl, c_h, Fb, Qt, gb, chb);
+        const double hx = 0.5 * Wb * sx, hy = 0.5 * Wb * sy;
+        Qt[5] += hx; Qt[6] += hy;
+        gb[5] += hx; gb[6] += hy;
+        bc_ghost_vjp(bc, t, sx, sy, ph, gb, Qt, pb);
+      }
+    };
+    {
+      double QA[9], QB[9];
+      end_point(nfirst, true, QA);
+      __builtin_amdgcn_sched_barrier(0);
+      end_point(!nfirst, false, QB);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < N; ++s) {
+        const double LA = nfirst ? ops.L[N][s] : ops.L[0][s], LB = nfirst ? ops.L[0][s] : ops.L[N][s];
+#pragma unroll
+        for (int v = 0; v < 9; ++v) A[s][v] = fma(QB[v], LB, QA[v] * LA);
+      }
+    }
+    // interior flux points (compflux.f90:53-104) and the divB weight of the trace
+#pragma unroll
+    for (int r = 1; r < N; ++r) {
+      double t[9], Fb[9], Wb, Qt[9];
+      point(ops.L[r], ops.M[r], t, Fb, Wb);
+      iflux_n_vjp(t, c_h, msx[r], msy[r], Fb, Qt, chb);
+      Qt[5] = fma(Wb, msx[r], Qt[5]);
+      Qt[6] = fma(Wb, msy[r], Qt[6]);
+#pragma unroll
+      for (int s = 0; s < N; ++s)
+#pragma unroll
+        for (int v = 0; v < 9; ++v) A[s][v] = fma(Qt[v], ops.L[r][s], A[s][v]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the points' direct part (Powell source and GLM damping), cin * rbar, and
+    // the auxiliary register's cotangent, for the variables this family finishes
+    const double *dv = a.divb + (size_t)tile * N2 * T + ci;
+    auto direct = [&](auto v0c, auto v1c) __attribute__((always_inline)) {
+      constexpr int V0 = decltype(v0c)::value, V1 = decltype(v1c)::value;
+#pragma unroll
+      for (int s = 0; s < N; ++s) {
+        const int p = p0 + ps * s;
+        double q[9], b[9], d[9];
+        load_vars<N, 0, 8>(qs, p, ci, q);
+        load_vars<N, 0, 9>(rs, p, ci, b);
+        const double w = -a.rscale * dv[p * T];   // the residual's cotangent is rscale * b
+        const double ri = rcp(q[0]);
+        const double ux = q[1] * ri, uy = q[2] * ri, uz = q[3] * ri;
+        const double ubx = w * (b[4] * q[5] + b[5]), uby = w * (b[4] * q[6] + b[6]),
+                     ubz = w * (b[4] * q[7] + b[7]);
+        d[0] = -(ubx * ux + uby * uy + ubz * uz) * ri;
+        d[1] = ubx * ri;
+        d[2] = uby * ri;
+        d[3] = ubz * ri;
+        d[4] = 0.0;
+        d[5] = w * (b[1] + b[4] * ux);
+        d[6] = w * (b[2] + b[4] * uy);
+        d[7] = w * (b[3] + b[4] * uz);
+        d[8] = -a.alpha * a.rscale * b[8];
+#pragma unroll
+        for (int v = V0; v < V1; ++v) A[s][v] += d[v] + a.cin * b[v];
+        if (a.abar) {
+          double *ab = a.abar + (size_t)tile * QT;
+          double x[V1 - V0];
+          if (a.aadd) {
+            load_vars<N, V0, V1>(ab, p, ci, x);
+#pragma unroll
+            for (int v = V0; v < V1; ++v) x[v - V0] = fma(a.ca, b[v], x[v - V0]);
+          } else {
+#pragma unroll
+            for (int v = V0; v < V1; ++v) x[v - V0] = a.ca * b[v];
+          }
+          store_vars<N, V0, V1>(ab, p, ci, x);
+        }
+      }
+    };
+    if (fam == 0) direct(std::integral_constant<int, 0>{}, std::integral_constant<int, 4>{});
+    else direct(std::integral_constant<int, 4>{}, std::integral_constant<int, 9>{});
+  }
+  {   // partial sums of the block
     const int w = tid >> 6, l = tid & 63;
     double x[ADJ_NPART] = {chb, pb[0], pb[1], pb[2], pb[3], pb[4], pb[5]};
 #pragma unroll
     for (int j = 0; j < ADJ_NPART; ++j) {
       x[j] = wave_sum(x[j]);
-      if (l == 0) lds[LD::RED + j * NW + w] = x[j];
+      if (l == 0) lds[LD::RED + j * (STAGE_THREADS / 64) + w] = x[j];
+    }
+  }
+  __syncthreads();   // every read of the staged tile is done
+  if (tid < ADJ_NPART)
+    a.part[(size_t)tile * ADJ_NPART + tid] = lds[LD::RED + 2 * tid] + lds[LD::RED + 2 * tid + 1];
+  if (valid) {
+#pragma unroll
+    for (int s = 0; s < N; ++s) {
+      if (fam) xput<N, 4>(lds + LD::XA, p0 + ps * s, ci, A[s]);
+      else xput<N, 5>(lds + LD::XB, p0 + ps * s, ci, A[s] + 4);
     }
   }
   __syncthreads();
-  if (tid < ADJ_NPART) {
-    constexpr int NW = STAGE_THREADS / 64;
-    double s = 0.0;
-    for (int w = 0; w < NW; ++w) s += lds[LD::RED + tid * NW + w];
-    a.part[(size_t)tile * ADJ_NPART + tid] = s;
-  }
-  if (!valid || fam != 0) return;
-  const int js = line;
-  double *qb = a.qbar + (size_t)tile * G::QT;
+  if (!valid) return;
+  double *qb = a.qbar + (size_t)tile * QT;
+  auto finish = [&](auto v0c, auto v1c) __attribute__((always_inline)) {
+    constexpr int V0 = decltype(v0c)::value, V1 = decltype(v1c)::value;
 #pragma unroll
-  for (int is = 0; is < N; ++is)
+    for (int s = 0; s < N; ++s) {
+      const int p = p0 + ps * s;
+      xadd<N, V1 - V0>(lds + (fam ? LD::XB : LD::XA), p, ci, A[s] + V0);
+      if (a.qadd) {
+        double x[V1 - V0];
+        load_vars<N, V0, V1>(qb, p, ci, x);
 #pragma unroll
-    for (int v = 0; v < 9; ++v) {
-      double acc = 0.0;
-#pragma unroll
-      for (int r = 0; r < NF; ++r) acc += ops.L[r][is] * lds[LD::at(0, js, r, v, ci)];
-#pragma unroll
-      for (int r = 0; r < NF; ++r) acc += ops.L[r][js] * lds[LD::at(1, is, r, v, ci)];
-      qb[qo<N>(v, is + N * js, ci)] += acc;
+        for (int v = V0; v < V1; ++v) A[s][v] += x[v - V0];
+      }
+      store_vars<N, V0, V1>(qb, p, ci, A[s] + V0);
     }
+  };
+  if (fam == 0) finish(std::integral_constant<int, 0>{}, std::integral_constant<int, 4>{});
+  else finish(std::integral_constant<int, 4>{}, std::integral_constant<int, 9>{});
 }
 
 // ---- wall drag ------------------------------------------------------------------
@@ -494,39 +647,44 @@ __global__ __launch_bounds__(STAGE_THREADS) void adj_line_kernel(AdjArgs a, Ops 
 // trace, S the cell's metric vector at the point (S1(1,:) or S2(2,:),
 // whose length is the face's arc length per unit reference coordinate),
 // signed outwards, and w_i the weights of the interpolatory quadrature on
-// the solution-point positions Xs of the face.  One thread per cell: the
-// value per cell, and with qbar set, Qbar += scale * dD/dQ.
+// the solution-point positions Xs of the face.  One wave per tile, one lane
+// per line of a cell, the four faces one after the other: the drag per tile,
+// and with qbar set, Qbar += scale * dD/dQ (the lines of one face share no
+// point; a cell's next wall face comes after the barrier).
 template <int N>
-__global__ void drag_kernel(const double *q, const int *ftab, const double *met, const double *wq,
-                            Ops ops_arg, int ncell, int ntile, double *dcell, double *qbar,
-                            double scale) {
+__global__ __launch_bounds__(64) void drag_kernel(const double *q, const int *ftab,
+                                                  const double *met, const double *wq, Ops ops,
+                                                  double *dtile, double *qbar, double scale) {
   using G = Geo<N>;
-  constexpr int T = G::CPW, N2 = G::N2, NF = N + 1;
-  __shared__ double so[sizeof(Ops) / sizeof(double)];
-  const Ops &ops = ops_to_lds<0>(so, ops_arg);
-  const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= ntile * T) return;
-  const int tile = slot / T, ci = slot % T;
+  constexpr int T = G::CPW, NF = N + 1;
+  static_assert(N * T <= 64, "one lane per line");
+  const int tile = blockIdx.x, line = threadIdx.x / T, ci = threadIdx.x % T;
+  const bool on = line < N;
   double d = 0.0;
-  {   // (a padding slot has no wall face: d stays 0)
+  int bc[4];
+  bool any = false;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {   // (a padding slot has no wall face)
+    const int info = ftab[((size_t)tile * 8 + k * 2 + 1) * T + ci];
+    bc[k] = (info >> 3) & 7;
+    any |= bc[k] == FT_WALL;
+  }
+  if (__syncthreads_or(any)) {
     const double *qc = q + (size_t)tile * G::QT;
     const double *mt = met + (size_t)tile * G::NM * T + ci;
+#pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const int info = ftab[((size_t)tile * 8 + k * 2 + 1) * T + ci];
-      if (((info >> 3) & 7) != FT_WALL) continue;
-      // the face's points: own lines of the family crossing it
-      const int fam = (k == 1 || k == 3) ? 0 : 1;
-      const int rfp = (k == 0 || k == 3) ? 0 : N;
-      const int mx = fam ? G::S2X : G::S1X;
-      const double sgn = (k == 0 || k == 3) ? -1.0 : 1.0;
-      for (int line = 0; line < N; ++line) {
+      if (on && bc[k] == FT_WALL) {
+        // the face's points: own lines of the family crossing it
+        const int fam = (k == 1 || k == 3) ? 0 : 1;
+        const int rfp = (k == 0 || k == 3) ? 0 : N;
+        const int mx = fam ? G::S2X : G::S1X;
+        const double sgn = (k == 0 || k == 3) ? -1.0 : 1.0;
         const int p0 = fam ? line : N * line, ps = fam ? N : 1;
         double t[9];
-        for (int v = 0; v < 9; ++v) {
-          double acc = 0.0;
-          for (int s = 0; s < N; ++s) acc = fma(qc[qo<N>(v, p0 + ps * s, ci)], ops.L[rfp][s], acc);
-          t[v] = acc;
-        }
+        line_vals<N, double>(qc, p0, ps, ci, [&](int v, const double *x) {
+          t[v] = line_trace<N, double>(x, ops.L[rfp]);
+        });
         const double g1 = GAM - 1.0;
         const double ke = 0.5 * (t[1] * t[1] + t[2] * t[2] + t[3] * t[3]) / t[0];
         const double pr = g1 * (t[4] - ke - 0.5 * (t[5] * t[5] + t[6] * t[6] + t[7] * t[7]) -
@@ -535,24 +693,24 @@ __global__ void drag_kernel(const double *q, const int *ftab, const double *met,
         d += wq[line] * pr * nx;
         if (qbar) {
           const double c = scale * wq[line] * nx * g1;
-          double pt[9];
-          pt[0] = c * ke / t[0];
-          pt[1] = -c * t[1] / t[0];
-          pt[2] = -c * t[2] / t[0];
-          pt[3] = -c * t[3] / t[0];
-          pt[4] = c;
-          pt[5] = -c * t[5];
-          pt[6] = -c * t[6];
-          pt[7] = -c * t[7];
-          pt[8] = -c * t[8];
+          const double pt[9] = {c * ke / t[0], -c * t[1] / t[0], -c * t[2] / t[0],
+                                -c * t[3] / t[0], c, -c * t[5], -c * t[6], -c * t[7], -c * t[8]};
           double *qb = qbar + (size_t)tile * G::QT;
-          for (int v = 0; v < 9; ++v)
-            for (int s = 0; s < N; ++s) qb[qo<N>(v, p0 + ps * s, ci)] += pt[v] * ops.L[rfp][s];
+#pragma unroll
+          for (int s = 0; s < N; ++s) {
+            double x[9];
+            load_vars<N, 0, 9>(qb, p0 + ps * s, ci, x);
+#pragma unroll
+            for (int v = 0; v < 9; ++v) x[v] += pt[v] * ops.L[rfp][s];
+            store_vars<N, 0, 9>(qb, p0 + ps * s, ci, x);
+          }
         }
       }
+      if (qbar) __syncthreads();
     }
   }
-  dcell[slot] = d;
+  d = wave_sum(d);
+  if (threadIdx.x == 0) dtile[tile] = d;
 }
 
 // ---- the running maxima behind c_h -------------------------------------------------
@@ -619,63 +777,15 @@ __device__ __forceinline__ void adj_point_geom(const AdjArgs &a, const Ops &ops,
   if (((info >> 3) & 7) == FT_INTERIOR) neighbour_line<N>(info & 3, nfp, np0, nst, endN);
 }
 
-// pass 0: the maxima of eig and um over all flux points (bit patterns of
-// non-negative doubles, atomicMax); pass 1: the smallest location code
-// attaining each maximum (atomicMin)
+// Qbar += w * d(speed)/dQ at flux point `loc` (kind 0: eig, 1: um), called by
+// one block: lane kk < 9 takes variable kk of the cell's own trace, lane
+// 9 + v variable v of the neighbour's, after a barrier (on a one-cell wide
+// periodic mesh the two lines may share points).
 template <int N>
-__global__ __launch_bounds__(STAGE_THREADS) void adj_argmax_kernel(AdjArgs a, Ops ops_arg,
-                                                                   unsigned long long *amax,
-                                                                   int *aloc, int pass) {
-  using G = Geo<N>;
-  constexpr int T = G::CPW, NF = N + 1, NT = 2 * N * T, QT = G::QT;
-  __shared__ double so[sizeof(Ops) / sizeof(double)];
-  const Ops &ops = ops_to_lds<0>(so, ops_arg);
-  const int tid = threadIdx.x, tile = blockIdx.x;
-  const int ci = tid % T, fl = tid / T;
-  const int fam = fl >= N ? 1 : 0, line = fl - fam * N;
-  if (!(tid < NT && a.s2c[tile * T + ci] >= 0)) return;
-  const int p0 = fam ? line : N * line, ps = fam ? N : 1;
-  double be = 0.0, bu = 0.0;
-  for (int r = 0; r < NF; ++r) {
-    double sx, sy;
-    int info, k, nbase, np0, nst;
-    bool endN;
-    adj_point_geom<N>(a, ops, tile, ci, fam, line, r, sx, sy, info, k, nbase, np0, nst, endN);
-    const bool face = r == 0 || r == N;
-    double Lr[N], t[9], qn[9];
-    for (int s = 0; s < N; ++s) Lr[s] = ops.L[r][s];
-    adj_trace<N>(a.q, tile * QT + ci, p0, ps, Lr, t);
-    if (face && ((info >> 3) & 7) == FT_INTERIOR) {
-      double Ln[N];
-      for (int s = 0; s < N; ++s) Ln[s] = endN ? ops.L[N][s] : ops.L[0][s];
-      adj_trace<N>(a.q, nbase, np0, nst, Ln, qn);
-    }
-    double e, u;
-    adj_point_speeds<N, double>(a, info, k, r, face, sx, sy, t, qn, e, u);
-    const int loc = (((tile * T + ci) * 2 + fam) * N + line) * NF + r;
-    if (pass == 0) {
-      be = e > be ? e : be;
-      bu = u > bu ? u : bu;
-    } else {
-      if (face && __double_as_longlong(e) == (long long)amax[0]) atomicMin(aloc, loc);
-      if (__double_as_longlong(u) == (long long)amax[1]) atomicMin(aloc + 1, loc);
-    }
-  }
-  if (pass == 0) {
-    atomicMax(amax, (unsigned long long)__double_as_longlong(be));
-    atomicMax(amax + 1, (unsigned long long)__double_as_longlong(bu));
-  }
-}
-
-// Qbar += w * d(speed)/dQ at one flux point (kind 0: eig, 1: um): one
-// thread, both cells of a face.
-template <int N>
-__global__ void adj_argmax_apply(AdjArgs a, Ops ops_arg, int loc, int kind, double w) {
-  using G = Geo<N>;
-  constexpr int T = G::CPW, N2 = G::N2, NF = N + 1, QT = G::QT;
-  __shared__ double so[sizeof(Ops) / sizeof(double)];
-  const Ops &ops = ops_to_lds<0>(so, ops_arg);
-  if (threadIdx.x != 0) return;
+__device__ __forceinline__ void adj_speed_apply(const AdjArgs &a, const Ops &ops, int loc, int kind,
+                                                double w) {
+  constexpr int T = Geo<N>::CPW, NF = N + 1, QT = Geo<N>::QT;
+  const int kk = threadIdx.x;
   const int r = loc % NF, line = (loc / NF) % N, fam = (loc / (NF * N)) % 2;
   const int slot = loc / (NF * N * 2), tile = slot / T, ci = slot % T;
   const int p0 = fam ? line : N * line, ps = fam ? N : 1;
@@ -685,29 +795,142 @@ __global__ void adj_argmax_apply(AdjArgs a, Ops ops_arg, int loc, int kind, doub
   adj_point_geom<N>(a, ops, tile, ci, fam, line, r, sx, sy, info, k, nbase, np0, nst, endN);
   const bool face = r == 0 || r == N;
   const bool nbr = face && ((info >> 3) & 7) == FT_INTERIOR;
-  double Lr[N], Ln[N], t[9], qn[9];
-  for (int s = 0; s < N; ++s) {
-    Lr[s] = ops.L[r][s];
-    Ln[s] = endN ? ops.L[N][s] : ops.L[0][s];
-  }
-  adj_trace<N>(a.q, tile * QT + ci, p0, ps, Lr, t);
-  if (nbr) adj_trace<N>(a.q, nbase, np0, nst, Ln, qn);
-  double *qob = a.qbar + (size_t)tile * QT;
   const int nbt = nbase / QT, nbc = nbase - nbt * QT;
-  double *qnb = a.qbar + (size_t)nbt * QT;
-  for (int kk = 0; kk < (nbr ? 18 : 9); ++kk) {
+  double d = 0.0;
+  if (kk < (nbr ? 18 : 9)) {
+    double Lr[N], Ln[N], t[9], qn[9];
+    for (int s = 0; s < N; ++s) {
+      Lr[s] = ops.L[r][s];
+      Ln[s] = endN ? ops.L[N][s] : ops.L[0][s];
+    }
+    adj_trace<N>(a.q, tile * QT + ci, p0, ps, Lr, t);
+    if (nbr) adj_trace<N>(a.q, nbase, np0, nst, Ln, qn);
     Dual td[9], nd[9], e, u;
+#pragma unroll
     for (int v = 0; v < 9; ++v) {
       td[v] = Dual(t[v], kk == v ? 1.0 : 0.0);
       nd[v] = Dual(nbr ? qn[v] : 0.0, kk == 9 + v ? 1.0 : 0.0);
     }
     adj_point_speeds<N, Dual>(a, info, k, r, face, sx, sy, td, nd, e, u);
-    const double d = w * (kind == 0 ? e.d : u.d);
-    if (kk < 9) {
-      for (int s = 0; s < N; ++s) qob[qo<N>(kk, p0 + ps * s, ci)] += d * Lr[s];
-    } else {
-      for (int s = 0; s < N; ++s) qnb[qo<N>(kk - 9, np0 + nst * s, nbc)] += d * Ln[s];
+    d = w * (kind == 0 ? e.d : u.d);
+  }
+  if (kk < 9)
+    for (int s = 0; s < N; ++s)
+      a.qbar[(size_t)tile * QT + qo<N>(kk, p0 + ps * s, ci)] += d * ops.L[r][s];
+  __syncthreads();
+  if (nbr && kk >= 9 && kk < 18)
+    for (int s = 0; s < N; ++s)
+      a.qbar[(size_t)nbt * QT + qo<N>(kk - 9, np0 + nst * s, nbc)] +=
+          d * (endN ? ops.L[N][s] : ops.L[0][s]);
+  __syncthreads();
+}
+
+// What the reverse pass carries from one evaluation to the next, on the
+// device: the pending cotangents of the running maxima, the free stream's,
+// the c_h cotangent of a single evaluation, and whether a maximum's flux point
+// was not found.
+struct AdjCarry {
+  double PE, PU, p[6], ch;
+  int missed;
+};
+
+// After adj_stage_kernel of one evaluation (one block): the tiles' partial
+// sums in a fixed order; where this evaluation raised a maximum (g0 -> g1) the
+// pending cotangent of the later evaluations' c_h goes to the flux point that
+// attained it (the smallest location code on a tie); and this evaluation's own
+// c_h = sqrt(E (E - U)) is passed on to the maxima before it.
+// 128 x 256 cells, N = 4: 13 us; it replaces two searches over all flux points
+// (71 us each), a single-thread evaluation of the 18 directions (106 us) and
+// the copy of the partial sums to the host, which waited for every stage.
+constexpr int ADJ_TAIL_THREADS = 512;
+template <int N>
+__global__ __launch_bounds__(ADJ_TAIL_THREADS) void adj_tail_kernel(AdjArgs a, Ops ops_arg,
+                                                                    const double *tmax,
+                                                                    const int *tloc,
+                                                                    const double *g1, AdjCarry *cy,
+                                                                    double *chbar) {
+  constexpr int NT = ADJ_TAIL_THREADS;
+  __shared__ double so[sizeof(Ops) / sizeof(double)];
+  __shared__ double sum[ADJ_NPART][NT / 64], mv[2][NT / 64];
+  __shared__ int ml[2][NT / 64];
+  const Ops &ops = ops_to_lds<0>(so, ops_arg);
+  const int t = threadIdx.x, w = t >> 6, l = t & 63;
+  const int none = 0x7fffffff;
+  const double E = a.gm[0], U = a.gm[1];
+  const double PE = cy->PE, PU = cy->PU;
+  const bool raised[2] = {g1[0] > E, g1[1] > U};
+  double x[ADJ_NPART] = {0, 0, 0, 0, 0, 0, 0}, best[2] = {0.0, 0.0};
+  int loc[2] = {none, none};
+  for (int i = t; i < a.ntile; i += NT) {
+#pragma unroll
+    for (int j = 0; j < ADJ_NPART; ++j) x[j] += a.part[(size_t)i * ADJ_NPART + j];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (!raised[j]) continue;
+      const double v = tmax[2 * (size_t)i + j];
+      const int c = tloc[2 * (size_t)i + j];
+      if (v > best[j] || (v == best[j] && c < loc[j])) { best[j] = v; loc[j] = c; }
     }
+  }
+#pragma unroll
+  for (int j = 0; j < ADJ_NPART; ++j) {
+    x[j] = wave_sum(x[j]);
+    if (l == 0) sum[j][w] = x[j];
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    for (int o = 32; o > 0; o >>= 1) {
+      const double v = __shfl_xor(best[j], o, 64);
+      const int c = __shfl_xor(loc[j], o, 64);
+      if (v > best[j] || (v == best[j] && c < loc[j])) { best[j] = v; loc[j] = c; }
+    }
+    if (l == 0) { mv[j][w] = best[j]; ml[j][w] = loc[j]; }
+  }
+  __syncthreads();
+  for (int j = 0; j < 2; ++j) {
+    const double p = j == 0 ? PE : PU;
+    if (!raised[j] || p == 0.0) continue;   // uniform over the block
+    double v = mv[j][0];
+    int c = ml[j][0];
+    for (int k = 1; k < NT / 64; ++k)
+      if (mv[j][k] > v || (mv[j][k] == v && ml[j][k] < c)) { v = mv[j][k]; c = ml[j][k]; }
+    if (c == none || v != g1[j]) {
+      if (t == 0) cy->missed = 1;
+      continue;
+    }
+    adj_speed_apply<N>(a, ops, c, j, p);
+  }
+  if (t < ADJ_NPART) {
+    double s = 0.0;
+    for (int k = 0; k < NT / 64; ++k) s += sum[t][k];
+    if (t > 0) cy->p[t - 1] += s;
+    else {
+      const double ch = sqrt(E * (E - U));
+      double pe = raised[0] ? 0.0 : PE, pu = raised[1] ? 0.0 : PU;
+      if (ch > 0.0) {
+        pe += s * (2.0 * E - U) / (2.0 * ch);
+        pu += s * (-E) / (2.0 * ch);
+      }
+      cy->PE = pe;
+      cy->PU = pu;
+      if (chbar) *chbar = s;
+    }
+  }
+}
+
+// The drag of one state added to *J, summed in a fixed order (one block).
+__global__ __launch_bounds__(1024) void k_drag_sum(const double *__restrict__ dtile, int n,
+                                                   double *__restrict__ J) {
+  __shared__ double s[16];
+  double x = 0.0;
+  for (int i = threadIdx.x; i < n; i += 1024) x += dtile[i];
+  x = wave_sum(x);
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = x;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int k = 0; k < 16; ++k) t += s[k];
+    *J += t;
   }
 }
 

@@ -19,41 +19,48 @@
 // E, U of the wave speeds over all earlier evaluations: its cotangent is
 // carried backwards (pools PE, PU) to the last earlier evaluation that
 // raised the maximum, and there to the flux point whose speed attained it
-// (adj_argmax_kernel / adj_argmax_apply).
+// (recorded by the recomputed stage, M_TRACE; adj_tail_kernel).
+
+// Everything the reverse pass accumulates stays on the device (AdjCarry), so
+// no stage waits for the host: per reversed stage one adj_stage_kernel (the
+// residual's reverse sweep and the RK combination) and one adj_tail_kernel.
 
 struct AdjState {
   int nsteps = 0, ckpt = 0;
   bool have_fwd = false;
   double J = 0.0;
-  double *q[6] = {};          // stage states Q0..Q5 of one step (tile layout)
-  double *b[6] = {};          // cotangents
-  double *g = nullptr;        // Dbar / wbar per point
-  double *divb = nullptr;     // divB per point of the evaluation being reversed
+  double *t[4] = {};          // stage states Q1..Q4 of one step (tile layout)
+  double *b[6] = {};          // cotangents of Q0..Q5
+  double *divb = nullptr;     // divB per point of the five evaluations of a step
   double *part = nullptr;     // per tile partial sums
-  double *gm = nullptr;       // gmax before each of the 5 stages (device)
-  unsigned long long *slots = nullptr;   // scratch maxima of recomputed evaluations
-  double *dcell = nullptr;    // drag per slot
+  double *gm = nullptr;       // gmax before each of the 5 stages and after (device)
+  double *tmax = nullptr;     // per evaluation and tile: largest speeds and where
+  int *tloc = nullptr;
+  AdjCarry *carry = nullptr;  // what goes from one reversed evaluation to the next
+  double *chb = nullptr;      // c_h cotangents, 5 per step
+  int chb_n = 0;
+  unsigned long long *slots = nullptr;   // scratch maxima of sd2d_compresid_vjp
+  double *dtile = nullptr;    // drag per tile
+  double *Jd = nullptr;       // running sum of the drag
   double *wq = nullptr;       // face quadrature weights
   std::vector<double *> ck;   // checkpoint states (index = step / ckpt) + final state
   std::vector<std::array<double, 4>> ckm;   // their maxima
   std::vector<int32_t> cki;   // their iter and ctime
   std::vector<double> ckt;
-  std::vector<double *> seg;  // step inputs of one segment
-  std::vector<std::array<double, 4>> segm;
+  std::vector<double *> seg;  // step inputs of one segment and its output
+  double *segm = nullptr;     // the maxima before each step of the segment (4 each)
+  int segm_n = 0;
   double fin_ctime = 0.0;
   int fin_iter = 0;
-  unsigned long long *amax = nullptr;   // argmax search: maxima and locations
-  int *aloc = nullptr;
-  double PE = 0.0, PU = 0.0;            // pending cotangents of the running maxima
-  int argmax_missed = 0;                // maxima whose flux point was not found
 };
 
 static void adj_free(AdjState *A) {
   if (!A) return;
-  for (double *p : A->q) if (p) (void)hipFree(p);
+  for (double *p : A->t) if (p) (void)hipFree(p);
   for (double *p : A->b) if (p) (void)hipFree(p);
-  for (void *p : {(void *)A->g, (void *)A->divb, (void *)A->part, (void *)A->gm, (void *)A->slots,
-                  (void *)A->dcell, (void *)A->wq, (void *)A->amax, (void *)A->aloc})
+  for (void *p : {(void *)A->divb, (void *)A->part, (void *)A->gm, (void *)A->tmax,
+                  (void *)A->tloc, (void *)A->carry, (void *)A->chb, (void *)A->slots,
+                  (void *)A->dtile, (void *)A->Jd, (void *)A->wq, (void *)A->segm})
     if (p) (void)hipFree(p);
   for (double *p : A->ck) if (p) (void)hipFree(p);
   for (double *p : A->seg) if (p) (void)hipFree(p);
@@ -62,21 +69,35 @@ static void adj_free(AdjState *A) {
 
 static size_t state_len(const sd2d_ctx *c) { return (size_t)c->ntile * 9 * c->N * c->N * c->cpw; }
 
-__global__ void k_axpby(size_t n, double a, const double *__restrict__ x, double b,
-                        double *__restrict__ y) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x)
-    y[i] = (b == 0.0 ? 0.0 : b * y[i]) + a * x[i];
+// The running maxima (slots and gmax of one run) to and from four doubles on
+// the device: eigvmax, umax, eigvmax_g, umax_g.
+__global__ void k_save_max(const unsigned long long *slots, const double *gmax, double *m) {
+  double e = __longlong_as_double((long long)slots[2 * threadIdx.x]);
+  double u = __longlong_as_double((long long)slots[2 * threadIdx.x + 1]);
+  __shared__ double s[2][NSLOT / 64];
+  e = wave_max(e);
+  u = wave_max(u);
+  if ((threadIdx.x & 63) == 0) {
+    s[0][threadIdx.x >> 6] = e;
+    s[1][threadIdx.x >> 6] = u;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    double x = s[threadIdx.x][0];
+    for (int k = 1; k < NSLOT / 64; ++k) x = s[threadIdx.x][k] > x ? s[threadIdx.x][k] : x;
+    m[threadIdx.x] = x;
+    m[2 + threadIdx.x] = gmax[threadIdx.x];
+  }
+}
+__global__ void k_load_max(const double *m, unsigned long long *slots, double *gmax) {
+  const int t = threadIdx.x;
+  slots[2 * t] = t == 0 ? (unsigned long long)__double_as_longlong(m[0]) : 0ull;
+  slots[2 * t + 1] = t == 0 ? (unsigned long long)__double_as_longlong(m[1]) : 0ull;
+  if (t < 2) gmax[t] = m[2 + t];
 }
 
 __global__ void k_copy2(const double *__restrict__ s, double *__restrict__ d) {
   if (threadIdx.x < 2) d[threadIdx.x] = s[threadIdx.x];
-}
-
-static int axpby(sd2d_ctx *c, double a, const double *x, double b, double *y) {
-  hipLaunchKernelGGL(k_axpby, dim3(2048), dim3(256), 0, c->stream, state_len(c), a, x, b, y);
-  HIPCHK(c, hipGetLastError());
-  return SD2D_OK;
 }
 
 static int adj_maxima_get(sd2d_ctx *c, std::array<double, 4> &m) {
@@ -113,52 +134,69 @@ static std::vector<double> face_weights(const double *xs, int N) {
   return w;
 }
 
-static int adj_alloc(sd2d_ctx *c, AdjState *A, int nck) {
+// What one residual's reverse sweep needs, and (steps) the whole reverse pass.
+static int adj_alloc(sd2d_ctx *c, AdjState *A, int nck, bool steps) {
   const size_t n = state_len(c);
-  const int N = c->N, N2 = N * N, T = c->cpw;
-  for (auto &p : A->q) if (!p) HIPCHK(c, hipMalloc(&p, n * sizeof(double)));
-  for (auto &p : A->b) if (!p) HIPCHK(c, hipMalloc(&p, n * sizeof(double)));
-  if (!A->g) HIPCHK(c, hipMalloc(&A->g, (size_t)c->ntile * 10 * N2 * T * sizeof(double)));
-  if (!A->part) HIPCHK(c, hipMalloc(&A->part, (size_t)c->ntile * ADJ_NPART * sizeof(double)));
-  if (!A->gm) HIPCHK(c, hipMalloc(&A->gm, 12 * sizeof(double)));
-  if (!A->amax) HIPCHK(c, hipMalloc(&A->amax, 2 * sizeof(unsigned long long)));
-  if (!A->aloc) HIPCHK(c, hipMalloc(&A->aloc, 2 * sizeof(int)));
-  if (!A->slots) HIPCHK(c, hipMalloc(&A->slots, 2 * NSLOT * sizeof(unsigned long long)));
-  if (!A->dcell) HIPCHK(c, hipMalloc(&A->dcell, (size_t)c->ntile * T * sizeof(double)));
-  if (!A->divb) HIPCHK(c, hipMalloc(&A->divb, (size_t)c->ntile * N2 * T * sizeof(double)));
+  const size_t np = (size_t)c->ntile * c->N * c->N * c->cpw;
+  auto get = [&](auto *&p, size_t count) -> int {
+    if (!p) HIPCHK(c, hipMalloc(&p, count * sizeof(*p)));
+    return SD2D_OK;
+  };
+  int r;
+#define ADJGET(p, count) do { if ((r = get(p, count))) return r; } while (0)
+  for (int i = 0; i < (steps ? 6 : 2); ++i) ADJGET(A->b[i], n);
+  ADJGET(A->divb, 5 * np);
+  ADJGET(A->part, (size_t)c->ntile * ADJ_NPART);
+  ADJGET(A->carry, 1);
+  ADJGET(A->slots, 2 * NSLOT);
+  if (!steps) return SD2D_OK;
+  for (auto &p : A->t) ADJGET(p, n);
+  ADJGET(A->gm, 12);
+  ADJGET(A->tmax, 10 * (size_t)c->ntile);
+  ADJGET(A->tloc, 10 * (size_t)c->ntile);
+  ADJGET(A->dtile, c->ntile);
+  ADJGET(A->Jd, 1);
+  if (A->chb_n < 5 * A->nsteps) {
+    if (A->chb) { HIPCHK(c, hipFree(A->chb)); A->chb = nullptr; A->chb_n = 0; }
+    ADJGET(A->chb, (size_t)5 * A->nsteps);
+    A->chb_n = 5 * A->nsteps;
+  }
+  const int nseg = std::min(A->ckpt, A->nsteps);
+  if (A->segm_n < nseg) {
+    if (A->segm) { HIPCHK(c, hipFree(A->segm)); A->segm = nullptr; A->segm_n = 0; }
+    ADJGET(A->segm, (size_t)4 * nseg);
+    A->segm_n = nseg;
+  }
+#undef ADJGET
   while ((int)A->ck.size() < nck) {
     double *p = nullptr;
     HIPCHK(c, hipMalloc(&p, n * sizeof(double)));
     A->ck.push_back(p);
   }
   A->ckm.resize(A->ck.size());
-  while ((int)A->seg.size() < A->ckpt) {
+  while ((int)A->seg.size() < nseg + 1) {
     double *p = nullptr;
     HIPCHK(c, hipMalloc(&p, n * sizeof(double)));
     A->seg.push_back(p);
   }
-  A->segm.resize(A->seg.size());
   return SD2D_OK;
 }
 
-// time-step quadrature of the wall drag at state q (and, with qbar, its
-// cotangent scale * dD/dq added to qbar)
-static int drag_eval(sd2d_ctx *c, const double *q, double *D, double *qbar, double scale) {
+// The wall drag at state q added to A->Jd (sum), or with qbar its cotangent
+// scale * dD/dq added to qbar.
+static int drag_eval(sd2d_ctx *c, const double *q, bool sum, double *qbar, double scale) {
   AdjState *A = c->adj;
-  const int nsl = c->ntile * c->cpw, tb = 256, nb = (nsl + tb - 1) / tb;
+  const dim3 grid(c->ntile), block(64);
   switch (c->N) {
-    case 3: hipLaunchKernelGGL(drag_kernel<3>, dim3(nb), dim3(tb), 0, c->stream, q, c->ftab, c->met, A->wq, c->ops, c->ncell, c->ntile, A->dcell, qbar, scale); break;
-    case 4: hipLaunchKernelGGL(drag_kernel<4>, dim3(nb), dim3(tb), 0, c->stream, q, c->ftab, c->met, A->wq, c->ops, c->ncell, c->ntile, A->dcell, qbar, scale); break;
-    default: hipLaunchKernelGGL(drag_kernel<5>, dim3(nb), dim3(tb), 0, c->stream, q, c->ftab, c->met, A->wq, c->ops, c->ncell, c->ntile, A->dcell, qbar, scale); break;
+    case 3: hipLaunchKernelGGL(drag_kernel<3>, grid, block, 0, c->stream, q, c->ftab, c->met, A->wq, c->ops, A->dtile, qbar, scale); break;
+    case 4: hipLaunchKernelGGL(drag_kernel<4>, grid, block, 0, c->stream, q, c->ftab, c->met, A->wq, c->ops, A->dtile, qbar, scale); break;
+    default: hipLaunchKernelGGL(drag_kernel<5>, grid, block, 0, c->stream, q, c->ftab, c->met, A->wq, c->ops, A->dtile, qbar, scale); break;
   }
   HIPCHK(c, hipGetLastError());
-  if (D) {
-    std::vector<double> d(nsl);
-    HIPCHK(c, hipMemcpyAsync(d.data(), A->dcell, nsl * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    double s = 0.0;
-    for (double x : d) s += x;
-    *D = s;
+  if (sum) {
+    hipLaunchKernelGGL(k_drag_sum, dim3(1), dim3(1024), 0, c->stream, A->dtile, c->ntile,
+                       A->Jd);
+    HIPCHK(c, hipGetLastError());
   }
   return SD2D_OK;
 }
@@ -173,155 +211,107 @@ static const AdjStage kS5P3[5] = {
     {3, 0, 4, 0.632066208361863, 0.367933791638137, 0.238458932846290},
     {4, 2, 5, 0.762406163401431, 0.237593836598569, 0.287632146308408}};
 
-// Recompute the five stage inputs of one step from q[0] and the maxima m,
-// recording gmax before every stage in A->gm (the forward's launches).
-static int adj_recompute_step(sd2d_ctx *c, const std::array<double, 4> &m) {
+// The five stages of one step from qs[0] (the forward's launches), its states
+// into qs[1..5]; with trace, what the reverse sweep needs of each evaluation
+// is recorded as well (divB, the maxima before every stage and after the last,
+// and where each tile's largest speeds are attained).
+static int adj_stages(sd2d_ctx *c, double *const *qs, bool trace) {
   AdjState *A = c->adj;
-  int r = adj_maxima_set(c, m);
-  if (r) return r;
   const int av = (c->p.artiv == 1 && c->p.vismode == 1) ? M_AV : 0;
+  const size_t np = (size_t)c->ntile * c->N * c->N * c->cpw;
   for (int s = 0; s < 5; ++s) {
     const AdjStage &st = kS5P3[s];
-    hipLaunchKernelGGL(k_copy2, dim3(1), dim3(64), 0, c->stream, c->gmax, A->gm + 2 * s);
-    HIPCHK(c, hipGetLastError());
     StageArgs a = base_args(c);
-    a.qin = A->q[st.in];
-    a.qout = A->q[st.out];
+    a.qin = qs[st.in];
+    a.qout = qs[st.out];
     a.cin = st.cin;
     a.cr = st.b * c->p.dt;
     a.naux = st.aux >= 0 ? 1 : 0;
-    a.aux[0] = st.aux >= 0 ? A->q[st.aux] : nullptr;
+    a.aux[0] = st.aux >= 0 ? qs[st.aux] : nullptr;
     a.ca[0] = st.ca;
-    const int mode = M_RK | (a.naux ? M_AUX1 : 0) | (s == 4 ? av : 0);
+    a.rev = c->nlaunch++ & 1;
+    int mode = M_RK | (a.naux ? M_AUX1 : 0) | (s == 4 ? av : 0);
+    if (trace) {
+      mode |= M_TRACE;
+      a.divb = A->divb + s * np;
+      a.gmrec = A->gm + 2 * s;
+      a.tmax = A->tmax + 2 * (size_t)c->ntile * s;
+      a.tloc = A->tloc + 2 * (size_t)c->ntile * s;
+    }
     HIPCHK(c, launch_stage(c, a, mode));
-    r = finalize_stage(c);
+    const int r = finalize_stage(c);
     if (r) return r;
   }
-  hipLaunchKernelGGL(k_copy2, dim3(1), dim3(64), 0, c->stream, c->gmax, A->gm + 10);
-  HIPCHK(c, hipGetLastError());
+  if (trace) {
+    hipLaunchKernelGGL(k_copy2, dim3(1), dim3(64), 0, c->stream, c->gmax, A->gm + 10);
+    HIPCHK(c, hipGetLastError());
+  }
   return SD2D_OK;
 }
 
-static AdjArgs adj_args(sd2d_ctx *c, const double *q, double *qbar) {
+// One evaluation backwards: adj_stage_kernel, then adj_tail_kernel with the
+// maxima g1 after the evaluation.
+template <int N>
+static hipError_t adj_launch_n(sd2d_ctx *c, const AdjArgs &a, const double *tmax, const int *tloc,
+                               const double *g1, double *chbar) {
+  AdjState *A = c->adj;
+  static_assert(adj_lds_bytes<N>() <= 65536, "adjoint kernel LDS above 64 KiB");
+  hipLaunchKernelGGL(adj_stage_kernel<N>, dim3(c->ntile), dim3(STAGE_THREADS), adj_lds_bytes<N>(),
+                     c->stream, a, c->ops);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(adj_tail_kernel<N>, dim3(1), dim3(ADJ_TAIL_THREADS), 0, c->stream, a, c->ops,
+                     tmax, tloc, g1, A->carry, chbar);
+  return hipGetLastError();
+}
+static int adj_launch(sd2d_ctx *c, const AdjArgs &a, const double *tmax, const int *tloc,
+                      const double *g1, double *chbar) {
+  switch (c->N) {
+    case 3: HIPCHK(c, adj_launch_n<3>(c, a, tmax, tloc, g1, chbar)); break;
+    case 4: HIPCHK(c, adj_launch_n<4>(c, a, tmax, tloc, g1, chbar)); break;
+    default: HIPCHK(c, adj_launch_n<5>(c, a, tmax, tloc, g1, chbar)); break;
+  }
+  return SD2D_OK;
+}
+
+static AdjArgs adj_args(sd2d_ctx *c) {
   AdjState *A = c->adj;
   AdjArgs a{};
-  a.q = q; a.rscale = 1.0; a.divb = A->divb; a.met = c->met; a.ftab = c->ftab;
-  a.s2c = c->s2c; a.phm = c->phm; a.g = A->g; a.qbar = qbar; a.part = A->part;
-  a.alpha = c->ph.alpha; a.ncell = c->ncell; a.ntile = c->ntile;
+  a.rscale = 1.0; a.met = c->met; a.ftab = c->ftab; a.tinfo = c->tinfo; a.phm = c->phm;
+  a.part = A->part; a.alpha = c->ph.alpha; a.ntile = c->ntile;
   return a;
 }
 
-// The flux point where the evaluation of state q attained its largest eig
-// (kind 0) or um (kind 1), and qbar += w * d(that speed)/dq.
-static int adj_argmax_push(sd2d_ctx *c, const double *q, double *qbar, int kind, double w) {
-  AdjState *A = c->adj;
-  AdjArgs a = adj_args(c, q, qbar);
-  HIPCHK(c, hipMemsetAsync(A->amax, 0, 2 * sizeof(unsigned long long), c->stream));
-  HIPCHK(c, hipMemsetAsync(A->aloc, 0x7f, 2 * sizeof(int), c->stream));
-  for (int pass = 0; pass < 2; ++pass) {
-    switch (c->N) {
-      case 3: hipLaunchKernelGGL(adj_argmax_kernel<3>, dim3(c->ntile), dim3(STAGE_THREADS), 0, c->stream, a, c->ops, A->amax, A->aloc, pass); break;
-      case 4: hipLaunchKernelGGL(adj_argmax_kernel<4>, dim3(c->ntile), dim3(STAGE_THREADS), 0, c->stream, a, c->ops, A->amax, A->aloc, pass); break;
-      default: hipLaunchKernelGGL(adj_argmax_kernel<5>, dim3(c->ntile), dim3(STAGE_THREADS), 0, c->stream, a, c->ops, A->amax, A->aloc, pass); break;
-    }
-    HIPCHK(c, hipGetLastError());
-  }
-  int loc[2];
-  HIPCHK(c, hipMemcpyAsync(loc, A->aloc, sizeof(loc), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (loc[kind] == 0x7f7f7f7f) { A->argmax_missed += 1; return SD2D_OK; }
-  switch (c->N) {
-    case 3: hipLaunchKernelGGL(adj_argmax_apply<3>, dim3(1), dim3(64), 0, c->stream, a, c->ops, loc[kind], kind, w); break;
-    case 4: hipLaunchKernelGGL(adj_argmax_apply<4>, dim3(1), dim3(64), 0, c->stream, a, c->ops, loc[kind], kind, w); break;
-    default: hipLaunchKernelGGL(adj_argmax_apply<5>, dim3(1), dim3(64), 0, c->stream, a, c->ops, loc[kind], kind, w); break;
-  }
-  HIPCHK(c, hipGetLastError());
-  return SD2D_OK;
-}
-
-// Qbar += (dR/dq)^T (rscale * rbar) for the residual of q whose c_h came
-// from gm; acc[0] += c_hbar, acc[1..6] += free-stream cotangents.
-static int adj_resid_vjp(sd2d_ctx *c, const double *q, const double *gm, const double *rbar,
-                         double rscale, double *qbar, double *acc) {
-  AdjState *A = c->adj;
-  // divB of q, as the stepping kernel forms it for the Powell source, with
-  // scratch maxima
-  StageArgs s = base_args(c);
-  s.qin = q;
-  s.gmax = gm;
-  s.slots = A->slots;
-  s.divb = A->divb;
-  HIPCHK(c, launch_stage(c, s, M_DIVB));
-  AdjArgs a{};
-  a.q = q; a.rbar = rbar; a.rscale = rscale; a.divb = A->divb; a.met = c->met;
-  a.ftab = c->ftab; a.s2c = c->s2c; a.phm = c->phm; a.gm = gm; a.g = A->g; a.qbar = qbar;
-  a.part = A->part; a.alpha = c->ph.alpha; a.ncell = c->ncell; a.ntile = c->ntile;
-  switch (c->N) {
-    case 3:
-      hipLaunchKernelGGL(adj_point_kernel<3>, dim3(c->ntile), dim3(STAGE_THREADS), 0, c->stream, a);
-      hipLaunchKernelGGL(adj_line_kernel<3>, dim3(c->ntile), dim3(STAGE_THREADS), adj_lds_bytes<3>(), c->stream, a, c->ops);
-      break;
-    case 4:
-      hipLaunchKernelGGL(adj_point_kernel<4>, dim3(c->ntile), dim3(STAGE_THREADS), 0, c->stream, a);
-      hipLaunchKernelGGL(adj_line_kernel<4>, dim3(c->ntile), dim3(STAGE_THREADS), adj_lds_bytes<4>(), c->stream, a, c->ops);
-      break;
-    default:
-      hipLaunchKernelGGL(adj_point_kernel<5>, dim3(c->ntile), dim3(STAGE_THREADS), 0, c->stream, a);
-      hipLaunchKernelGGL(adj_line_kernel<5>, dim3(c->ntile), dim3(STAGE_THREADS), adj_lds_bytes<5>(), c->stream, a, c->ops);
-      break;
-  }
-  HIPCHK(c, hipGetLastError());
-  std::vector<double> part((size_t)c->ntile * ADJ_NPART);
-  HIPCHK(c, hipMemcpyAsync(part.data(), A->part, part.size() * sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int t = 0; t < c->ntile; ++t)
-    for (int j = 0; j < ADJ_NPART; ++j) acc[j] += part[(size_t)t * ADJ_NPART + j];
-  return SD2D_OK;
-}
-
 // Reverse one RK_S5P3 step: A->b[5] holds the cotangent of the step's
-// output (Q5), on return A->b[0] that of its input (Q0).  A->q[0..4] and
-// A->gm hold the recomputed stage inputs and their maxima.
-static int adj_step_vjp(sd2d_ctx *c, double *pacc, double *chbar5) {
+// output (Q5), on return A->b[0] that of its input (Q0).  qs[0..4] are the
+// recomputed stage inputs (adj_stages with trace).
+static int adj_step_vjp(sd2d_ctx *c, double *const *qs, double *chbar5) {
   AdjState *A = c->adj;
   double **B = A->b;
-  const double dt = c->p.dt;
-  int r;
-  double acc[ADJ_NPART];
-  double gm[12];   // running maxima (eigvmax_g, umax_g) before each stage and after the last
-  HIPCHK(c, hipMemcpyAsync(gm, A->gm, sizeof(gm), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  // zero the stage cotangents
-  for (int k = 0; k < 5; ++k)
-    HIPCHK(c, hipMemsetAsync(B[k], 0, state_len(c) * sizeof(double), c->stream));
+  const size_t np = (size_t)c->ntile * c->N * c->N * c->cpw;
+  bool have[5] = {false, false, false, false, false};   // cotangents already begun
   for (int s = 4; s >= 0; --s) {
     const AdjStage &st = kS5P3[s];
     // Q_out = cin Q_in + ca Q_aux + b dt R(Q_in)
-    if ((r = axpby(c, st.cin, B[st.out], 1.0, B[st.in]))) return r;
-    if (st.aux >= 0 && (r = axpby(c, st.ca, B[st.out], 1.0, B[st.aux]))) return r;
-    // the maxima this evaluation raised take the pending cotangents of the
-    // later evaluations' c_h
-    const double *g0 = gm + 2 * s, *g1 = gm + 2 * (s + 1);
-    if (g1[0] > g0[0]) {
-      if (A->PE != 0.0 && (r = adj_argmax_push(c, A->q[st.in], B[st.in], 0, A->PE))) return r;
-      A->PE = 0.0;
+    AdjArgs a = adj_args(c);
+    a.q = qs[st.in];
+    a.rbar = B[st.out];
+    a.rscale = st.b * c->p.dt;
+    a.cin = st.cin;
+    a.ca = st.ca;
+    a.divb = A->divb + s * np;
+    a.gm = A->gm + 2 * s;
+    a.qbar = B[st.in];
+    a.qadd = have[st.in];
+    have[st.in] = true;
+    if (st.aux >= 0) {
+      a.abar = B[st.aux];
+      a.aadd = have[st.aux];
+      have[st.aux] = true;
     }
-    if (g1[1] > g0[1]) {
-      if (A->PU != 0.0 && (r = adj_argmax_push(c, A->q[st.in], B[st.in], 1, A->PU))) return r;
-      A->PU = 0.0;
-    }
-    for (double &x : acc) x = 0.0;
-    r = adj_resid_vjp(c, A->q[st.in], A->gm + 2 * st.in, B[st.out], st.b * dt, B[st.in], acc);
+    const int r = adj_launch(c, a, A->tmax + 2 * (size_t)c->ntile * s,
+                             A->tloc + 2 * (size_t)c->ntile * s, A->gm + 2 * (s + 1), chbar5 + s);
     if (r) return r;
-    if (chbar5) chbar5[s] = acc[0];
-    for (int j = 0; j < 6; ++j) pacc[j] += acc[1 + j];
-    // c_h = sqrt(E (E - U)) of this evaluation, from the maxima before it
-    const double E = g0[0], U = g0[1], ch = std::sqrt(E * (E - U));
-    if (ch > 0.0) {
-      A->PE += acc[0] * (2.0 * E - U) / (2.0 * ch);
-      A->PU += acc[0] * (-E) / (2.0 * ch);
-    }
   }
   return SD2D_OK;
 }
@@ -352,13 +342,13 @@ int sd2d_fwd(sd2d_ctx *c, int32_t nsteps, int32_t ckpt, double *objective) {
   A->ckpt = ckpt;
   A->have_fwd = false;
   const int nck = (nsteps + ckpt - 1) / ckpt + 1;   // segment starts + the final state
-  int r = adj_alloc(c, A, nck);
+  int r = adj_alloc(c, A, nck, true);
   if (r) return r;
   if ((r = adj_weights(c, A))) return r;
   A->cki.assign(nck, 0);
   A->ckt.assign(nck, 0.0);
   const size_t nb = state_len(c) * sizeof(double);
-  double J = 0.0;
+  HIPCHK(c, hipMemsetAsync(A->Jd, 0, sizeof(double), c->stream));
   for (int n = 0; n < nsteps; ++n) {
     if (n % ckpt == 0) {
       HIPCHK(c, hipMemcpyAsync(A->ck[n / ckpt], c->q[c->cur], nb, hipMemcpyDeviceToDevice, c->stream));
@@ -369,10 +359,10 @@ int sd2d_fwd(sd2d_ctx *c, int32_t nsteps, int32_t ckpt, double *objective) {
     c->iter += 1;
     if ((r = step_rk(c, false))) return r;
     c->have_av = c->p.artiv == 1 && c->p.vismode == 1;
-    double D;
-    if ((r = drag_eval(c, c->q[c->cur], &D, nullptr, 0.0))) return r;
-    J += D;
+    if ((r = drag_eval(c, c->q[c->cur], true, nullptr, 0.0))) return r;
   }
+  double J = 0.0;
+  HIPCHK(c, hipMemcpyAsync(&J, A->Jd, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(A->ck[nck - 1], c->q[c->cur], nb, hipMemcpyDeviceToDevice, c->stream));
   if ((r = adj_maxima_get(c, A->ckm[nck - 1]))) return r;
   A->fin_ctime = c->ctime;
@@ -403,31 +393,38 @@ int sd2d_vjp(sd2d_ctx *c, const double *qbar_final, double jbar, double *qbar_in
   } else {
     HIPCHK(c, hipMemsetAsync(A->b[5], 0, nb, c->stream));
   }
-  double pacc[6] = {0, 0, 0, 0, 0, 0};
-  A->PE = A->PU = 0.0;
-  A->argmax_missed = 0;
+  HIPCHK(c, hipMemsetAsync(A->carry, 0, sizeof(AdjCarry), c->stream));
   for (int sg = (nsteps - 1) / ckpt; sg >= 0; --sg) {
-    const int n0 = sg * ckpt, n1 = std::min(nsteps, n0 + ckpt);
-    // the segment's step inputs, recomputed from its checkpoint
-    HIPCHK(c, hipMemcpyAsync(A->q[0], A->ck[sg], nb, hipMemcpyDeviceToDevice, c->stream));
-    std::array<double, 4> m = A->ckm[sg];
-    for (int i = 0; i < n1 - n0; ++i) {
-      HIPCHK(c, hipMemcpyAsync(A->seg[i], A->q[0], nb, hipMemcpyDeviceToDevice, c->stream));
-      A->segm[i] = m;
-      if (i + 1 < n1 - n0) {
-        if ((r = adj_recompute_step(c, m))) return r;
-        if ((r = adj_maxima_get(c, m))) return r;
-        HIPCHK(c, hipMemcpyAsync(A->q[0], A->q[5], nb, hipMemcpyDeviceToDevice, c->stream));
-      }
+    const int n0 = sg * ckpt, n1 = std::min(nsteps, n0 + ckpt), len = n1 - n0;
+    // the segment's step inputs and the maxima before them, recomputed from
+    // its checkpoint
+    HIPCHK(c, hipMemcpyAsync(A->seg[0], A->ck[sg], nb, hipMemcpyDeviceToDevice, c->stream));
+    if ((r = adj_maxima_set(c, A->ckm[sg]))) return r;
+    auto step_states = [&](int i, double **qs) {
+      qs[0] = A->seg[i];
+      for (int k = 0; k < 4; ++k) qs[1 + k] = A->t[k];
+      qs[5] = A->seg[i + 1];
+    };
+    double *qs[6];
+    for (int i = 0; i < len; ++i) {
+      hipLaunchKernelGGL(k_save_max, dim3(1), dim3(NSLOT), 0, c->stream, c->slots, c->gmax,
+                         A->segm + 4 * i);
+      HIPCHK(c, hipGetLastError());
+      if (i + 1 == len) break;   // the last step runs once, below
+      step_states(i, qs);
+      if ((r = adj_stages(c, qs, false))) return r;
     }
-    for (int i = n1 - n0 - 1; i >= 0; --i) {
+    for (int i = len - 1; i >= 0; --i) {
       const int n = n0 + i;   // step n takes Q_n to Q_{n+1}
-      HIPCHK(c, hipMemcpyAsync(A->q[0], A->seg[i], nb, hipMemcpyDeviceToDevice, c->stream));
-      if ((r = adj_recompute_step(c, A->segm[i]))) return r;
+      hipLaunchKernelGGL(k_load_max, dim3(1), dim3(NSLOT), 0, c->stream, A->segm + 4 * i, c->slots,
+                         c->gmax);
+      HIPCHK(c, hipGetLastError());
+      step_states(i, qs);
+      if ((r = adj_stages(c, qs, true))) return r;
       // the drag of the step's output enters the objective with weight 1/nsteps
-      if (jbar != 0.0 && (r = drag_eval(c, A->q[5], nullptr, A->b[5], jbar / nsteps))) return r;
-      if ((r = adj_step_vjp(c, pacc, chbar ? chbar + 5 * n : nullptr))) return r;
-      HIPCHK(c, hipMemcpyAsync(A->b[5], A->b[0], nb, hipMemcpyDeviceToDevice, c->stream));
+      if (jbar != 0.0 && (r = drag_eval(c, qs[5], false, A->b[5], jbar / nsteps))) return r;
+      if ((r = adj_step_vjp(c, qs, A->chb + 5 * n))) return r;
+      std::swap(A->b[0], A->b[5]);
     }
   }
   if (qbar_init) {
@@ -435,8 +432,14 @@ int sd2d_vjp(sd2d_ctx *c, const double *qbar_final, double jbar, double *qbar_in
     const size_t n = (size_t)c->ncell * 9 * c->N * c->N;
     HIPCHK(c, hipMemcpyAsync(qbar_init, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   }
-  if (pbar) for (int j = 0; j < 6; ++j) pbar[j] = pacc[j];
-  if (A->argmax_missed)
+  AdjCarry cy{};
+  HIPCHK(c, hipMemcpyAsync(&cy, A->carry, sizeof(cy), hipMemcpyDeviceToHost, c->stream));
+  if (chbar)
+    HIPCHK(c, hipMemcpyAsync(chbar, A->chb, (size_t)5 * nsteps * sizeof(double), hipMemcpyDeviceToHost,
+                             c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (pbar) for (int j = 0; j < 6; ++j) pbar[j] = cy.p[j];
+  if (cy.missed)
     return fail(c, SD2D_EINVAL, "adjoint: the flux point of a running maximum was not found");
   // the context returns to the final state of sd2d_fwd
   HIPCHK(c, hipMemcpyAsync(c->q[c->cur], A->ck[nck - 1], nb, hipMemcpyDeviceToDevice, c->stream));
@@ -512,7 +515,7 @@ int sd2d_adj_load(sd2d_ctx *c, const char *prefix) {
   A->nsteps = hv[2];
   A->ckpt = hv[3];
   const int nck = (A->nsteps + A->ckpt - 1) / A->ckpt + 1;
-  int r = adj_alloc(c, A, nck);
+  int r = adj_alloc(c, A, nck, true);
   if (r) return r;
   if ((r = adj_weights(c, A))) return r;
   A->cki.assign(nck, 0);
@@ -558,23 +561,36 @@ int sd2d_compresid_vjp(sd2d_ctx *c, const double *rbar, double *qbar, double *ch
   if (!c->adj) c->adj = new (std::nothrow) AdjState();
   AdjState *A = c->adj;
   if (!A) return fail(c, SD2D_ENOMEM, "host allocation failed");
-  if (A->ckpt <= 0) A->ckpt = 1;
-  int r = adj_alloc(c, A, 0);
+  int r = adj_alloc(c, A, 0, false);
   if (r) return r;
   const size_t n = (size_t)c->ncell * 9 * c->N * c->N;
   HIPCHK(c, hipMemcpyAsync(c->stagef, rbar, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   if ((r = f2t(c, c->stagef, A->b[1]))) return r;
-  HIPCHK(c, hipMemsetAsync(A->b[0], 0, state_len(c) * sizeof(double), c->stream));
-  double acc[ADJ_NPART] = {0, 0, 0, 0, 0, 0, 0};
-  r = adj_resid_vjp(c, c->q[c->cur], c->gmax, A->b[1], 1.0, A->b[0], acc);
-  if (r) return r;
+  // divB of the state as the stepping kernel forms it for the Powell source,
+  // with scratch maxima
+  const double *q = c->q[c->cur];
+  StageArgs s = base_args(c);
+  s.qin = q;
+  s.slots = A->slots;
+  s.divb = A->divb;
+  HIPCHK(c, launch_stage(c, s, M_DIVB));
+  AdjArgs a = adj_args(c);
+  a.q = q;
+  a.rbar = A->b[1];
+  a.divb = A->divb;
+  a.gm = c->gmax;
+  a.qbar = A->b[0];
+  HIPCHK(c, hipMemsetAsync(A->carry, 0, sizeof(AdjCarry), c->stream));
+  if ((r = adj_launch(c, a, nullptr, nullptr, c->gmax, &A->carry->ch))) return r;   // raises nothing
   if (qbar) {
     if ((r = t2f(c, A->b[0], c->stagef))) return r;
     HIPCHK(c, hipMemcpyAsync(qbar, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   }
+  AdjCarry cy{};
+  HIPCHK(c, hipMemcpyAsync(&cy, A->carry, sizeof(cy), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (chbar) *chbar = acc[0];
-  if (pbar) for (int j = 0; j < 6; ++j) pbar[j] = acc[1 + j];
+  if (chbar) *chbar = cy.ch;
+  if (pbar) for (int j = 0; j < 6; ++j) pbar[j] = cy.p[j];
   return SD2D_OK;
 }
 

@@ -61,7 +61,12 @@ struct StageArgs {
   // kernel arguments so that its entries are scalar loads)
   double avf[NMAX * NMAX];
   const double *visres;     // viscous divergence dFv + dGv (tile layout), M_VIS
-  double *divb;             // divB per solution point [tile][p][ci], M_DIVB
+  double *divb;             // divB per solution point [tile][p][ci], M_DIVB and M_TRACE
+  // M_TRACE, for the adjoint: the maxima c_h was formed from (2), and per tile
+  // the largest wave speed and velocity bound of this evaluation and the
+  // smallest location code that attains each
+  double *gmrec, *tmax;     // tmax[2*tile]: eig, um
+  int *tloc;                // tloc[2*tile]
   const int *s2c;           // slot -> mesh cell, for the cell-indexed outputs
   // per tile (member << 6 | valid cells), member 0 for one run; an
   // ensemble of runs also has per-member dt (qout then uses cr * dt, null
@@ -82,8 +87,17 @@ struct StageArgs {
 // M_DIVB (no RK update, no Fortran-layout output) stores only divB at every
 // solution point, in tile layout: what the adjoint's reverse sweep of the
 // Powell source needs, with the arithmetic of the stepping kernel.
+// M_TRACE (with M_RK) is a stepping launch that also records what the reverse
+// sweep of its residual needs: divB per point, c_h's maxima, and where the
+// tile's largest speeds are attained.
 enum { M_RK = 1, M_AV = 2, M_NORMS = 4, M_COMPAT = 8, M_AUX1 = 16, M_AUX4 = 32,
-       M_RSTORE = 64, M_VIS = 128, M_DIVB = 256 };
+       M_RSTORE = 64, M_VIS = 128, M_DIVB = 256, M_TRACE = 512 };
+
+// Location code of flux point rfp of a line (slot = tile * T + ci).
+template <int N>
+__host__ __device__ constexpr int flux_point_code(int slot, int fam, int line, int rfp) {
+  return ((slot * 2 + fam) * N + line) * (N + 1) + rfp;
+}
 
 // XCD-aware block order: consecutive positions of the tile launch order go
 // to the same XCD (and its L2), so the neighbour lines a tile reads were
@@ -467,8 +481,9 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
   constexpr int T = G::CPW, N2 = G::N2, NF = N + 1;
   constexpr bool AV = (MODE & M_AV) != 0, NORMS = (MODE & M_NORMS) != 0;
   constexpr bool COMPAT = (MODE & M_COMPAT) != 0, RK = (MODE & M_RK) != 0;
-  constexpr bool DIVB = (MODE & M_DIVB) != 0;
+  constexpr bool DIVB = (MODE & M_DIVB) != 0, TRACE = (MODE & M_TRACE) != 0;
   static_assert(!DIVB || (!RK && !COMPAT), "M_DIVB is a mode of its own");
+  static_assert(!TRACE || RK, "M_TRACE is a stepping mode");
   constexpr int NAUX = (MODE & M_AUX4) ? 4 : ((MODE & M_AUX1) ? 1 : 0);
   constexpr bool RSTORE = (MODE & M_RSTORE) != 0, VIS = (MODE & M_VIS) != 0;
   static_assert(N * T <= 64 && STAGE_THREADS == 128, "one wavefront per line family");
@@ -549,6 +564,23 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
   const Phys &ph = a.phm[mem];                            // the member's free stream
   const double c_h = sqrt(ge * (ge - gu));   // lagged GLM speed, compflux.f90:6
   double eig = 0.0, um = 0.0, nres = 0.0, ndiv = 0.0;
+  if (TRACE && blockIdx.x == 0 && tid == 0) {
+    a.gmrec[0] = ge;
+    a.gmrec[1] = gu;
+  }
+  // M_TRACE: the flux point of the line that attains eig and um (the smaller
+  // number on a tie; the points come in the order 0, N, 1, ..., N-1)
+  int re = 0, ru = 0;
+  double eigp = 0.0, ump = 0.0;
+  auto trace_max = [&](int r) {
+    const bool be = eigp > eig, bu = (ump > um) | ((ump == um) & (r < ru));
+    re = be ? r : re;
+    eig = be ? eigp : eig;
+    ru = bu ? r : ru;
+    um = bu ? ump : um;
+    eigp = ump = 0.0;
+  };
+  double &eigw = TRACE ? eigp : eig, &umw = TRACE ? ump : um;
   __syncthreads();
   if (valid && lci0 >= 0) face_trace_lds<N, double>(lds + LD::Q0, ops, info0, fam, line, 0, lci0, qn0);
   if (valid && lciN >= 0) face_trace_lds<N, double>(lds + LD::Q0, ops, infoN, fam, line, N, lciN, qnN);
@@ -566,7 +598,8 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
       });
       const double sx = msx[0], sy = msy[0];
       double Qv[9];
-      face_flux<N, double>(info0, fam, 0, ph, c_h, t0, qn0, sx, sy, F0, Qv, eig, um);
+      face_flux<N, double>(info0, fam, 0, ph, c_h, t0, qn0, sx, sy, F0, Qv, eigw, umw);
+      if (TRACE) trace_max(0);
       // gradient weights of the averaged field (nablaQsp, compflux.f90:107-157:
       // divB = dBx/dx + dBy/dy, Jz = dBy/dx - dBx/dy)
       wb0 = Qv[5] * sx + Qv[6] * sy;
@@ -584,7 +617,8 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
       });
       const double sx = msx[N], sy = msy[N];
       double FN[9], Qv[9];
-      face_flux<N, double>(infoN, fam, N, ph, c_h, tN, qnN, sx, sy, FN, Qv, eig, um);
+      face_flux<N, double>(infoN, fam, N, ph, c_h, tN, qnN, sx, sy, FN, Qv, eigw, umw);
+      if (TRACE) trace_max(N);
       const double wbN = Qv[5] * sx + Qv[6] * sy;
       const double wjN = Qv[6] * sx - Qv[5] * sy;
       if (COMPAT) {
@@ -606,7 +640,8 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
     auto interior_point = [&](int r, const double *tr) {
       const double sx = msx[r], sy = msy[r];
       double F[9];
-      iflux_n<double>(tr, c_h, sx, sy, F, um);
+      iflux_n<double>(tr, c_h, sx, sy, F, umw);
+      if (TRACE) trace_max(r);
       const double wb = tr[5] * sx + tr[6] * sy;
       const double wj = tr[6] * sx - tr[5] * sy;
 #pragma unroll
@@ -797,7 +832,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
 #pragma unroll
         for (int v = V0; v < V1; ++v) a.resid_f[v + 9 * pf] = R[v];
       }
-      if (DIVB && V0 == 0) a.divb[(size_t)tile * N2 * T + (size_t)p * T + ci] = divB;
+      if ((DIVB || TRACE) && V0 == 0) a.divb[(size_t)tile * N2 * T + (size_t)p * T + ci] = divB;
       if (RK) {
         const size_t off = (size_t)tile * G::QT;
         // several registers (FiveStageRk's last stage): their weighted sum,
@@ -854,11 +889,25 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
   {
     constexpr int NW = STAGE_THREADS / 64;
     const int w = tid >> 6, l = tid & 63;
+    const double el = eig, ul = um;
     eig = wave_max(eig);
     um = wave_max(um);
     if (NORMS) {
       nres = wave_sum(nres);
       ndiv = wave_sum(ndiv);
+    }
+    if (TRACE) {   // the smallest code that attains the wave's maxima
+      const int none = 0x7fffffff;
+      int ce = valid && el == eig ? flux_point_code<N>(cell, fam, line, re) : none;
+      int cu = valid && ul == um ? flux_point_code<N>(cell, fam, line, ru) : none;
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        const int x = __shfl_xor(ce, o, 64), y = __shfl_xor(cu, o, 64);
+        ce = x < ce ? x : ce;
+        cu = y < cu ? y : cu;
+      }
+      nres = ce;   // (codes are exact in a double; a trace launch forms no norms)
+      ndiv = cu;
     }
     if (l == 0) {
       lds[LD::RED + w] = eig;
@@ -870,6 +919,15 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
     if (tid == 0) {
       double e = lds[LD::RED], u = lds[LD::RED + NW];
       double s1 = lds[LD::RED + 2 * NW], s2 = lds[LD::RED + 3 * NW];
+      if (TRACE) {
+        static_assert(!TRACE || (!NORMS && NW == 2), "the codes take the norms' slots");
+        const double e2 = lds[LD::RED + 1], u2 = lds[LD::RED + NW + 1];
+        const double c1 = lds[LD::RED + 2 * NW + 1], c2 = lds[LD::RED + 3 * NW + 1];
+        a.tmax[2 * tile] = e2 > e ? e2 : e;
+        a.tmax[2 * tile + 1] = u2 > u ? u2 : u;
+        a.tloc[2 * tile] = (int)(e2 > e || (e2 == e && c1 < s1) ? c1 : s1);
+        a.tloc[2 * tile + 1] = (int)(u2 > u || (u2 == u && c2 < s2) ? c2 : s2);
+      }
 #pragma unroll
       for (int k = 1; k < NW; ++k) {
         e = lds[LD::RED + k] > e ? lds[LD::RED + k] : e;

@@ -48,9 +48,10 @@ struct sd2d_ctx {
   int *ftab = nullptr;
   int *c2s = nullptr, *s2c = nullptr;          // cell <-> slot maps of the tile shape
   double avf[NMAX * NMAX] = {};               // AV smoothing filter (kernel arguments)
-  double *gmax = nullptr;                       // eigvmax_g, umax_g
-  double *lastch = nullptr;                     // c_h of the last evaluation (per member)
-  unsigned long long *slots = nullptr;
+  // the running maxima: three sets of MSTRIDE per member (sd2d_device.hpp);
+  // mset is the one the next evaluation reads (the last one's is still before it)
+  unsigned long long *maxs = nullptr;
+  int mset = 0;
   double *sm_ind = nullptr;
   double *normbuf = nullptr, *normout = nullptr;
   double *stagef = nullptr;                     // Fortran-layout staging (Q or resid)
@@ -184,38 +185,6 @@ __global__ void k_t2f(const double *__restrict__ t, double *__restrict__ f,
   }
 }
 
-// running maxima: g = max over slots (one block per ensemble member).
-// The values g holds on entry are the ones the stage just finished formed
-// its c_h from (compflux.f90:6), so that c_h is recorded first, with the
-// kernel's own formula.  No NaN reaches the slots: every point adopts a
-// speed only through `speed > running max`, which a NaN never passes
-// (getrusanov.f90:116-123).
-__global__ void k_finalize_max(const unsigned long long *__restrict__ slots,
-                               double *__restrict__ gmax, double *__restrict__ lastch) {
-  __shared__ unsigned long long s[2][NSLOT];
-  const int t = threadIdx.x;
-  slots += 2 * NSLOT * (size_t)blockIdx.x;
-  gmax += 2 * blockIdx.x;
-  if (t == 0) {
-    const double ge = gmax[0], gu = gmax[1];
-    lastch[blockIdx.x] = sqrt(ge * (ge - gu));
-  }
-  s[0][t] = slots[2 * t];
-  s[1][t] = slots[2 * t + 1];
-  __syncthreads();
-  for (int o = NSLOT / 2; o > 0; o >>= 1) {
-    if (t < o) {
-      s[0][t] = s[0][t] > s[0][t + o] ? s[0][t] : s[0][t + o];
-      s[1][t] = s[1][t] > s[1][t + o] ? s[1][t] : s[1][t + o];
-    }
-    __syncthreads();
-  }
-  if (t == 0) {
-    gmax[0] = __longlong_as_double((long long)s[0][0]);
-    gmax[1] = __longlong_as_double((long long)s[1][0]);
-  }
-}
-
 // Non-finite scan of a state in tile layout (the opt-in check of
 // sd2d_set_check_finite): flags[member] = 1 when a tile of that member holds
 // a NaN or an infinity.  Padding slots hold zeros, so they never raise it.
@@ -232,13 +201,25 @@ __global__ void k_scan_finite(const double2 *__restrict__ q, const int *__restri
   }
 }
 
-// set the running maxima (slot 0 = given local maxima, others 0) and g
-__global__ void k_set_max(unsigned long long *slots, double *gmax, double e, double u,
-                          double eg, double ug) {
-  const int t = threadIdx.x;
-  slots[2 * t] = t == 0 ? (unsigned long long)__double_as_longlong(e) : 0ull;
-  slots[2 * t + 1] = t == 0 ? (unsigned long long)__double_as_longlong(u) : 0ull;
-  if (t == 0) { gmax[0] = eg; gmax[1] = ug; }
+// set the running maxima of one member and the pair c_h is formed from
+__global__ void k_set_max(unsigned long long *set, double e, double u, double eg, double ug) {
+  set[0] = as_bits(e);
+  set[1] = as_bits(u);
+  set[2] = as_bits(eg);
+  set[3] = as_bits(ug);
+}
+
+// A member's running maxima from its set (host copy).  No NaN reaches them:
+// every point adopts a speed only through `speed > running max`, which a NaN
+// never passes (getrusanov.f90:116-123).
+static sd2d_maxima fold_maxima(const unsigned long long *set) {
+  const bool apart = set[2] != MAX_NONE;
+  sd2d_maxima r;
+  std::memcpy(&r.eigvmax, set, 8);
+  std::memcpy(&r.umax, set + 1, 8);
+  std::memcpy(&r.eigvmax_g, set + (apart ? 2 : 0), 8);
+  std::memcpy(&r.umax_g, set + (apart ? 3 : 1), 8);
+  return r;
 }
 
 // deterministic sum of the per-tile norm partials (single block, fixed order)
@@ -456,12 +437,23 @@ static int collect_profile(sd2d_ctx *c) {
   return SD2D_OK;
 }
 
+// set k (mod 3) of the running maxima, at member `mem`
+static unsigned long long *max_set(const sd2d_ctx *c, int k, int mem = 0) {
+  return c->maxs + (size_t)MSTRIDE * ((size_t)(k % 3) * c->nmem + mem);
+}
+
+// the sets of the next evaluation
+static void set_maxima(const sd2d_ctx *c, StageArgs &a) {
+  a.mread = max_set(c, c->mset);
+  a.mwrite = max_set(c, c->mset + 1);
+  a.mclear = max_set(c, c->mset + 2);
+}
+
 static StageArgs base_args(sd2d_ctx *c) {
   StageArgs a{};
   a.met = c->met;
   a.ftab = c->ftab;
-  a.gmax = c->gmax;
-  a.slots = c->slots;
+  set_maxima(c, a);
   std::memcpy(a.avf, c->avf, sizeof(a.avf));
   a.ncell = c->ncell;
   a.ntile = c->ntile;
@@ -500,12 +492,8 @@ static int check_finite_now(sd2d_ctx *c) {
   return SD2D_OK;
 }
 
-static int finalize_stage(sd2d_ctx *c) {
-  hipLaunchKernelGGL(k_finalize_max, dim3(c->nmem), dim3(NSLOT), 0, c->stream, c->slots, c->gmax,
-                     c->lastch);
-  HIPCHK(c, hipGetLastError());
-  return SD2D_OK;
-}
+// After an evaluation's launch: the set it raised is the next one's.
+static void rotate_maxima(sd2d_ctx *c) { c->mset = (c->mset + 1) % 3; }
 
 // Device allocations and uploads of a context from its host tables.  An
 // ensemble group passes its members' per-tile info, time steps and free
@@ -559,11 +547,9 @@ static int ctx_upload(sd2d_ctx *c, const HostTables &tb, int nwall, int nmem,
   CK(hipMalloc(&c->ftab, ft.size() * sizeof(int)));
   CK(hipMalloc(&c->c2s, tb.c2s.size() * sizeof(int)));
   CK(hipMalloc(&c->s2c, tb.s2c.size() * sizeof(int)));
-  CK(hipMalloc(&c->gmax, 2 * (size_t)nmem * sizeof(double)));
-  CK(hipMalloc(&c->lastch, (size_t)nmem * sizeof(double)));
+  c->nmem = nmem;
+  CK(hipMalloc(&c->maxs, 3 * (size_t)MSTRIDE * nmem * sizeof(unsigned long long)));
   CK(hipMalloc(&c->nfflag, (size_t)nmem * sizeof(int)));
-  CK(hipMemsetAsync(c->lastch, 0, (size_t)nmem * sizeof(double), c->stream));
-  CK(hipMalloc(&c->slots, 2 * NSLOT * (size_t)nmem * sizeof(unsigned long long)));
   CK(hipMalloc(&c->sm_ind, 2 * (size_t)nc * sizeof(double)));
   CK(hipMalloc(&c->normbuf, 2 * (size_t)nt * sizeof(double)));
   CK(hipMalloc(&c->normout, 2 * sizeof(double)));
@@ -607,11 +593,11 @@ static int ctx_upload(sd2d_ctx *c, const HostTables &tb, int nwall, int nmem,
     CK(hipMemcpyAsync(c->phm, ph.data(), ph.size() * sizeof(Phys), hipMemcpyHostToDevice,
                       c->stream));
   }
-  c->nmem = nmem;
-  for (int k = 0; k < nmem; ++k) {
-    hipLaunchKernelGGL(k_set_max, dim3(1), dim3(NSLOT), 0, c->stream, c->slots + 2 * NSLOT * (size_t)k,
-                       c->gmax + 2 * k, 0.0, 0.0, 0.0, 0.0);
-    CK(hipGetLastError());
+  {
+    std::vector<unsigned long long> m(3 * (size_t)MSTRIDE * nmem, 0ull);
+    for (size_t k = 0; k < 3 * (size_t)nmem; ++k)
+      m[k * MSTRIDE + 2] = m[k * MSTRIDE + 3] = MAX_NONE;
+    CK(hipMemcpy(c->maxs, m.data(), m.size() * sizeof(m[0]), hipMemcpyHostToDevice));
   }
   CK(hipStreamSynchronize(c->stream));
 #undef CK
@@ -665,7 +651,8 @@ int sd2d_create(const sd2d_mesh *m, const sd2d_params *p, sd2d_ctx **out) {
   c->xs.assign(m->xs, m->xs + N);
   {
     // one run: member 0 and the valid cells of every tile
-    const std::vector<int> tinfo(tb.tvalid.begin(), tb.tvalid.end());
+    std::vector<int> tinfo(tb.tvalid.begin(), tb.tvalid.end());
+    tinfo[0] |= TI_FIRST;
     const int r = ctx_upload(c, tb, m->nwall, 1, &tinfo, nullptr, nullptr);
     if (r) { g_err = c->err; sd2d_destroy(c); return r; }
   }
@@ -679,7 +666,7 @@ void sd2d_destroy(sd2d_ctx *c) {
   adj_free(c->adj);
   for (double *b : c->q) if (b) (void)hipFree(b);
   for (double *b : c->fsr) if (b) (void)hipFree(b);
-  void *ptrs[] = {c->met, c->metf, c->ftab, c->gmax, c->lastch, c->nfflag, c->slots, c->sm_ind, c->normbuf,
+  void *ptrs[] = {c->met, c->metf, c->ftab, c->maxs, c->nfflag, c->sm_ind, c->normbuf,
                   c->normout, c->stagef, c->nablaf, c->gq, c->dei, c->visres, c->metw,
                   c->c2s, c->s2c, c->tinfo, c->dtm, c->phm};
   for (void *b : ptrs) if (b) (void)hipFree(b);
@@ -720,7 +707,7 @@ int sd2d_set_state(sd2d_ctx *c, const double *q, const sd2d_maxima *mx) {
     c->next_stage = 1;   // a step in progress is abandoned
   }
   if (mx) {
-    hipLaunchKernelGGL(k_set_max, dim3(1), dim3(NSLOT), 0, c->stream, c->slots, c->gmax,
+    hipLaunchKernelGGL(k_set_max, dim3(1), dim3(1), 0, c->stream, max_set(c, c->mset),
                        mx->eigvmax, mx->umax, mx->eigvmax_g, mx->umax_g);
     HIPCHK(c, hipGetLastError());
   }
@@ -738,17 +725,10 @@ int sd2d_get_state(sd2d_ctx *c, double *q, sd2d_maxima *mx) {
     HIPCHK(c, hipMemcpyAsync(q, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   }
   if (mx) {
-    unsigned long long s[2 * NSLOT];
-    double g[2];
-    HIPCHK(c, hipMemcpyAsync(s, c->slots, sizeof(s), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(g, c->gmax, sizeof(g), hipMemcpyDeviceToHost, c->stream));
+    unsigned long long m[MSTRIDE];
+    HIPCHK(c, hipMemcpyAsync(m, max_set(c, c->mset), sizeof(m), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    unsigned long long e = 0, u = 0;
-    for (int i = 0; i < NSLOT; ++i) { e = std::max(e, s[2 * i]); u = std::max(u, s[2 * i + 1]); }
-    long long ei = (long long)e, ui = (long long)u;
-    std::memcpy(&mx->eigvmax, &ei, 8);
-    std::memcpy(&mx->umax, &ui, 8);
-    mx->eigvmax_g = g[0]; mx->umax_g = g[1];
+    *mx = fold_maxima(m);
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return SD2D_OK;
@@ -765,7 +745,6 @@ int sd2d_compresid(sd2d_ctx *c, double *resid_out, double *nablaqs_out) {
   SD2D_NOT_MID_STEP(c, "sd2d_compresid");
   const size_t n = (size_t)c->ncell * 9 * c->N * c->N;
   if (!c->nablaf) HIPCHK(c, hipMalloc(&c->nablaf, 2 * n * sizeof(double)));
-  int r;
   StageArgs a = base_args(c);
   a.qin = c->q[c->cur];
   a.resid_f = c->stagef;
@@ -778,8 +757,7 @@ int sd2d_compresid(sd2d_ctx *c, double *resid_out, double *nablaqs_out) {
   }
   HIPCHK(c, launch_stage(c, a, mode));
   c->have_av = (mode & M_AV) != 0;
-  r = finalize_stage(c);
-  if (r) return r;
+  rotate_maxima(c);
   if (resid_out)
     HIPCHK(c, hipMemcpyAsync(resid_out, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   if (nablaqs_out)
@@ -831,8 +809,7 @@ int sd2d_compresid_noalloc(sd2d_ctx *c, double *resid_out, double *nablaqs_out) 
   }
   HIPCHK(c, launch_stage_raw(c, a, mode));
   c->have_av = (mode & M_AV) != 0;
-  const int r = finalize_stage(c);
-  if (r) return r;
+  rotate_maxima(c);
   if (resid_out)
     HIPCHK(c, hipMemcpyAsync(resid_out, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   if (nablaqs_out)
@@ -853,13 +830,15 @@ static int step_rk(sd2d_ctx *c, bool norms, int only = 0) {
     if (only > 0 && ++idx != only) return 0;
     if (mode & M_NORMS) a.normbuf = c->normbuf;
     a.rev = c->nlaunch++ & 1;   // alternate the tile order stage by stage
+    set_maxima(c, a);
     if (c->vis) {
       HIPCHK(c, launch_vis(c, a.qin));
       a.visres = c->visres;
       mode |= M_VIS;
     }
     HIPCHK(c, launch_stage(c, a, mode));
-    return finalize_stage(c);
+    rotate_maxima(c);
+    return 0;
   };
   const int r = (c->p.k_stage == 5) ? fsrk_sequence(rb, c->p.dt, norms, av, base_args(c), launch)
                                     : s5p3_sequence(rb, c->p.dt, norms, av, base_args(c), launch);
@@ -1096,10 +1075,15 @@ int sd2d_get_profile(sd2d_ctx *c, double *stage_ms, int32_t *nlaunch) {
 
 int sd2d_get_diag(sd2d_ctx *c, sd2d_diag *d) {
   if (!c || !d) return fail(c, SD2D_EINVAL, "NULL argument");
-  double g[2], ch = 0.0;
-  HIPCHK(c, hipMemcpyAsync(g, c->gmax, sizeof(g), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(&ch, c->lastch, sizeof(ch), hipMemcpyDeviceToHost, c->stream));
+  // c_h of the last evaluation is formed from the set before the current one
+  unsigned long long m[2][MSTRIDE];
+  HIPCHK(c, hipMemcpyAsync(m[0], max_set(c, c->mset), sizeof(m[0]), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipMemcpyAsync(m[1], max_set(c, c->mset + 2), sizeof(m[1]), hipMemcpyDeviceToHost,
+                           c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  const sd2d_maxima now = fold_maxima(m[0]), last = fold_maxima(m[1]);
+  const double g[2] = {now.eigvmax_g, now.umax_g};
+  const double ch = std::sqrt(last.eigvmax_g * (last.eigvmax_g - last.umax_g));
   d->resid_rms = c->resid_rms;
   d->divb_rms = c->divb_rms;
   d->eigvmax_g = g[0];
@@ -1199,10 +1183,11 @@ int sd2d_get_av(sd2d_ctx *c, double *sm_ind, double *muav, double *epsilon0) {
   if (c->p.artiv != 1 || c->p.vismode != 1)
     return fail(c, SD2D_EINVAL, "the AV sensor runs only with vismode=1 and ARTIV=1");
   std::vector<double> sm((size_t)2 * c->ncell);
-  double g[2];
+  unsigned long long m[MSTRIDE];
   HIPCHK(c, hipMemcpyAsync(sm.data(), c->sm_ind, sm.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(g, c->gmax, sizeof(g), hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipMemcpyAsync(m, max_set(c, c->mset), sizeof(m), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  const double g[1] = {fold_maxima(m).eigvmax_g};
   // AV.f90:106-140
   const double h = std::sqrt(c->p.dxcycl * c->p.dycycl / (double)c->p.ncellglob);
   const double eps = g[0] * h / (double)(c->N - 1) * 0.05;

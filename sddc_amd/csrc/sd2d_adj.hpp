@@ -39,7 +39,7 @@ struct AdjArgs {
   const double *divb;      // divB of q per solution point [tile][p][ci]
   const double *met;
   const int *ftab;
-  const int *tinfo;        // per tile: member << 6 | valid cells
+  const int *tinfo;        // per tile: member << 6 | TI_FIRST | valid cells
   const Phys *phm;         // free stream
   const double *gm;        // eigvmax_g, umax_g that the evaluation's c_h came from
   double *qbar, *abar;     // cotangents of Qin and Qaux (abar may be null)
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void adj_stage_kernel(AdjArgs a, 
     for (int k = 0; k < NSW - 1; ++k) dst[l + k * 64] = st[k];
     if (l + (NSW - 1) * 64 < NV2) dst[l + (NSW - 1) * 64] = st[NSW - 1];
   }
-  const bool valid = line < N && ci < (ti & 63);
+  const bool valid = line < N && ci < (ti & TI_VALID);
   const double *mt = a.met + (size_t)tile * G::NM * T + ci;
   const int p0 = fam ? line : N * line, ps = fam ? N : 1;
   const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;

@@ -69,35 +69,26 @@ static void adj_free(AdjState *A) {
 
 static size_t state_len(const sd2d_ctx *c) { return (size_t)c->ntile * 9 * c->N * c->N * c->cpw; }
 
-// The running maxima (slots and gmax of one run) to and from four doubles on
-// the device: eigvmax, umax, eigvmax_g, umax_g.
-__global__ void k_save_max(const unsigned long long *slots, const double *gmax, double *m) {
-  double e = __longlong_as_double((long long)slots[2 * threadIdx.x]);
-  double u = __longlong_as_double((long long)slots[2 * threadIdx.x + 1]);
-  __shared__ double s[2][NSLOT / 64];
-  e = wave_max(e);
-  u = wave_max(u);
-  if ((threadIdx.x & 63) == 0) {
-    s[0][threadIdx.x >> 6] = e;
-    s[1][threadIdx.x >> 6] = u;
+// The running maxima of one run (a set) to and from four doubles on the device:
+// eigvmax, umax, eigvmax_g, umax_g; `only_g` the last two alone.
+__global__ void k_save_max(const unsigned long long *set, double *m, bool only_g) {
+  const bool apart = set[2] != MAX_NONE;
+  double *g = only_g ? m : m + 2;
+  if (!only_g) {
+    m[0] = __longlong_as_double((long long)set[0]);
+    m[1] = __longlong_as_double((long long)set[1]);
   }
-  __syncthreads();
-  if (threadIdx.x < 2) {
-    double x = s[threadIdx.x][0];
-    for (int k = 1; k < NSLOT / 64; ++k) x = s[threadIdx.x][k] > x ? s[threadIdx.x][k] : x;
-    m[threadIdx.x] = x;
-    m[2 + threadIdx.x] = gmax[threadIdx.x];
-  }
+  g[0] = __longlong_as_double((long long)set[apart ? 2 : 0]);
+  g[1] = __longlong_as_double((long long)set[apart ? 3 : 1]);
 }
-__global__ void k_load_max(const double *m, unsigned long long *slots, double *gmax) {
-  const int t = threadIdx.x;
-  slots[2 * t] = t == 0 ? (unsigned long long)__double_as_longlong(m[0]) : 0ull;
-  slots[2 * t + 1] = t == 0 ? (unsigned long long)__double_as_longlong(m[1]) : 0ull;
-  if (t < 2) gmax[t] = m[2 + t];
+__global__ void k_load_max(const double *m, unsigned long long *set) {
+  set[threadIdx.x] = as_bits(m[threadIdx.x]);
 }
 
-__global__ void k_copy2(const double *__restrict__ s, double *__restrict__ d) {
-  if (threadIdx.x < 2) d[threadIdx.x] = s[threadIdx.x];
+static int save_max(sd2d_ctx *c, double *m, bool only_g) {
+  hipLaunchKernelGGL(k_save_max, dim3(1), dim3(1), 0, c->stream, max_set(c, c->mset), m, only_g);
+  HIPCHK(c, hipGetLastError());
+  return SD2D_OK;
 }
 
 static int adj_maxima_get(sd2d_ctx *c, std::array<double, 4> &m) {
@@ -108,7 +99,7 @@ static int adj_maxima_get(sd2d_ctx *c, std::array<double, 4> &m) {
 }
 
 static int adj_maxima_set(sd2d_ctx *c, const std::array<double, 4> &m) {
-  hipLaunchKernelGGL(k_set_max, dim3(1), dim3(NSLOT), 0, c->stream, c->slots, c->gmax, m[0], m[1],
+  hipLaunchKernelGGL(k_set_max, dim3(1), dim3(1), 0, c->stream, max_set(c, c->mset), m[0], m[1],
                      m[2], m[3]);
   HIPCHK(c, hipGetLastError());
   return SD2D_OK;
@@ -149,9 +140,9 @@ static int adj_alloc(sd2d_ctx *c, AdjState *A, int nck, bool steps) {
   ADJGET(A->part, (size_t)c->ntile * ADJ_NPART);
   ADJGET(A->carry, 1);
   ADJGET(A->slots, 2 * NSLOT);
+  ADJGET(A->gm, 12);
   if (!steps) return SD2D_OK;
   for (auto &p : A->t) ADJGET(p, n);
-  ADJGET(A->gm, 12);
   ADJGET(A->tmax, 10 * (size_t)c->ntile);
   ADJGET(A->tloc, 10 * (size_t)c->ntile);
   ADJGET(A->dtile, c->ntile);
@@ -239,14 +230,9 @@ static int adj_stages(sd2d_ctx *c, double *const *qs, bool trace) {
       a.tloc = A->tloc + 2 * (size_t)c->ntile * s;
     }
     HIPCHK(c, launch_stage(c, a, mode));
-    const int r = finalize_stage(c);
-    if (r) return r;
+    rotate_maxima(c);
   }
-  if (trace) {
-    hipLaunchKernelGGL(k_copy2, dim3(1), dim3(64), 0, c->stream, c->gmax, A->gm + 10);
-    HIPCHK(c, hipGetLastError());
-  }
-  return SD2D_OK;
+  return trace ? save_max(c, A->gm + 10, true) : SD2D_OK;
 }
 
 // One evaluation backwards: adj_stage_kernel, then adj_tail_kernel with the
@@ -407,17 +393,15 @@ int sd2d_vjp(sd2d_ctx *c, const double *qbar_final, double jbar, double *qbar_in
     };
     double *qs[6];
     for (int i = 0; i < len; ++i) {
-      hipLaunchKernelGGL(k_save_max, dim3(1), dim3(NSLOT), 0, c->stream, c->slots, c->gmax,
-                         A->segm + 4 * i);
-      HIPCHK(c, hipGetLastError());
+      if ((r = save_max(c, A->segm + 4 * i, false))) return r;
       if (i + 1 == len) break;   // the last step runs once, below
       step_states(i, qs);
       if ((r = adj_stages(c, qs, false))) return r;
     }
     for (int i = len - 1; i >= 0; --i) {
       const int n = n0 + i;   // step n takes Q_n to Q_{n+1}
-      hipLaunchKernelGGL(k_load_max, dim3(1), dim3(NSLOT), 0, c->stream, A->segm + 4 * i, c->slots,
-                         c->gmax);
+      hipLaunchKernelGGL(k_load_max, dim3(1), dim3(MSTRIDE), 0, c->stream, A->segm + 4 * i,
+                         max_set(c, c->mset));
       HIPCHK(c, hipGetLastError());
       step_states(i, qs);
       if ((r = adj_stages(c, qs, true))) return r;
@@ -569,8 +553,11 @@ int sd2d_compresid_vjp(sd2d_ctx *c, const double *rbar, double *qbar, double *ch
   // divB of the state as the stepping kernel forms it for the Powell source,
   // with scratch maxima
   const double *q = c->q[c->cur];
+  if ((r = save_max(c, A->gm, true))) return r;
   StageArgs s = base_args(c);
   s.qin = q;
+  s.mread = nullptr;
+  s.gmax = A->gm;
   s.slots = A->slots;
   s.divb = A->divb;
   HIPCHK(c, launch_stage(c, s, M_DIVB));
@@ -578,10 +565,10 @@ int sd2d_compresid_vjp(sd2d_ctx *c, const double *rbar, double *qbar, double *ch
   a.q = q;
   a.rbar = A->b[1];
   a.divb = A->divb;
-  a.gm = c->gmax;
+  a.gm = A->gm;
   a.qbar = A->b[0];
   HIPCHK(c, hipMemsetAsync(A->carry, 0, sizeof(AdjCarry), c->stream));
-  if ((r = adj_launch(c, a, nullptr, nullptr, c->gmax, &A->carry->ch))) return r;   // raises nothing
+  if ((r = adj_launch(c, a, nullptr, nullptr, A->gm, &A->carry->ch))) return r;   // raises nothing
   if (qbar) {
     if ((r = t2f(c, A->b[0], c->stagef))) return r;
     HIPCHK(c, hipMemcpyAsync(qbar, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));

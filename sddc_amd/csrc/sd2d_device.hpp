@@ -15,6 +15,18 @@ namespace sd2d {
 constexpr int NMAX = 5;
 constexpr int NSLOT = 256;          // running-maximum slots (spread atomics)
 
+// The running maxima of a run (or of one ensemble member) between its residual
+// evaluations, as bit patterns: eigvmax and umax, then eigvmax_g and umax_g
+// that the next c_h is formed from where the caller set them apart (MAX_NONE
+// otherwise).  A context holds three such sets in rotation: an evaluation
+// reads one, raises the next and clears the third, so no launch is needed
+// between evaluations.
+constexpr int MSTRIDE = 4;
+constexpr unsigned long long MAX_NONE = ~0ull;
+// flag of a member's first tile in its tile info (member << 6 | flag | valid
+// cells); at most 20 cells are valid
+constexpr int TI_FIRST = 32, TI_VALID = 31;
+
 // Cells per tile for each order.  One 128-thread workgroup of the stage
 // kernel owns one tile and runs one thread per grid line of each cell (2N
 // lines per cell): 120, 128 and 120 busy threads for N = 5, 4, 3.  Every

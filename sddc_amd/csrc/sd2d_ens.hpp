@@ -69,6 +69,11 @@ static void ens_free_group(sd2d_ens *e, int g) {
   e->grp[g] = nullptr;
 }
 
+// A step moves the state by two of its three buffers and the running maxima
+// by five, that is two, of their three sets, so both stand at position e->cur
+// between steps, whether a graph or direct launches ran the step.
+static void ens_sync_cur(const sd2d_ens *e, sd2d_ctx *c) { c->cur = c->mset = e->cur; }
+
 // (Re)build group g with tile shape `shape`: host tables of every member,
 // concatenated, uploaded into a fresh context.  Member states are not kept.
 static int ens_build_group(sd2d_ens *e, int g, int shape) {
@@ -110,7 +115,7 @@ static int ens_build_group(sd2d_ens *e, int g, int shape) {
     gt.met.insert(gt.met.end(), tb.met.begin(), tb.met.end());
     for (int t = 0; t < tb.ntile; ++t) {
       const int nv = tb.tvalid[t];
-      tinfo.push_back((m.local << 6) | nv);
+      tinfo.push_back((m.local << 6) | (t == 0 ? TI_FIRST : 0) | nv);
     }
     for (int sl = 0; sl < tb.ntile * CPW; ++sl)
       gt.s2c.push_back(tb.s2c[sl] < 0 ? -1 : tb.s2c[sl] + (int)cells);
@@ -150,7 +155,7 @@ static int ens_build_group(sd2d_ens *e, int g, int shape) {
     ENSCHK(e, hipMemcpy(m.s2c, ms2c[k].data(), ms2c[k].size() * sizeof(int), hipMemcpyHostToDevice));
     ++k;
   }
-  c->cur = e->cur;
+  ens_sync_cur(e, c);
   e->grp_shape[g] = shape;
   return SD2D_OK;
 }
@@ -174,8 +179,7 @@ static int ens_member_state(sd2d_ens *e, int i, const double *qin, double *qout,
     ENSCHK(e, hipGetLastError());
   }
   if (mxin) {
-    hipLaunchKernelGGL(k_set_max, dim3(1), dim3(NSLOT), 0, c->stream,
-                       c->slots + 2 * NSLOT * (size_t)m.local, c->gmax + 2 * m.local,
+    hipLaunchKernelGGL(k_set_max, dim3(1), dim3(1), 0, c->stream, max_set(c, e->cur, m.local),
                        mxin->eigvmax, mxin->umax, mxin->eigvmax_g, mxin->umax_g);
     ENSCHK(e, hipGetLastError());
   }
@@ -189,18 +193,11 @@ static int ens_member_state(sd2d_ens *e, int i, const double *qin, double *qout,
     ENSCHK(e, hipMemcpyAsync(qout, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   }
   if (mxout) {
-    std::vector<unsigned long long> s(2 * NSLOT);
-    double gm[2];
-    ENSCHK(e, hipMemcpyAsync(s.data(), c->slots + 2 * NSLOT * (size_t)m.local,
-                             s.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream));
-    ENSCHK(e, hipMemcpyAsync(gm, c->gmax + 2 * m.local, sizeof(gm), hipMemcpyDeviceToHost, c->stream));
+    unsigned long long s[MSTRIDE];
+    ENSCHK(e, hipMemcpyAsync(s, max_set(c, e->cur, m.local), sizeof(s), hipMemcpyDeviceToHost,
+                             c->stream));
     ENSCHK(e, hipStreamSynchronize(c->stream));
-    unsigned long long a = 0, b = 0;
-    for (int k = 0; k < NSLOT; ++k) { a = std::max(a, s[2 * k]); b = std::max(b, s[2 * k + 1]); }
-    long long ai = (long long)a, bi = (long long)b;
-    std::memcpy(&mxout->eigvmax, &ai, 8);
-    std::memcpy(&mxout->umax, &bi, 8);
-    mxout->eigvmax_g = gm[0]; mxout->umax_g = gm[1];
+    *mxout = fold_maxima(s);
   }
   ENSCHK(e, hipStreamSynchronize(c->stream));
   return SD2D_OK;
@@ -209,7 +206,7 @@ static int ens_member_state(sd2d_ens *e, int i, const double *qin, double *qout,
 // The stages of one RK_S5P3 step of group g, on the group's stream.
 static int ens_group_step(sd2d_ens *e, int g) {
   sd2d_ctx *c = e->grp[g];
-  c->cur = e->cur;
+  ens_sync_cur(e, c);
   const bool prof = c->prof;
   c->prof = false;
   const int r = step_rk(c, false);
@@ -395,7 +392,7 @@ static int ens_check_finite(sd2d_ens *e, int steps_done) {
   e->nonfinite.assign(e->nmem, 0);
   for (size_t g = 0; g < e->grp.size(); ++g) {
     sd2d_ctx *c = e->grp[g];
-    c->cur = e->cur;
+    ens_sync_cur(e, c);
     std::vector<int> fl(c->nmem, 0);
     const int r = scan_finite(c, fl.data());
     if (r) { e->err = c->err; return r; }
@@ -426,12 +423,12 @@ int sd2d_ens_step(sd2d_ens *e, int32_t nsteps) {
       m.iter += 1;
     }
     if (e->check_every > 0 && ((s + 1) % e->check_every == 0 || s == nsteps - 1)) {
-      for (sd2d_ctx *c : e->grp) c->cur = e->cur;
+      for (sd2d_ctx *c : e->grp) ens_sync_cur(e, c);
       const int r = ens_check_finite(e, s + 1);
       if (r) return r;
     }
   }
-  for (sd2d_ctx *c : e->grp) c->cur = e->cur;
+  for (sd2d_ctx *c : e->grp) ens_sync_cur(e, c);
   ENSCHK(e, hipStreamSynchronize(e->stream));
   return SD2D_OK;
 }
@@ -498,7 +495,7 @@ int sd2d_ens_tune(sd2d_ens *e, int32_t trial_steps, int32_t *shapes) {
       if (!r && hipEventSynchronize(t1) == hipSuccess) (void)hipEventElapsedTime(&ms, t0, t1);
       (void)hipEventDestroy(t0);
       (void)hipEventDestroy(t1);
-      c->cur = e->cur;
+      ens_sync_cur(e, c);
       if (r) { e->err = c->err; return r; }
       if (ms < best) { best = ms; best_shape = shape; }
     }

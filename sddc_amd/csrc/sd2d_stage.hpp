@@ -48,8 +48,13 @@ struct StageArgs {
   double *rstore;           // resid (tile layout) for FiveStageRk, or null
   const double *met;        // metrics (tile layout)
   const int *ftab;          // per-cell face table (tile layout)
-  const double *gmax;       // eigvmax_g, umax_g of the previous evaluation
-  unsigned long long *slots;  // running maxima, NSLOT x 2 (bit patterns)
+  // the running maxima before this evaluation, to raise and to clear (MSTRIDE
+  // per member); or, mread null (an evaluation outside the sequence), the pair
+  // to form c_h from and NSLOT x 2 slots to raise
+  const unsigned long long *mread;
+  unsigned long long *mwrite, *mclear;
+  const double *gmax;
+  unsigned long long *slots;
   double *sm_ind;           // SM_IND(2,NCELL) or null
   double *normbuf;          // per-tile sums of resid^2 and divB^2, or null
   double *resid_f;          // resid(9,N,N,NCELL) Fortran layout, or null
@@ -68,9 +73,9 @@ struct StageArgs {
   double *gmrec, *tmax;     // tmax[2*tile]: eig, um
   int *tloc;                // tloc[2*tile]
   const int *s2c;           // slot -> mesh cell, for the cell-indexed outputs
-  // per tile (member << 6 | valid cells), member 0 for one run; an
+  // per tile (member << 6 | TI_FIRST | valid cells), member 0 for one run; an
   // ensemble of runs also has per-member dt (qout then uses cr * dt, null
-  // for one run), and gmax / slots hold one entry per member
+  // for one run), and the maxima hold one entry per member
   const int *tinfo;
   const double *dtm;
   int rev;                  // walk the launch order backwards (alternate stages)
@@ -161,6 +166,59 @@ __device__ __forceinline__ double wave_sum(double x) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
   return x;
+}
+
+__device__ __forceinline__ unsigned long long as_bits(double x) {
+  return (unsigned long long)__double_as_longlong(x);
+}
+
+// eigvmax_g and umax_g (ge, gu) that this evaluation's c_h is formed from, and
+// the maxima (me, mu) it starts with.  The member's first tile also carries
+// those over into the set this evaluation raises and clears the set of the
+// evaluation before, whose values nothing reads any more.
+// 32 x 64 cells, N = 4 (launch-bound), 20 steps and the state's download:
+// 1.75 ms when a launch after every stage folded 256 slots into the pair
+// (3.4 us and two launch gaps a stage), 1.52 ms with this.
+__device__ __forceinline__ void lagged_maxima(const StageArgs &a, int ti, int tid, double &ge,
+                                              double &gu, double &me, double &mu) {
+  const size_t mem = ti >> 6;
+  if (!a.mread) {
+    ge = a.gmax[2 * mem];
+    gu = a.gmax[2 * mem + 1];
+    me = mu = -1.0;
+    return;
+  }
+  const unsigned long long *m = a.mread + MSTRIDE * mem;
+  const unsigned long long e = m[0], u = m[1], g = m[2], h = m[3];
+  if ((ti & TI_FIRST) && tid == 0) {
+    unsigned long long *w = a.mwrite + MSTRIDE * mem, *z = a.mclear + MSTRIDE * mem;
+    atomicMax(w, e);
+    atomicMax(w + 1, u);
+    z[0] = z[1] = 0ull;
+    z[2] = z[3] = MAX_NONE;
+  }
+  me = __longlong_as_double((long long)e);
+  mu = __longlong_as_double((long long)u);
+  ge = g != MAX_NONE ? __longlong_as_double((long long)g) : me;
+  gu = g != MAX_NONE ? __longlong_as_double((long long)h) : mu;
+}
+
+// A tile's largest wave speed e and velocity bound u into the running maxima.
+// A maximum is one address that all XCDs share, so an atomic is issued only
+// where the tile raises it, and after a reset (every tile raises it) only
+// where no other tile has raised it as far: 512 x 1024 cells, N = 5, one
+// atomic per tile and value on 256 / 64 addresses: 824 / 920 us; this: 801 us.
+__device__ __forceinline__ void raise_maxima(const StageArgs &a, int mem, double e, double u,
+                                             double me, double mu) {
+  if (!a.mread) {
+    unsigned long long *sl = a.slots + 2 * ((size_t)mem * NSLOT + blockIdx.x % NSLOT);
+    atomicMax(sl, as_bits(e));
+    atomicMax(sl + 1, as_bits(u));
+    return;
+  }
+  unsigned long long *w = a.mwrite + (size_t)MSTRIDE * mem;
+  if (e > me && as_bits(e) > *(volatile unsigned long long *)w) atomicMax(w, as_bits(e));
+  if (u > mu && as_bits(u) > *(volatile unsigned long long *)(w + 1)) atomicMax(w + 1, as_bits(u));
 }
 
 // AV smoothness sensor (AV.f90:14-83) of the cells of one tile, by one
@@ -531,7 +589,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
     for (int k = 0; k < NSW - 1; ++k) dst[l + k * 64] = st[k];
     if (l + (NSW - 1) * 64 < NV2) dst[l + (NSW - 1) * 64] = st[NSW - 1];
   }
-  const int mem = ti >> 6, nvt = ti & 63;
+  const int mem = ti >> 6, nvt = ti & TI_VALID;
   const bool valid = line < N && ci < nvt;
   const double *mt = a.met + (size_t)tile * G::NM * T + ci;
   const int p0 = fam ? line : N * line;      // point of s = 0 on this line
@@ -559,7 +617,8 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
   }
   // the member's lagged maxima, step and free stream (needed from the face
   // fluxes on)
-  const double ge = a.gmax[2 * mem], gu = a.gmax[2 * mem + 1];
+  double ge, gu, me, mu;
+  lagged_maxima(a, ti, tid, ge, gu, me, mu);
   const double cr = a.dtm ? a.cr * a.dtm[mem] : a.cr;   // b * dt of the member
   const Phys &ph = a.phm[mem];                            // the member's free stream
   const double c_h = sqrt(ge * (ge - gu));   // lagged GLM speed, compflux.f90:6
@@ -935,9 +994,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
         s1 += lds[LD::RED + 2 * NW + k];
         s2 += lds[LD::RED + 3 * NW + k];
       }
-      unsigned long long *sl = a.slots + 2 * ((size_t)mem * NSLOT + blockIdx.x % NSLOT);
-      atomicMax(sl, (unsigned long long)__double_as_longlong(e));
-      atomicMax(sl + 1, (unsigned long long)__double_as_longlong(u));
+      raise_maxima(a, mem, e, u, me, mu);
       if (NORMS) {
         a.normbuf[2 * tile] = s1;
         a.normbuf[2 * tile + 1] = s2;

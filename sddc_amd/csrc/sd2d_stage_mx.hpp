@@ -111,7 +111,7 @@ void stage_kernel_mx(StageArgs a, OpsF ops, const float *__restrict__ metf) {
       if (k < NSW - 1 || i < NV2) dst[i] = make_float2(float(st[k].x), float(st[k].y));
     }
   }
-  const int mem = ti >> 6, nvt = ti & 63;
+  const int mem = ti >> 6, nvt = ti & TI_VALID;
   const bool valid = line < N && ci < nvt;
   const float *mtf = metf + (size_t)tile * G::NM * T + ci;
   const double *mt = a.met + (size_t)tile * G::NM * T + ci;
@@ -138,7 +138,8 @@ void stage_kernel_mx(StageArgs a, OpsF ops, const float *__restrict__ metf) {
   }
   // the member's lagged maxima, step and free stream (needed from the face
   // fluxes on)
-  const double ge = a.gmax[2 * mem], gu = a.gmax[2 * mem + 1];
+  double ge, gu, me, mu;
+  lagged_maxima(a, ti, tid, ge, gu, me, mu);
   const double cr = a.dtm ? a.cr * a.dtm[mem] : a.cr;   // b * dt of the member
   const Phys &ph = a.phm[mem];                            // the member's free stream
   const float c_h = float(sqrt(ge * (ge - gu)));   // compflux.f90:6
@@ -385,9 +386,7 @@ void stage_kernel_mx(StageArgs a, OpsF ops, const float *__restrict__ metf) {
           s2 += lds[LD::RED + 3 * NW + k];
         }
       }
-      unsigned long long *sl = a.slots + 2 * ((size_t)mem * NSLOT + blockIdx.x % NSLOT);
-      atomicMax(sl, (unsigned long long)__double_as_longlong(em));
-      atomicMax(sl + 1, (unsigned long long)__double_as_longlong(ummax));
+      raise_maxima(a, mem, em, ummax, me, mu);
       if (NORMS) {
         a.normbuf[2 * tile] = s1;
         a.normbuf[2 * tile + 1] = s2;

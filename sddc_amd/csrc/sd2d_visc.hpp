@@ -45,7 +45,7 @@ struct VisArgs {
   double *gq;              // gradient (go layout)
   double *dei;             // d(e)/dxi, d(e)/deta [tile][k*N2 + p][ci] (walls)
   double *visres;          // dFv + dGv of variables 0-7, state tile layout (qo)
-  const int *tinfo;        // per tile: member << 6 | valid cells
+  const int *tinfo;        // per tile: member << 6 | TI_FIRST | valid cells
   double mu, eta0;
   int ntile, walls;
   int rev, sfam;           // as StageArgs
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void vis_grad_kernel(VisArgs va, 
     if (l + (NSW - 1) * 64 < NV2) dst[l + (NSW - 1) * 64] = st[NSW - 1];
   }
   if (tid == 0) lds[LD::FLAG] = 0.0;
-  const bool valid = line < N && ci < (ti & 63);
+  const bool valid = line < N && ci < (ti & TI_VALID);
   const double *mt = va.met + (size_t)tile * G::NM * T + ci;
   const int p0 = fam ? line : N * line, ps = fam ? N : 1;
   const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;
@@ -442,7 +442,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void vis_flux_kernel(VisArgs va, 
     for (int k = 0; k < NR - 1; ++k) dst[tid + k * STAGE_THREADS] = st[k];
     if (tid + (NR - 1) * STAGE_THREADS < NV2) dst[tid + (NR - 1) * STAGE_THREADS] = st[NR - 1];
   }
-  const bool valid = line < N && ci < (ti & 63);
+  const bool valid = line < N && ci < (ti & TI_VALID);
   const double *mt = va.met + (size_t)tile * G::NM * T + ci;
   const int p0 = fam ? line : N * line, ps = fam ? N : 1;
   const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;

@@ -26,6 +26,7 @@
 #include "sd2d_visc.hpp"
 #include "sd2d_adj.hpp"
 #include "sd2d_rkseq.hpp"
+#include "sd2d_xfer.hpp"
 
 using namespace sd2d;
 
@@ -87,6 +88,7 @@ struct sd2d_ctx {
   size_t nev_used = 0;
   double prof_ms = 0.0;
   int prof_n = 0;
+  RingUser ring;                  // the pinned staging of large copies
   std::string err;
 };
 
@@ -143,6 +145,15 @@ static const char *const vismode_msg =
       return SD2D_EHIP;                                                         \
     }                                                                           \
   } while (0)
+
+// State-sized copies between the caller's arrays and the device, in the order
+// of the context's stream (the caller synchronises).
+static hipError_t to_host(const sd2d_ctx *c, double *host, const double *dev, size_t n) {
+  return HostRing::get().copy(c->stream, host, const_cast<double *>(dev), n * sizeof(double), true);
+}
+static hipError_t to_device(const sd2d_ctx *c, double *dev, const double *host, size_t n) {
+  return HostRing::get().copy(c->stream, const_cast<double *>(host), dev, n * sizeof(double), false);
+}
 
 static int fail(sd2d_ctx *c, int code, const std::string &m) {
   if (c) c->err = m; else g_err = m;
@@ -701,7 +712,7 @@ int sd2d_set_state(sd2d_ctx *c, const double *q, const sd2d_maxima *mx) {
   if (!c) return fail(nullptr, SD2D_EINVAL, "ctx is NULL");
   const size_t n = (size_t)c->ncell * 9 * c->N * c->N;
   if (q) {
-    HIPCHK(c, hipMemcpyAsync(c->stagef, q, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, to_device(c, c->stagef, q, n));
     int r = f2t(c, c->stagef, c->q[c->cur]);
     if (r) return r;
     c->next_stage = 1;   // a step in progress is abandoned
@@ -722,7 +733,7 @@ int sd2d_get_state(sd2d_ctx *c, double *q, sd2d_maxima *mx) {
   if (q) {
     int r = t2f(c, c->q[c->cur], c->stagef);
     if (r) return r;
-    HIPCHK(c, hipMemcpyAsync(q, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, to_host(c, q, c->stagef, n));
   }
   if (mx) {
     unsigned long long m[MSTRIDE];
@@ -759,9 +770,9 @@ int sd2d_compresid(sd2d_ctx *c, double *resid_out, double *nablaqs_out) {
   c->have_av = (mode & M_AV) != 0;
   rotate_maxima(c);
   if (resid_out)
-    HIPCHK(c, hipMemcpyAsync(resid_out, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, to_host(c, resid_out, c->stagef, n));
   if (nablaqs_out)
-    HIPCHK(c, hipMemcpyAsync(nablaqs_out, c->nablaf, 2 * n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, to_host(c, nablaqs_out, c->nablaf, 2 * n));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return SD2D_OK;
 }
@@ -1168,7 +1179,7 @@ int sd2d_plot_nodes(sd2d_ctx *c, int32_t nre, int32_t nnode, const int32_t *xadj
                                 (int)np1, dh, dmu, dq, dav); break;
   }
   PLOTCHK(hipGetLastError());
-  PLOTCHK(hipMemcpyAsync(plotq, dq, (size_t)9 * nnode * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  PLOTCHK(to_host(c, plotq, dq, (size_t)9 * nnode));
   if (plotav)
     PLOTCHK(hipMemcpyAsync(plotav, dav, (size_t)2 * nnode * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));

@@ -374,7 +374,7 @@ int sd2d_vjp(sd2d_ctx *c, const double *qbar_final, double jbar, double *qbar_in
   // cotangent of the final state
   if (qbar_final) {
     const size_t n = (size_t)c->ncell * 9 * c->N * c->N;
-    HIPCHK(c, hipMemcpyAsync(c->stagef, qbar_final, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, to_device(c, c->stagef, qbar_final, n));
     if ((r = f2t(c, c->stagef, A->b[5]))) return r;
   } else {
     HIPCHK(c, hipMemsetAsync(A->b[5], 0, nb, c->stream));
@@ -414,7 +414,7 @@ int sd2d_vjp(sd2d_ctx *c, const double *qbar_final, double jbar, double *qbar_in
   if (qbar_init) {
     if ((r = t2f(c, A->b[5], c->stagef))) return r;
     const size_t n = (size_t)c->ncell * 9 * c->N * c->N;
-    HIPCHK(c, hipMemcpyAsync(qbar_init, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, to_host(c, qbar_init, c->stagef, n));
   }
   AdjCarry cy{};
   HIPCHK(c, hipMemcpyAsync(&cy, A->carry, sizeof(cy), hipMemcpyDeviceToHost, c->stream));
@@ -454,7 +454,7 @@ int sd2d_adj_save(sd2d_ctx *c, const char *prefix) {
   for (int k = 0; k < nck; ++k) {
     int r = t2f(c, A->ck[k], c->stagef);
     if (r) return r;
-    HIPCHK(c, hipMemcpyAsync(q.data(), c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, to_host(c, q.data(), c->stagef, n));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     const std::string path = adj_ck_path(prefix, k);
     const sd2d_maxima m{A->ckm[k][0], A->ckm[k][1], A->ckm[k][2], A->ckm[k][3]};
@@ -514,7 +514,7 @@ int sd2d_adj_load(sd2d_ctx *c, const char *prefix) {
     std::string e = read_restart_file(path.c_str(), c->N, c->ncell, it, t, q);
     if (e.empty()) e = read_max_file(path.c_str(), it, t, m);
     if (!e.empty()) return fail(c, SD2D_EINVAL, e);
-    HIPCHK(c, hipMemcpyAsync(c->stagef, q.data(), n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, to_device(c, c->stagef, q.data(), n));
     if ((r = f2t(c, c->stagef, A->ck[k]))) return r;
     HIPCHK(c, hipStreamSynchronize(c->stream));   // q is reused by the next file
     A->ckm[k] = {m.eigvmax, m.umax, m.eigvmax_g, m.umax_g};
@@ -548,7 +548,7 @@ int sd2d_compresid_vjp(sd2d_ctx *c, const double *rbar, double *qbar, double *ch
   int r = adj_alloc(c, A, 0, false);
   if (r) return r;
   const size_t n = (size_t)c->ncell * 9 * c->N * c->N;
-  HIPCHK(c, hipMemcpyAsync(c->stagef, rbar, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, to_device(c, c->stagef, rbar, n));
   if ((r = f2t(c, c->stagef, A->b[1]))) return r;
   // divB of the state as the stepping kernel forms it for the Powell source,
   // with scratch maxima
@@ -571,7 +571,7 @@ int sd2d_compresid_vjp(sd2d_ctx *c, const double *rbar, double *qbar, double *ch
   if ((r = adj_launch(c, a, nullptr, nullptr, A->gm, &A->carry->ch))) return r;   // raises nothing
   if (qbar) {
     if ((r = t2f(c, A->b[0], c->stagef))) return r;
-    HIPCHK(c, hipMemcpyAsync(qbar, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, to_host(c, qbar, c->stagef, n));
   }
   AdjCarry cy{};
   HIPCHK(c, hipMemcpyAsync(&cy, A->carry, sizeof(cy), hipMemcpyDeviceToHost, c->stream));

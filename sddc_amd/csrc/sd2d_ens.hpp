@@ -170,7 +170,7 @@ static int ens_member_state(sd2d_ens *e, int i, const double *qin, double *qout,
   double *tq = c->q[e->cur] + (size_t)m.tile0 * QT;
   const int blocks = 1024;
   if (qin) {
-    ENSCHK(e, hipMemcpyAsync(c->stagef, qin, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    ENSCHK(e, to_device(c, c->stagef, qin, n));
     switch (N) {
       case 3: hipLaunchKernelGGL(k_f2t<3>, dim3(blocks), dim3(256), 0, c->stream, c->stagef, tq, m.s2c, m.ntile); break;
       case 4: hipLaunchKernelGGL(k_f2t<4>, dim3(blocks), dim3(256), 0, c->stream, c->stagef, tq, m.s2c, m.ntile); break;
@@ -190,7 +190,7 @@ static int ens_member_state(sd2d_ens *e, int i, const double *qin, double *qout,
       default: hipLaunchKernelGGL(k_t2f<5>, dim3(blocks), dim3(256), 0, c->stream, tq, c->stagef, m.c2s, m.ncell); break;
     }
     ENSCHK(e, hipGetLastError());
-    ENSCHK(e, hipMemcpyAsync(qout, c->stagef, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    ENSCHK(e, to_host(c, qout, c->stagef, n));
   }
   if (mxout) {
     unsigned long long s[MSTRIDE];

@@ -153,7 +153,7 @@ class Sd2d:
                     "sd2d_set_state")
 
     def get_state(self):
-        Q = np.zeros((9, self.N, self.N, self.nc), order="F")
+        Q = np.empty((9, self.N, self.N, self.nc), order="F")
         mx = abi.Sd2dMaxima()
         self._check(self.L.sd2d_get_state(self.h, _ptr(Q), C.byref(mx)), "sd2d_get_state")
         return Q, np.array([mx.eigvmax, mx.umax, mx.eigvmax_g, mx.umax_g])
@@ -170,8 +170,8 @@ class Sd2d:
 
     # -- the path ----------------------------------------------------------
     def compresid(self, want_resid=True, want_nabla=True):
-        r = np.zeros((9, self.N, self.N, self.nc), order="F") if want_resid else None
-        g = np.zeros((9, 2, self.N, self.N, self.nc), order="F") if want_nabla else None
+        r = np.empty((9, self.N, self.N, self.nc), order="F") if want_resid else None
+        g = np.empty((9, 2, self.N, self.N, self.nc), order="F") if want_nabla else None
         self._check(self.L.sd2d_compresid(self.h, _ptr(r), _ptr(g)), "sd2d_compresid")
         return r, g
 
@@ -194,7 +194,7 @@ class Sd2d:
         nn = topo.nnode
         xadj = np.ascontiguousarray(topo.xadj, dtype=np.int32)
         occ = np.ascontiguousarray(topo.contrib, dtype=np.int32)
-        q = np.zeros((9, nn), order="F")
+        q = np.empty((9, nn), order="F")
         av = np.zeros((2, nn), order="F") if muav is not None else None
         mu = None if muav is None else np.asfortranarray(muav, dtype=np.float64)
         self._check(self.L.sd2d_plot_nodes(self.h, int(topo.nre), nn, _ptr(xadj), _ptr(occ),
@@ -250,7 +250,7 @@ class Sd2d:
         (rinf, pinf, uinf, vinf, bxinf, byinf) after fwd(); optionally the
         per-evaluation c_h cotangents."""
         qf = None if qbar_final is None else np.asfortranarray(qbar_final, dtype=np.float64)
-        q0 = np.zeros((9, self.N, self.N, self.nc), order="F")
+        q0 = np.empty((9, self.N, self.N, self.nc), order="F")
         pb = np.zeros(6)
         ch = np.zeros(5 * 100000) if want_chbar else None
         self._check(self.L.sd2d_vjp(self.h, _ptr(qf), float(jbar), _ptr(q0), _ptr(pb), _ptr(ch)),
@@ -269,7 +269,7 @@ class Sd2d:
 
     def compresid_vjp(self, rbar):
         rb = np.asfortranarray(rbar, dtype=np.float64)
-        q = np.zeros((9, self.N, self.N, self.nc), order="F")
+        q = np.empty((9, self.N, self.N, self.nc), order="F")
         ch = C.c_double()
         pb = np.zeros(6)
         self._check(self.L.sd2d_compresid_vjp(self.h, _ptr(rb), _ptr(q), C.byref(ch), _ptr(pb)),
@@ -333,7 +333,7 @@ class Sd2dEnsemble:
 
     def get_state(self, i):
         c = self.cases[i]
-        Q = np.zeros((9, c.N, c.N, c.ncell), order="F")
+        Q = np.empty((9, c.N, c.N, c.ncell), order="F")
         mx = abi.Sd2dMaxima()
         self._check(self.L.sd2d_ens_get_state(self.h, i, _ptr(Q), C.byref(mx)),
                     "sd2d_ens_get_state")

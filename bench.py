@@ -390,7 +390,7 @@ def main() -> int:
     ms, nlaunch = g.get_profile()
     g.set_profiling(False)
     avg_s = ms / 1e3 / max(nlaunch, 1)
-    balg = cases.alg_bytes_per_dof_stage(N, case.params.k_stage)
+    balg = cases.alg_bytes_per_dof_stage(N, case.params.k_stage, lines_share=True)
     achieved = ndof * balg / avg_s / 1e9
     d = g.diag()
     nsteps_done = args.warmup + 2 * args.steps
@@ -448,7 +448,8 @@ def main() -> int:
         den[[3, 7, 8]] = nb.max()      # w, Bz, psi: against the largest variable
         l2 = np.sqrt(((a - b) ** 2).sum(axis=1)) / den
         avg_m = ms_m / 1e3 / max(n_m, 1)
-        balg_m = cases.alg_bytes_per_dof_stage(N, case.params.k_stage, metric_bytes=4)
+        balg_m = cases.alg_bytes_per_dof_stage(N, case.params.k_stage, metric_bytes=4,
+                                                lines_share=True)
         vm = ndof * 5 * args.steps / wall_m
         res["mixed"] = {
             "value": vm, "unit": "DOF-stage/s", "ms_per_step": wall_m / args.steps * 1e3,

@@ -152,11 +152,13 @@ def dof(case: M.Case) -> int:
     return case.ncell * case.N * case.N
 
 
-def alg_bytes_per_dof_stage(N: int, k_stage: int = 3, metric_bytes: int = 8) -> float:
+def alg_bytes_per_dof_stage(N: int, k_stage: int = 3, metric_bytes: int = 8,
+                            lines_share: bool = False) -> float:
     """Compulsory HBM bytes per DOF-stage of a fused stage: the RK state
     traffic (RK_S5P3: 13 state passes of 72 B over 5 stages; FiveStageRk:
     18 + the stored residual) plus Jac and the face-normal metric vectors
-    S1(1,:), S2(2,:) read once per stage."""
+    S1(1,:), S2(2,:) read once per stage; with lines_share (4-node cells)
+    the N+1 vectors that the N lines of a family share."""
     state = 13 * 72 / 5 if k_stage == 3 else 18 * 72 / 5
-    metrics = metric_bytes * (N * N + 4 * N * (N + 1)) / (N * N)
+    metrics = metric_bytes * (N * N + 4 * (1 if lines_share else N) * (N + 1)) / (N * N)
     return state + metrics

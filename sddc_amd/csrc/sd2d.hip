@@ -46,6 +46,7 @@ struct sd2d_ctx {
   int cur = 0;                                  // buffer holding the state
   double *fsr[4] = {nullptr, nullptr, nullptr, nullptr};  // FiveStageRk registers
   double *met = nullptr;
+  int mcomp = 0;                                // met (and metf) in the compact form
   int *ftab = nullptr;
   int *c2s = nullptr, *s2c = nullptr;          // cell <-> slot maps of the tile shape
   double avf[NMAX * NMAX] = {};               // AV smoothing filter (kernel arguments)
@@ -395,7 +396,7 @@ static hipError_t launch_stage_raw(sd2d_ctx *c, const StageArgs &a, int mode) {
 template <int N>
 static hipError_t launch_vis_n(sd2d_ctx *c, const double *qin) {
   VisArgs va{};
-  va.qin = qin; va.ftab = c->ftab; va.met = c->met; va.metw = c->metw;
+  va.qin = qin; va.ftab = c->ftab; va.met = c->met; va.mcomp = c->mcomp; va.metw = c->metw;
   va.gq = c->gq; va.dei = c->dei; va.visres = c->visres;
   va.mu = c->p.mu; va.eta0 = c->p.eta0;
   va.ntile = c->ntile; va.walls = c->dei != nullptr; va.tinfo = c->tinfo; va.sfam = c->sfam;
@@ -463,6 +464,7 @@ static void set_maxima(const sd2d_ctx *c, StageArgs &a) {
 static StageArgs base_args(sd2d_ctx *c) {
   StageArgs a{};
   a.met = c->met;
+  a.mcomp = c->mcomp;
   a.ftab = c->ftab;
   set_maxima(c, a);
   std::memcpy(a.avf, c->avf, sizeof(a.avf));
@@ -519,6 +521,7 @@ static int ctx_upload(sd2d_ctx *c, const HostTables &tb, int nwall, int nmem,
   const sd2d_params *p = &c->p;
   const std::vector<int> &ft = tb.ft;
   const std::vector<double> &met = tb.met;
+  c->mcomp = tb.mcomp;
 
 #define CK(call)                                                                   \
   do {                                                                             \
@@ -645,7 +648,7 @@ int sd2d_create(const sd2d_mesh *m, const sd2d_params *p, sd2d_ctx **out) {
   HostTables tb;
   {
     std::string e;
-    const int r = build_host_tables(m, p, tb, e);
+    const int r = build_host_tables(m, p, tb, e, lines_share_metrics(m));
     if (r) { delete c; return fail(nullptr, r, e); }
   }
   const int N = m->N, nc = m->ncell, CPW = tb.cpw;

@@ -38,6 +38,7 @@ struct AdjArgs {
   double cin, ca;          // qbar gets cin * rbar besides, abar ca * rbar
   const double *divb;      // divB of q per solution point [tile][p][ci]
   const double *met;
+  int mcomp;               // as StageArgs
   const int *ftab;
   const int *tinfo;        // per tile: member << 6 | TI_FIRST | valid cells
   const Phys *phm;         // free stream
@@ -411,9 +412,8 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void adj_stage_kernel(AdjArgs a, 
     if (l + (NSW - 1) * 64 < NV2) dst[l + (NSW - 1) * 64] = st[NSW - 1];
   }
   const bool valid = line < N && ci < (ti & TI_VALID);
-  const double *mt = a.met + (size_t)tile * G::NM * T + ci;
+  const MetLine<N, double> ml(a.met, a.mcomp, tile, ci, fam, line);
   const int p0 = fam ? line : N * line, ps = fam ? N : 1;
-  const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;
   const bool i0 = ((info0 >> 3) & 7) == FT_INTERIOR, iN = ((infoN >> 3) & 7) == FT_INTERIOR;
   const bool far0 = i0 && nb0 / QT != tile, farN = iN && nbN / QT != tile;
   const bool nfirst = farN && !far0;   // the end whose traces are gathered first
@@ -432,7 +432,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void adj_stage_kernel(AdjArgs a, 
       Lr[s] = endN ? ops.L[N][s] : ops.L[0][s];
       Mr[s] = endN ? ops.M[N][s] : ops.M[0][s];
     }
-    const double *ji = a.met + ((size_t)nt * G::NM + G::JI) * T + nci;
+    const double *ji = MetLine<N, double>(a.met, a.mcomp, nt, nci, 0, 0).ji;
     sgn = a.ftab[((size_t)nt * 8 + kn * 2 + 1) * T + nci];
     if (staged)
       adj_far_line<N>(lds + LD::Q0, lds + LD::R0, ji, np0, nst, nci, Lr, Mr, a.rscale, tn, Fn, Wn);
@@ -444,11 +444,11 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void adj_stage_kernel(AdjArgs a, 
   if (valid) {
     if (far0 || farN) other_side(nfirst, false);
 #pragma unroll
-    for (int s = 0; s < N; ++s) ji[s] = mt[(G::JI + (fam ? s : line) + N * (fam ? line : s)) * T];
+    for (int s = 0; s < N; ++s) ji[s] = ml.ji[((fam ? s : line) + N * (fam ? line : s)) * T];
 #pragma unroll
     for (int r = 0; r < NF; ++r) {
-      msx[r] = mt[(mx + r + NF * line) * T];
-      msy[r] = mt[(my + r + NF * line) * T];
+      msx[r] = ml.x[r * T];
+      msy[r] = ml.y[r * T];
     }
   }
   const double ge = a.gm[0], gu = a.gm[1];
@@ -653,7 +653,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void adj_stage_kernel(AdjArgs a, 
 // point; a cell's next wall face comes after the barrier).
 template <int N>
 __global__ __launch_bounds__(64) void drag_kernel(const double *q, const int *ftab,
-                                                  const double *met, const double *wq, Ops ops,
+                                                  const double *met, int mcomp, const double *wq, Ops ops,
                                                   double *dtile, double *qbar, double scale) {
   using G = Geo<N>;
   constexpr int T = G::CPW, NF = N + 1;
@@ -671,15 +671,14 @@ __global__ __launch_bounds__(64) void drag_kernel(const double *q, const int *ft
   }
   if (__syncthreads_or(any)) {
     const double *qc = q + (size_t)tile * G::QT;
-    const double *mt = met + (size_t)tile * G::NM * T + ci;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       if (on && bc[k] == FT_WALL) {
         // the face's points: own lines of the family crossing it
         const int fam = (k == 1 || k == 3) ? 0 : 1;
         const int rfp = (k == 0 || k == 3) ? 0 : N;
-        const int mx = fam ? G::S2X : G::S1X;
         const double sgn = (k == 0 || k == 3) ? -1.0 : 1.0;
+        const MetLine<N, double> ml(met, mcomp, tile, ci, fam, line);
         const int p0 = fam ? line : N * line, ps = fam ? N : 1;
         double t[9];
         line_vals<N, double>(qc, p0, ps, ci, [&](int v, const double *x) {
@@ -689,7 +688,7 @@ __global__ __launch_bounds__(64) void drag_kernel(const double *q, const int *ft
         const double ke = 0.5 * (t[1] * t[1] + t[2] * t[2] + t[3] * t[3]) / t[0];
         const double pr = g1 * (t[4] - ke - 0.5 * (t[5] * t[5] + t[6] * t[6] + t[7] * t[7]) -
                                 0.5 * t[8] * t[8]);
-        const double nx = sgn * mt[(mx + rfp + NF * line) * T];
+        const double nx = sgn * ml.x[rfp * T];
         d += wq[line] * pr * nx;
         if (qbar) {
           const double c = scale * wq[line] * nx * g1;
@@ -763,10 +762,9 @@ __device__ __forceinline__ void adj_point_geom(const AdjArgs &a, const Ops &ops,
                                                bool &endN) {
   using G = Geo<N>;
   constexpr int T = G::CPW, NF = N + 1;
-  const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;
-  const double *mt = a.met + (size_t)tile * G::NM * T + ci;
-  sx = mt[(mx + r + NF * line) * T];
-  sy = mt[(my + r + NF * line) * T];
+  const MetLine<N, double> ml(a.met, a.mcomp, tile, ci, fam, line);
+  sx = ml.x[r * T];
+  sy = ml.y[r * T];
   info = 0; k = 0; nbase = 0; np0 = 0; nst = 1; endN = false;
   if (r != 0 && r != N) return;
   int nfp;

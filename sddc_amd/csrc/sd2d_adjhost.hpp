@@ -179,9 +179,9 @@ static int drag_eval(sd2d_ctx *c, const double *q, bool sum, double *qbar, doubl
   AdjState *A = c->adj;
   const dim3 grid(c->ntile), block(64);
   switch (c->N) {
-    case 3: hipLaunchKernelGGL(drag_kernel<3>, grid, block, 0, c->stream, q, c->ftab, c->met, A->wq, c->ops, A->dtile, qbar, scale); break;
-    case 4: hipLaunchKernelGGL(drag_kernel<4>, grid, block, 0, c->stream, q, c->ftab, c->met, A->wq, c->ops, A->dtile, qbar, scale); break;
-    default: hipLaunchKernelGGL(drag_kernel<5>, grid, block, 0, c->stream, q, c->ftab, c->met, A->wq, c->ops, A->dtile, qbar, scale); break;
+    case 3: hipLaunchKernelGGL(drag_kernel<3>, grid, block, 0, c->stream, q, c->ftab, c->met, c->mcomp, A->wq, c->ops, A->dtile, qbar, scale); break;
+    case 4: hipLaunchKernelGGL(drag_kernel<4>, grid, block, 0, c->stream, q, c->ftab, c->met, c->mcomp, A->wq, c->ops, A->dtile, qbar, scale); break;
+    default: hipLaunchKernelGGL(drag_kernel<5>, grid, block, 0, c->stream, q, c->ftab, c->met, c->mcomp, A->wq, c->ops, A->dtile, qbar, scale); break;
   }
   HIPCHK(c, hipGetLastError());
   if (sum) {
@@ -263,7 +263,7 @@ static int adj_launch(sd2d_ctx *c, const AdjArgs &a, const double *tmax, const i
 static AdjArgs adj_args(sd2d_ctx *c) {
   AdjState *A = c->adj;
   AdjArgs a{};
-  a.rscale = 1.0; a.met = c->met; a.ftab = c->ftab; a.tinfo = c->tinfo; a.phm = c->phm;
+  a.rscale = 1.0; a.met = c->met; a.mcomp = c->mcomp; a.ftab = c->ftab; a.tinfo = c->tinfo; a.phm = c->phm;
   a.part = A->part; a.alpha = c->ph.alpha; a.ntile = c->ntile;
   return a;
 }

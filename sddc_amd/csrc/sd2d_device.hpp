@@ -45,6 +45,10 @@ template <int N> struct Geo {
   static constexpr int S2Y = 3 * N * (N + 1);
   static constexpr int JI = 4 * N * (N + 1);
   static constexpr int NM = 4 * N * (N + 1) + N * N;
+  // the compact form, where the metric vectors are the same on every line of a
+  // family: S1(1,1:2,rfp), S2(2,1:2,rfp), 1/Jac
+  static constexpr int JIC = 4 * (N + 1);
+  static constexpr int NMC = JIC + N * N;
   static constexpr int QT = 9 * N2 * CPW;   // doubles per state tile
 };
 
@@ -81,6 +85,29 @@ inline int qo_rt(int N, int v, int p, int ci) {
   const int T = cpw_of(N), N2 = N * N;
   return v < 8 ? (((v >> 1) * N2 + p) * T + ci) * 2 + (v & 1) : 8 * N2 * T + p * T + ci;
 }
+
+// The metrics of one cell as a line thread reads them, from the full table
+// or the compact one (`comp`).  On 4-node cells the vector S1(1,:) of a xi-line
+// is (y_eta, -x_eta), a function of xi alone, and S2(2,:) of an eta-line one of
+// eta alone, so the N lines of a family share N+1 vectors: the host stores
+// them once where they are equal bit for bit (8-node cells keep the full
+// table).  A cell then has 49 metric values instead of 145 at N = 5, 16 % of
+// the bytes of a stage without an RK register, and the lanes of one load touch
+// one run of cells instead of N.
+// Stages of 512 x 1024 cells, N = 5: 691 / 791 / 826 -> 673 / 750 / 795 us
+// (none, one RK register, with the sensor); 512 x 512, N = 4, mixed: 189 / 228 /
+// 236 -> 184 / 222 / 230 us.
+template <int N, typename R> struct MetLine {
+  static constexpr int T = cpw_of(N), NF = N + 1;
+  const R *x, *y;   // the line's metric vector at flux point r: x[r*T], y[r*T]
+  const R *ji;      // 1/Jac of solution point (is, js): ji[(js + N*is)*T]
+  __device__ __forceinline__ MetLine(const R *met, int comp, int tile, int ci, int fam, int line) {
+    const R *b = met + (size_t)tile * ((comp ? Geo<N>::NMC : Geo<N>::NM) * T) + ci;
+    x = b + (comp ? (fam ? 2 * NF : 0) : (fam ? Geo<N>::S2X : 0) + NF * line) * T;
+    y = x + (comp ? NF : N * NF) * T;
+    ji = b + (comp ? Geo<N>::JIC : Geo<N>::JI) * T;
+  }
+};
 
 // Values handed between lanes of one wavefront through LDS: the LDS unit
 // performs a wavefront's operations in order, so no wait is needed between

@@ -76,7 +76,7 @@ static void ens_sync_cur(const sd2d_ens *e, sd2d_ctx *c) { c->cur = c->mset = e-
 
 // (Re)build group g with tile shape `shape`: host tables of every member,
 // concatenated, uploaded into a fresh context.  Member states are not kept.
-static int ens_build_group(sd2d_ens *e, int g, int shape) {
+static int ens_build_group(sd2d_ens *e, int g, int shape, bool full_metrics = false) {
   ens_free_group(e, g);
   ens_drop_graphs(e);
   const int N = e->grp_n[g], CPW = cpw_of(N), N2 = N * N, QT = 9 * N2 * CPW;
@@ -88,6 +88,10 @@ static int ens_build_group(sd2d_ens *e, int g, int shape) {
   std::vector<std::vector<int>> mc2s, ms2c;
   int nloc = 0, nwall = 0;
   long long tiles = 0, cells = 0;
+  // one metric layout for the whole group
+  bool compact = !full_metrics;
+  for (int i = 0; i < e->nmem && compact; ++i)
+    if (e->mem[i].group == g) compact = lines_share_metrics(&e->meshes[i]);
   for (int i = 0; i < e->nmem; ++i) {
     EnsMember &m = e->mem[i];
     if (m.group != g) continue;
@@ -95,8 +99,10 @@ static int ens_build_group(sd2d_ens *e, int g, int shape) {
     p.tile_shape = shape;
     HostTables tb;
     std::string err;
-    const int r = build_host_tables(&e->meshes[i], &p, tb, err);
+    const int r = build_host_tables(&e->meshes[i], &p, tb, err, compact);
     if (r) return ens_fail(e, r, "member " + std::to_string(i) + ": " + err);
+    if (compact && !tb.mcomp) return ens_build_group(e, g, shape, true);
+    gt.mcomp = tb.mcomp;
     if (nloc == 0) { gt.ops = tb.ops; gt.ph = tb.ph; gt.av = tb.av; }
     else if (std::memcmp(&gt.ops, &tb.ops, sizeof(Ops)) != 0)
       return ens_fail(e, SD2D_EINVAL, "members of one order differ in Lmat/Mmat");

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <map>
 #include <cstdint>
 #include <string>
@@ -25,6 +26,7 @@ struct HostTables {
   std::vector<int> ft;       // [tile][k][{neighbour base, info}][ci]
   std::vector<int> tvalid;   // valid cells of each tile (its first slots)
   std::vector<double> met;   // [tile][metric slot][ci]
+  int mcomp = 0;             // met is the compact table
   std::vector<double> av;    // AV smoothing filter F[is][k] (N x N)
   std::vector<double> metw;  // viscous path: other-family metrics at line ends
 };
@@ -380,9 +382,29 @@ inline std::vector<int> tile_order(int nt, int CPW, int tile_doubles,
   return bisection_order(nt, LEAF, xadj, ladj);
 }
 
-// Everything the kernels read besides the state.
+// Whether the metric vectors are, bit for bit, the same on every line of a
+// family in every cell (4-node cells), so that the compact table holds them.
+inline bool lines_share_metrics(const sd2d_mesh *m) {
+  const int N = m->N, NF = N + 1;
+  auto same = [](double a, double b) { return std::memcmp(&a, &b, sizeof(double)) == 0; };
+  for (int cell = 0; cell < m->ncell; ++cell) {
+    const double *s1 = m->s1 + (size_t)4 * NF * N * cell, *s2 = m->s2 + (size_t)4 * NF * N * cell;
+    for (int line = 1; line < N; ++line)
+      for (int r = 0; r < NF; ++r) {
+        const double *a = s1 + 4 * (r + NF * line), *a0 = s1 + 4 * r;
+        const double *b = s2 + 4 * (line + N * r), *b0 = s2 + 4 * (N * r);
+        if (!same(a[0], a0[0]) || !same(a[2], a0[2]) || !same(b[1], b0[1]) || !same(b[3], b0[3]))
+          return false;
+      }
+  }
+  return true;
+}
+
+// Everything the kernels read besides the state.  `compact` asks for the
+// compact metric table (the caller found that lines_share_metrics); t.mcomp
+// says whether it was made.
 inline int build_host_tables(const sd2d_mesh *m, const sd2d_params *p, HostTables &t,
-                             std::string &err) {
+                             std::string &err, bool compact = false) {
   using hostdetail::put_tile;
   const int N = m->N, nc = m->ncell, CPW = cpw_of(N), N2 = N * N;
   t.N = N; t.ncell = nc; t.cpw = CPW; t.ntile = (nc + CPW - 1) / CPW;
@@ -453,16 +475,30 @@ inline int build_host_tables(const sd2d_mesh *m, const sd2d_params *p, HostTable
   }
 
   // metrics: S1(1,1:2,rfp,js), S2(2,1:2,is,rfp), 1/Jac(is,js)
-  const int NM = 4 * N * (N + 1) + N2;
+  // (a face whose right cell takes the left's vector is no longer the same on
+  // every line, so such a mesh keeps the full table)
+  t.mcomp = compact && adopt.empty();
+  const int NM = (t.mcomp ? 4 * (N + 1) : 4 * N * (N + 1)) + N2;
   t.met.assign((size_t)nt * NM * CPW, 0.0);
   for (int cell = 0; cell < nc; ++cell) {
-    for (int js = 0; js < N; ++js)
+    if (t.mcomp) {
+      const int NF = N + 1;
+      for (int r = 0; r < NF; ++r) {
+        const double *s1 = m->s1 + 4 * (r + (size_t)NF * N * cell);
+        const double *s2 = m->s2 + 4 * ((size_t)N * (r + (size_t)NF * cell));
+        put_tile<double>(t.met, NM, CPW, t.c2s[cell], r, s1[0]);
+        put_tile<double>(t.met, NM, CPW, t.c2s[cell], NF + r, s1[2]);
+        put_tile<double>(t.met, NM, CPW, t.c2s[cell], 2 * NF + r, s2[1]);
+        put_tile<double>(t.met, NM, CPW, t.c2s[cell], 3 * NF + r, s2[3]);
+      }
+    }
+    for (int js = 0; js < N && !t.mcomp; ++js)
       for (int rfp = 0; rfp <= N; ++rfp) {
         const size_t b = 2 * (2 * (rfp + (size_t)(N + 1) * (js + (size_t)N * cell)));
         put_tile<double>(t.met, NM, CPW, t.c2s[cell], 0 + rfp + (N + 1) * js, m->s1[b + 0]);
         put_tile<double>(t.met, NM, CPW, t.c2s[cell], N * (N + 1) + rfp + (N + 1) * js, m->s1[b + 2]);
       }
-    for (int rfp = 0; rfp <= N; ++rfp)
+    for (int rfp = 0; rfp <= N && !t.mcomp; ++rfp)
       for (int is = 0; is < N; ++is) {
         const size_t b = 2 * (2 * (is + (size_t)N * (rfp + (size_t)(N + 1) * cell)));
         put_tile<double>(t.met, NM, CPW, t.c2s[cell], 2 * N * (N + 1) + rfp + (N + 1) * is, m->s2[b + 1]);
@@ -470,7 +506,7 @@ inline int build_host_tables(const sd2d_mesh *m, const sd2d_params *p, HostTable
       }
     for (int js = 0; js < N; ++js)
       for (int is = 0; is < N; ++is)
-        put_tile<double>(t.met, NM, CPW, t.c2s[cell], 4 * N * (N + 1) + js + N * is,
+        put_tile<double>(t.met, NM, CPW, t.c2s[cell], NM - N2 + js + N * is,
                          1.0 / m->jac[is + N * (js + (size_t)N * cell)]);
   }
   // the right cell of a face whose normals differ by rounding takes the

@@ -47,6 +47,7 @@ struct StageArgs {
   double *qout;             // may alias aux[i] (pointwise in-place)
   double *rstore;           // resid (tile layout) for FiveStageRk, or null
   const double *met;        // metrics (tile layout)
+  int mcomp;                // met is the compact table (MetLine)
   const int *ftab;          // per-cell face table (tile layout)
   // the running maxima before this evaluation, to raise and to clear (MSTRIDE
   // per member); or, mread null (an evaluation outside the sequence), the pair
@@ -591,10 +592,9 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
   }
   const int mem = ti >> 6, nvt = ti & TI_VALID;
   const bool valid = line < N && ci < nvt;
-  const double *mt = a.met + (size_t)tile * G::NM * T + ci;
+  const MetLine<N, double> ml(a.met, a.mcomp, tile, ci, fam, line);
   const int p0 = fam ? line : N * line;      // point of s = 0 on this line
   const int ps = fam ? N : 1;                // point stride along the line
-  const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;
   const double *qs = lds + LD::Q0;           // the staged tile (qo layout)
   // ---- neighbour traces at both end faces: gathered from memory for a
   //      neighbour in another tile, formed from the staged tile after the
@@ -611,8 +611,8 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
   if (valid) {
 #pragma unroll
     for (int r = 0; r < NF; ++r) {
-      msx[r] = mt[(mx + r + NF * line) * T];
-      msy[r] = mt[(my + r + NF * line) * T];
+      msx[r] = ml.x[r * T];
+      msy[r] = ml.y[r * T];
     }
   }
   // the member's lagged maxima, step and free stream (needed from the face
@@ -745,7 +745,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
 #pragma unroll
     for (int s = 0; s < N; ++s) {
       const int is = fam ? line : s, js = fam ? s : line;
-      jis[s] = mt[(G::JI + js + N * is) * T];
+      jis[s] = ml.ji[(js + N * is) * T];
     }
   }
   if (RK && NAUX == 1 && valid) {
@@ -820,12 +820,12 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
 #pragma unroll
         for (int r = 0; r < NF; ++r) {
           const double t = qv[r] * ops.M[r][s];
-          ax = fma(t, mt[(mx + r + NF * line) * T], ax);
-          ay = fma(t, mt[(my + r + NF * line) * T], ay);
+          ax = fma(t, ml.x[r * T], ax);
+          ay = fma(t, ml.y[r * T], ay);
         }
         const int p = p0 + ps * s;
         const int is = p % N, js = p / N;
-        const double ji = mt[(G::JI + js + N * is) * T];
+        const double ji = ml.ji[(js + N * is) * T];
         double *o = a.nabla_f + v + 9 * 2 * ((size_t)p + (size_t)N2 * a.s2c[cell]);
         if (add) { o[0] += ax * ji; o[9] += ay * ji; }
         else { o[0] = ax * ji; o[9] = ay * ji; }

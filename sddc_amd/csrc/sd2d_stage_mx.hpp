@@ -113,11 +113,10 @@ void stage_kernel_mx(StageArgs a, OpsF ops, const float *__restrict__ metf) {
   }
   const int mem = ti >> 6, nvt = ti & TI_VALID;
   const bool valid = line < N && ci < nvt;
-  const float *mtf = metf + (size_t)tile * G::NM * T + ci;
-  const double *mt = a.met + (size_t)tile * G::NM * T + ci;
+  const MetLine<N, float> mlf(metf, a.mcomp, tile, ci, fam, line);
+  const MetLine<N, double> ml(a.met, a.mcomp, tile, ci, fam, line);
   const int p0 = fam ? line : N * line;
   const int ps = fam ? N : 1;
-  const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;
   const float *qsf = ldf + LD::QF;            // the staged tile (qo layout, FP32)
   // ---- neighbour traces at both end faces (memory or the staged tile) -------
   float qn0[9], qnN[9];
@@ -132,8 +131,8 @@ void stage_kernel_mx(StageArgs a, OpsF ops, const float *__restrict__ metf) {
   if (valid) {
 #pragma unroll
     for (int r = 0; r < NF; ++r) {
-      msx[r] = mtf[(mx + r + NF * line) * T];
-      msy[r] = mtf[(my + r + NF * line) * T];
+      msx[r] = mlf.x[r * T];
+      msy[r] = mlf.y[r * T];
     }
   }
   // the member's lagged maxima, step and free stream (needed from the face
@@ -227,7 +226,7 @@ void stage_kernel_mx(StageArgs a, OpsF ops, const float *__restrict__ metf) {
 #pragma unroll
     for (int s = 0; s < N; ++s) {   // 1/J at the thread's points
       const int is = fam ? line : s, js = fam ? s : line;
-      jis[s] = mt[(G::JI + js + N * is) * T];
+      jis[s] = ml.ji[(js + N * is) * T];
     }
     if (fam == 0) {
       load_vars<N, 0, VS>(qg, p0, ci, qn);

@@ -41,6 +41,7 @@ struct VisArgs {
   const double *qin;       // state (tile layout)
   const int *ftab;         // per-cell face table (tile layout)
   const double *met;       // metrics (tile layout)
+  int mcomp;               // as StageArgs
   const double *metw;      // other-family metrics at the line ends, for walls
   double *gq;              // gradient (go layout)
   double *dei;             // d(e)/dxi, d(e)/deta [tile][k*N2 + p][ci] (walls)
@@ -169,9 +170,8 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void vis_grad_kernel(VisArgs va, 
   }
   if (tid == 0) lds[LD::FLAG] = 0.0;
   const bool valid = line < N && ci < (ti & TI_VALID);
-  const double *mt = va.met + (size_t)tile * G::NM * T + ci;
+  const MetLine<N, double> ml(va.met, va.mcomp, tile, ci, fam, line);
   const int p0 = fam ? line : N * line, ps = fam ? N : 1;
-  const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;
   double qn0[9], qnN[9];
   int lci0 = -1, lciN = -1;
   double msx[NF], msy[NF], ji[N];
@@ -180,12 +180,12 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void vis_grad_kernel(VisArgs va, 
                                 lciN);
 #pragma unroll
     for (int r = 0; r < NF; ++r) {
-      msx[r] = mt[(mx + r + NF * line) * T];
-      msy[r] = mt[(my + r + NF * line) * T];
+      msx[r] = ml.x[r * T];
+      msy[r] = ml.y[r * T];
     }
 #pragma unroll
     for (int s = 0; s < N; ++s)
-      ji[s] = mt[(G::JI + (fam ? s : line) + N * (fam ? line : s)) * T];
+      ji[s] = ml.ji[((fam ? s : line) + N * (fam ? line : s)) * T];
   }
   __syncthreads();
   const bool wall0 = valid && ((info0 >> 3) & 7) == FT_WALL;
@@ -443,9 +443,8 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void vis_flux_kernel(VisArgs va, 
     if (tid + (NR - 1) * STAGE_THREADS < NV2) dst[tid + (NR - 1) * STAGE_THREADS] = st[NR - 1];
   }
   const bool valid = line < N && ci < (ti & TI_VALID);
-  const double *mt = va.met + (size_t)tile * G::NM * T + ci;
+  const MetLine<N, double> ml(va.met, va.mcomp, tile, ci, fam, line);
   const int p0 = fam ? line : N * line, ps = fam ? N : 1;
-  const int mx = fam ? G::S2X : G::S1X, my = fam ? G::S2Y : G::S1Y;
   const double *qt = va.qin + (size_t)tile * QT;
   double q[N][9];
   double msx[NF], msy[NF];
@@ -482,8 +481,8 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void vis_flux_kernel(VisArgs va, 
     for (int s = 0; s < N; ++s) load_vars<N, 0, 9>(qt, p0 + ps * s, ci, q[s]);
 #pragma unroll
     for (int r = 0; r < NF; ++r) {
-      msx[r] = mt[(mx + r + NF * line) * T];
-      msy[r] = mt[(my + r + NF * line) * T];
+      msx[r] = ml.x[r * T];
+      msy[r] = ml.y[r * T];
     }
   }
   __syncthreads();

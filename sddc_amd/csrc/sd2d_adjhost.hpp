@@ -39,7 +39,6 @@ struct AdjState {
   AdjCarry *carry = nullptr;  // what goes from one reversed evaluation to the next
   double *chb = nullptr;      // c_h cotangents, 5 per step
   int chb_n = 0;
-  unsigned long long *slots = nullptr;   // scratch maxima of sd2d_compresid_vjp
   double *dtile = nullptr;    // drag per tile
   double *Jd = nullptr;       // running sum of the drag
   double *wq = nullptr;       // face quadrature weights
@@ -59,7 +58,7 @@ static void adj_free(AdjState *A) {
   for (double *p : A->t) if (p) (void)hipFree(p);
   for (double *p : A->b) if (p) (void)hipFree(p);
   for (void *p : {(void *)A->divb, (void *)A->part, (void *)A->gm, (void *)A->tmax,
-                  (void *)A->tloc, (void *)A->carry, (void *)A->chb, (void *)A->slots,
+                  (void *)A->tloc, (void *)A->carry, (void *)A->chb,
                   (void *)A->dtile, (void *)A->Jd, (void *)A->wq, (void *)A->segm})
     if (p) (void)hipFree(p);
   for (double *p : A->ck) if (p) (void)hipFree(p);
@@ -139,7 +138,6 @@ static int adj_alloc(sd2d_ctx *c, AdjState *A, int nck, bool steps) {
   ADJGET(A->divb, 5 * np);
   ADJGET(A->part, (size_t)c->ntile * ADJ_NPART);
   ADJGET(A->carry, 1);
-  ADJGET(A->slots, 2 * NSLOT);
   ADJGET(A->gm, 12);
   if (!steps) return SD2D_OK;
   for (auto &p : A->t) ADJGET(p, n);
@@ -550,15 +548,13 @@ int sd2d_compresid_vjp(sd2d_ctx *c, const double *rbar, double *qbar, double *ch
   const size_t n = (size_t)c->ncell * 9 * c->N * c->N;
   HIPCHK(c, to_device(c, c->stagef, rbar, n));
   if ((r = f2t(c, c->stagef, A->b[1]))) return r;
-  // divB of the state as the stepping kernel forms it for the Powell source,
-  // with scratch maxima
+  // divB of the state as the stepping kernel forms it for the Powell source
   const double *q = c->q[c->cur];
   if ((r = save_max(c, A->gm, true))) return r;
   StageArgs s = base_args(c);
   s.qin = q;
   s.mread = nullptr;
   s.gmax = A->gm;
-  s.slots = A->slots;
   s.divb = A->divb;
   HIPCHK(c, launch_stage(c, s, M_DIVB));
   AdjArgs a = adj_args(c);

@@ -51,7 +51,7 @@ struct StageArgs {
   const int *ftab;          // per-cell face table (tile layout)
   // the running maxima before this evaluation, to raise and to clear (MSTRIDE
   // per member); or, mread null (an evaluation outside the sequence), the pair
-  // to form c_h from and NSLOT x 2 slots to raise
+  // to form c_h from and NSLOT x 2 slots to raise (none by M_DIVB)
   const unsigned long long *mread;
   unsigned long long *mwrite, *mclear;
   const double *gmax;
@@ -204,11 +204,16 @@ __device__ __forceinline__ void lagged_maxima(const StageArgs &a, int ti, int ti
   gu = g != MAX_NONE ? __longlong_as_double((long long)h) : mu;
 }
 
-// A tile's largest wave speed e and velocity bound u into the running maxima.
+// A line's largest wave speed e and velocity bound u into the running maxima.
 // A maximum is one address that all XCDs share, so an atomic is issued only
-// where the tile raises it, and after a reset (every tile raises it) only
-// where no other tile has raised it as far: 512 x 1024 cells, N = 5, one
-// atomic per tile and value on 256 / 64 addresses: 824 / 920 us; this: 801 us.
+// where a line raises it, and after a reset (every line raises it) only where
+// no other has raised it as far.  Nothing is reduced over the workgroup first:
+// in the usual case no lane enters, and a barrier, two wave reductions and
+// their wait at the end of every workgroup are gone.
+// 512 x 1024 cells, N = 5, stages without and with an RK register: one atomic
+// per tile and value on 256 addresses 720 / 824 us, on 64 addresses 831 / 920,
+// only where a tile raises a maximum 701 / 801; and without the reduction over
+// the workgroup (compact metrics on both sides) 703 / 776 -> 687 / 746.
 __device__ __forceinline__ void raise_maxima(const StageArgs &a, int mem, double e, double u,
                                              double me, double mu) {
   if (!a.mread) {
@@ -801,6 +806,9 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
     }
   }
 
+  // the line's speeds (getrusanov.f90:116-123,188-191; an idle lane's are 0) into
+  // the running maxima; the divB pass of a pullback evaluates for no one's
+  if (!DIVB) raise_maxima(a, mem, eig, um, me, mu);
   // all-variable gradient nablaQs for the compresid output: the xi-line
   // threads store their part, the eta-line threads add theirs after the
   // barrier (each point has one writer of each kind)
@@ -943,14 +951,16 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
     av_sensor_lines<N, T, AVF == 0, 2>(a, lds + LD::Q0 + qo<N>(0, 0, 0), lds + LD::XJ,
                                        lds + LD::XJ, rho_s, jz2_s, line, ci, cell, valid);
 
-  // ---- block reductions: running maxima (getrusanov.f90:116-123,188-191) and
-  //      norms (iterations.f90:37-46) ----------------------------------------------
-  {
+  // ---- block reductions of the modes that have any: norms
+  //      (iterations.f90:37-46), or where the tile's largest speeds are ---------------
+  if constexpr (NORMS || TRACE) {
     constexpr int NW = STAGE_THREADS / 64;
     const int w = tid >> 6, l = tid & 63;
     const double el = eig, ul = um;
-    eig = wave_max(eig);
-    um = wave_max(um);
+    if (TRACE) {
+      eig = wave_max(eig);
+      um = wave_max(um);
+    }
     if (NORMS) {
       nres = wave_sum(nres);
       ndiv = wave_sum(ndiv);
@@ -976,32 +986,23 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
     }
     __syncthreads();
     if (tid == 0) {
-      double e = lds[LD::RED], u = lds[LD::RED + NW];
-      double s1 = lds[LD::RED + 2 * NW], s2 = lds[LD::RED + 3 * NW];
+      static_assert(NW == 2, "two waves");
+      const double e = lds[LD::RED], u = lds[LD::RED + NW];
+      const double s1 = lds[LD::RED + 2 * NW], s2 = lds[LD::RED + 3 * NW];
+      const double e2 = lds[LD::RED + 1], u2 = lds[LD::RED + NW + 1];
+      const double c1 = lds[LD::RED + 2 * NW + 1], c2 = lds[LD::RED + 3 * NW + 1];
       if (TRACE) {
-        static_assert(!TRACE || (!NORMS && NW == 2), "the codes take the norms' slots");
-        const double e2 = lds[LD::RED + 1], u2 = lds[LD::RED + NW + 1];
-        const double c1 = lds[LD::RED + 2 * NW + 1], c2 = lds[LD::RED + 3 * NW + 1];
+        static_assert(!TRACE || !NORMS, "the codes take the norms' slots");
         a.tmax[2 * tile] = e2 > e ? e2 : e;
         a.tmax[2 * tile + 1] = u2 > u ? u2 : u;
         a.tloc[2 * tile] = (int)(e2 > e || (e2 == e && c1 < s1) ? c1 : s1);
         a.tloc[2 * tile + 1] = (int)(u2 > u || (u2 == u && c2 < s2) ? c2 : s2);
-      }
-#pragma unroll
-      for (int k = 1; k < NW; ++k) {
-        e = lds[LD::RED + k] > e ? lds[LD::RED + k] : e;
-        u = lds[LD::RED + NW + k] > u ? lds[LD::RED + NW + k] : u;
-        s1 += lds[LD::RED + 2 * NW + k];
-        s2 += lds[LD::RED + 3 * NW + k];
-      }
-      raise_maxima(a, mem, e, u, me, mu);
-      if (NORMS) {
-        a.normbuf[2 * tile] = s1;
-        a.normbuf[2 * tile + 1] = s2;
+      } else {
+        a.normbuf[2 * tile] = s1 + c1;
+        a.normbuf[2 * tile + 1] = s2 + c2;
       }
     }
   }
-
 }
 
 }  // namespace sd2d

@@ -273,6 +273,9 @@ void stage_kernel_mx(StageArgs a, OpsF ops, const float *__restrict__ metf) {
     }
   }
 
+  // the line's speeds into the running maxima (an idle lane's are 0)
+  raise_maxima(a, mem, double(eig), double(um), me, mu);
+
   // ---- solution points, in FP64: point (is, js) = (s, line) of a xi-line,
   //      (line, s) of an eta-line; variables V0..V1-1 of it ----------------------
   double rho_s[N], jz2_s[N];
@@ -355,41 +358,21 @@ void stage_kernel_mx(StageArgs a, OpsF ops, const float *__restrict__ metf) {
     else points(std::integral_constant<int, VS>{}, std::integral_constant<int, 9>{});
   }
 
-  // ---- block reductions -----------------------------------------------------------
-  {
+  // ---- norms (iterations.f90:37-46) --------------------------------------------------
+  if constexpr (NORMS) {
     constexpr int NW = STAGE_THREADS / 64;
+    static_assert(NW == 2, "two waves");
     const int w = tid >> 6, l = tid & 63;
-    double e = wave_max(double(eig)), u = wave_max(double(um));
-    if (NORMS) {
-      nres = wave_sum(nres);
-      ndiv = wave_sum(ndiv);
-    }
+    nres = wave_sum(nres);
+    ndiv = wave_sum(ndiv);
     if (l == 0) {
-      lds[LD::RED + w] = e;
-      lds[LD::RED + NW + w] = u;
-      if (NORMS) {
-        lds[LD::RED + 2 * NW + w] = nres;
-        lds[LD::RED + 3 * NW + w] = ndiv;
-      }
+      lds[LD::RED + w] = nres;
+      lds[LD::RED + NW + w] = ndiv;
     }
     __syncthreads();
     if (tid == 0) {
-      double em = lds[LD::RED], ummax = lds[LD::RED + NW];
-      double s1 = NORMS ? lds[LD::RED + 2 * NW] : 0.0, s2 = NORMS ? lds[LD::RED + 3 * NW] : 0.0;
-#pragma unroll
-      for (int k = 1; k < NW; ++k) {
-        em = lds[LD::RED + k] > em ? lds[LD::RED + k] : em;
-        ummax = lds[LD::RED + NW + k] > ummax ? lds[LD::RED + NW + k] : ummax;
-        if (NORMS) {
-          s1 += lds[LD::RED + 2 * NW + k];
-          s2 += lds[LD::RED + 3 * NW + k];
-        }
-      }
-      raise_maxima(a, mem, em, ummax, me, mu);
-      if (NORMS) {
-        a.normbuf[2 * tile] = s1;
-        a.normbuf[2 * tile + 1] = s2;
-      }
+      a.normbuf[2 * tile] = lds[LD::RED] + lds[LD::RED + 1];
+      a.normbuf[2 * tile + 1] = lds[LD::RED + NW] + lds[LD::RED + NW + 1];
     }
   }
 

@@ -407,7 +407,7 @@ static hipError_t launch_vis_n(sd2d_ctx *c, const double *qin) {
   hipError_t r = hipGetLastError();
   if (r != hipSuccess) return r;
   va.rev = 1;   // start on the tiles the gradient kernel wrote last
-  hipLaunchKernelGGL(vis_flux_kernel<N>, dim3(c->ntile), dim3(STAGE_THREADS), lf, c->stream,
+  hipLaunchKernelGGL(vis_flux_kernel<N>, dim3(c->ntile), dim3(VIS_FLUX_THREADS), lf, c->stream,
                      va, c->ops, c->ph);
   return hipGetLastError();
 }

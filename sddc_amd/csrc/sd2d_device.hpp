@@ -120,6 +120,18 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// A value every lane of a wavefront holds alike, as the compiler cannot see by
+// itself (the wave's number): branches on it are scalar and what it selects
+// stays in scalar registers.  (The CPU emulation of the kernels has no lanes to
+// read it from.)
+__device__ __forceinline__ int wave_uniform(int x) {
+#ifdef __HIP__
+  return __builtin_amdgcn_readfirstlane(x);
+#else
+  return x;
+#endif
+}
+
 // Interpolation / differentiation operators (initsetup.f90:262-319),
 // passed by value in the kernarg.
 struct Ops {

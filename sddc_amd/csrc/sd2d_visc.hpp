@@ -83,13 +83,10 @@ template <int N> struct VisGradLds {
   static_assert(2 * N * NF <= 4 * N2, "the internal energy fits the exchange areas");
 };
 
-// LDS of vis_flux_kernel (in doubles): the tile's gradient (go layout); after
-// the fluxes, the derivatives the families hand each other: variables 1-3 for
-// the xi-lines, 4-7 for the eta-lines, [k][p][ci].
+// LDS of vis_flux_kernel (in doubles): the tile's gradient (go layout), then
+// the accumulators handed over, 2 x 7 values per point.
 template <int N> struct VisFluxLds {
-  static constexpr int T = Geo<N>::CPW, N2 = N * N;
-  static constexpr int XA = 0, XB = 3 * N2 * T;
-  static constexpr int TOTAL = 18 * N2 * T;
+  static constexpr int TOTAL = 18 * N * N * Geo<N>::CPW;
 };
 
 // The averaged state at end rfp of a line (BR1: interfaceflux_all.f90:79-91,
@@ -134,9 +131,9 @@ __device__ __forceinline__ double enei_of(const double *q) {
 // after the barrier adds the two, scales by 1/J and stores both components
 // as one 16-byte word.  The xi-lines finish variables 0-3 and d(psi)/dx, the
 // eta-lines 4-7 and d(psi)/dy, so both waves store half.
-// Bound by the L2 and the loads in flight (2 waves per SIMD: 184-216 VGPRs,
-// 31-41 KB of LDS).  128 x 256 cells, N = 5: 69 us, 3.1 TB/s of its compulsory
-// 262 bytes a point; N = 4: 35 us.  The form before it, which read every
+// Bound by the L2 and the loads in flight (2 waves per SIMD: 182-210 VGPRs,
+// 31-41 KB of LDS).  128 x 256 cells, N = 5: 63 us, 3.0 TB/s of its compulsory
+// 232 bytes a point; N = 4: 33 us.  The form before it, which read every
 // flux point's line and neighbour from memory (12 reads of the tile, one
 // 8-byte word at a time) and let one family store everything: 259 and 115 us.
 template <int N>
@@ -148,7 +145,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void vis_grad_kernel(VisArgs va, 
   extern __shared__ double lds[];
   const int tid = threadIdx.x;
   const int tile = tile_of_block(blockIdx.x, va.ntile, va.rev);
-  const int fam = tid >> 6, line = (tid & 63) / T, ci = (tid & 63) % T;
+  const int fam = wave_uniform(tid >> 6), line = (tid & 63) / T, ci = (tid & 63) % T;
   int nb0, nbN, info0, infoN;
   face_words<N>(va, tile, ci, fam, line, 0, nb0, info0);
   face_words<N>(va, tile, ci, fam, line, N, nbN, infoN);
@@ -397,206 +394,189 @@ __device__ __forceinline__ void grad_trace(const double *vals, const double *Lr,
 
 // Viscous flux divergence dFv + dGv at the solution points (variables 1-7).
 //
-// One thread per grid line; the tile's gradient (18 values a point) is staged
-// in LDS by both waves, the line's own state stays in registers.  The
-// neighbours' state and gradient traces of the two end faces are gathered
-// before the barrier where the neighbour lies in another tile (from the
-// staged gradient after it otherwise) and averaged with the own ones (BR1,
-// interfaceflux_all.f90:140-190; boundary ghosts: a copy, or the adiabatic
-// wall, bcflux.f90:380-666).  Each flux point's seven fluxes are folded into
-// the line's derivative accumulators, and the families exchange half of them
-// through the LDS the gradient occupied: the xi-lines finish variables 1-3,
-// the eta-lines 4-7.
-// 256 VGPRs and 40-152 AGPRs (the line's 9 N state values, 7 N accumulators,
-// the gathered traces), so one wave per SIMD; bound by the latency of its
-// loads, which nothing overlaps, then by FP64 issue.  128 x 256 cells, N = 5:
-// 136 us (406 us when every flux point read its lines from memory); N = 4:
-// 65 us (216).  Held to two waves per SIMD the kernel spills (250-370
-// bytes a lane) and takes 207 us at N = 5, with the state re-read from memory
-// per point 152 us; both lose at N = 3 and 4 as well.
+// Four waves per tile, two threads per grid line: wave 2*fam + half, where half
+// 0 takes the flux points 0 .. N/2 of the line, half 1 the others from N down.
+// The tile's gradient (18 values a point) is staged in LDS.  Before the
+// barrier a thread forms the state traces of its flux points and, where its
+// end face's neighbour lies in another tile, gathers that neighbour's gradient
+// trace (from the staged gradient after it otherwise); the end's traces are
+// averaged (BR1, interfaceflux_all.f90:140-190; boundary ghosts: a copy, or
+// the adiabatic wall, bcflux.f90:380-666).  Each flux point's seven fluxes are
+// folded into the thread's derivative accumulators; half 1 hands its
+// accumulators to half 0 through the LDS the gradient occupied, then the
+// families exchange: the xi-lines finish variables 1-3, the eta-lines 4-7.
+// Two waves per SIMD (193-254 VGPRs, 26-43 KB of LDS); bound by the vector
+// memory and LDS pipes together (95 16-byte loads and 180 LDS reads a thread
+// at N = 5), then by FP64 issue.  128 x 256 cells, N = 5: 111 us; with one
+// thread per line (both ends and all interior points: 376 registers, one wave
+// per SIMD) 133 us; when every flux point read its lines from memory, 406 us.
+// N = 4 (151 x 90): 34 / 35 / 108 us, N = 3 (128 x 256): 46 / 44 / 153 us.
+// All flux points' gradient traces in one pass over LDS spill (660 bytes a
+// lane at N = 5).
+constexpr int VIS_FLUX_THREADS = 256;
 template <int N>
-__global__ __launch_bounds__(STAGE_THREADS, 1) void vis_flux_kernel(VisArgs va, Ops ops, Phys ph) {
+__global__ __launch_bounds__(VIS_FLUX_THREADS, 2) void vis_flux_kernel(VisArgs va, Ops ops,
+                                                                       Phys ph) {
   using G = Geo<N>;
-  using LD = VisFluxLds<N>;
-  constexpr int T = G::CPW, N2 = G::N2, NF = N + 1, QT = G::QT;
-  static_assert(N * T <= 64 && STAGE_THREADS == 128, "one wavefront per line family");
+  constexpr int T = G::CPW, N2 = G::N2, QT = G::QT;
+  static_assert(N * T <= 64, "one wavefront per line family and half");
   extern __shared__ double lds[];
   const int tid = threadIdx.x;
   const int tile = tile_of_block(blockIdx.x, va.ntile, va.rev);
-  const int fam = tid >> 6, line = (tid & 63) / T, ci = (tid & 63) % T;
-  int nb0, nbN, info0, infoN;
-  face_words<N>(va, tile, ci, fam, line, 0, nb0, info0);
-  face_words<N>(va, tile, ci, fam, line, N, nbN, infoN);
+  // (uniform, so that each half runs its own code with a barrier of its own)
+  const int wv = wave_uniform(tid >> 6), fam = wv >> 1, half = wv & 1;
+  const int line = (tid & 63) / T, ci = (tid & 63) % T;
+  int nb, info;
+  face_words<N>(va, tile, ci, fam, line, half ? N : 0, nb, info);
   const int ti = va.tinfo[tile];
   {
-    constexpr int NV2 = 9 * N2 * T, NR = (NV2 + STAGE_THREADS - 1) / STAGE_THREADS;
+    constexpr int NV2 = 9 * N2 * T, NR = (NV2 + VIS_FLUX_THREADS - 1) / VIS_FLUX_THREADS;
     const double2 *src = reinterpret_cast<const double2 *>(va.gq + (size_t)tile * 2 * QT);
     double2 *dst = reinterpret_cast<double2 *>(lds);
     double2 st[NR];
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
-      const int i = tid + k * STAGE_THREADS;
+      const int i = tid + k * VIS_FLUX_THREADS;
       st[k] = src[(k < NR - 1 || i < NV2) ? i : 0];
     }
 #pragma unroll
-    for (int k = 0; k < NR - 1; ++k) dst[tid + k * STAGE_THREADS] = st[k];
-    if (tid + (NR - 1) * STAGE_THREADS < NV2) dst[tid + (NR - 1) * STAGE_THREADS] = st[NR - 1];
+    for (int k = 0; k < NR - 1; ++k) dst[tid + k * VIS_FLUX_THREADS] = st[k];
+    if (tid + (NR - 1) * VIS_FLUX_THREADS < NV2) dst[tid + (NR - 1) * VIS_FLUX_THREADS] = st[NR - 1];
   }
   const bool valid = line < N && ci < (ti & TI_VALID);
   const MetLine<N, double> ml(va.met, va.mcomp, tile, ci, fam, line);
   const int p0 = fam ? line : N * line, ps = fam ? N : 1;
   const double *qt = va.qin + (size_t)tile * QT;
-  double q[N][9];
-  double msx[NF], msy[NF];
-  const bool i0 = ((info0 >> 3) & 7) == FT_INTERIOR, iN = ((infoN >> 3) & 7) == FT_INTERIOR;
-  const bool far0 = i0 && nb0 / QT != tile, farN = iN && nbN / QT != tile;
-  // the neighbour's gradient line through the shared point of an end face
-  auto grad_line = [&](int rfp, int info, int &np0, int &nst, double *Lr) {
+  const bool inter = ((info >> 3) & 7) == FT_INTERIOR, far = inter && nb / QT != tile;
+  // the neighbour's line through the end face's shared point
+  int np0 = 0, nst = 0, nci = 0;
+  bool endN;
+  {
     int k, nfp;
-    end_face<N>(fam, line, rfp, k, nfp);
-    bool endN;
+    end_face<N>(fam, line, half ? N : 0, k, nfp);
     neighbour_line<N>(info & 3, nfp, np0, nst, endN);
-#pragma unroll
-    for (int s = 0; s < N; ++s) Lr[s] = endN ? ops.L[N][s] : ops.L[0][s];
-  };
-  // the traces of the line's first end whose neighbour lies in another tile,
-  // gathered now; a second such end waits until its flux is formed
-  double q1[9], g1[18];
-  auto far_traces = [&](int rfp, int nb, int info, double *qn, double *gn) {
-    const int nt = nb / QT, nci = nb - nt * QT;
-    int np0, nst;
-    double Lr[N];
-    grad_line(rfp, info, np0, nst, Lr);
-    line_vals<N, double>(va.qin + (size_t)nt * QT, np0, nst, nci, [&](int v, const double *vals) {
-      qn[v] = line_trace<N, double>(vals, Lr);
-    });
-    grad_vals<N>(va.gq + (size_t)nt * 2 * QT, np0, nst, nci, [&](int v, const double *vals) {
-      grad_trace<N>(vals, Lr, gn + 2 * v);
-    });
-  };
-  if (valid) {
-    if (far0 || farN)
-      far_traces(far0 ? 0 : N, far0 ? nb0 : nbN, far0 ? info0 : infoN, q1, g1);
-#pragma unroll
-    for (int s = 0; s < N; ++s) load_vars<N, 0, 9>(qt, p0 + ps * s, ci, q[s]);
-#pragma unroll
-    for (int r = 0; r < NF; ++r) {
-      msx[r] = ml.x[r * T];
-      msy[r] = ml.y[r * T];
-    }
   }
-  __syncthreads();
+  auto row = [&](int s) { return endN ? ops.L[N][s] : ops.L[0][s]; };
   double D[N][7];
-  if (valid) {
-    auto state_trace = [&](const double *Lr, double *t) {
-#pragma unroll
-      for (int v = 0; v < 9; ++v) {
-        double a = 0.0;
-#pragma unroll
-        for (int s = 0; s < N; ++s) a = fma(q[s][v], Lr[s], a);
-        t[v] = a;
-      }
-    };
-    // The two end faces, the one whose traces are at hand first: end N where
-    // only that one gathered, so the order is a value of the lane and the
-    // wave runs two passes, not three.
-    auto end_flux = [&](bool atN, bool gathered, double *F) {
-      const int rfp = atN ? N : 0, nb = atN ? nbN : nb0, info = atN ? infoN : info0;
-      const bool inter = atN ? iN : i0, far = atN ? farN : far0;
-      double Lo[N];
-#pragma unroll
-      for (int s = 0; s < N; ++s) Lo[s] = atN ? ops.L[N][s] : ops.L[0][s];
-      const double sx = atN ? msx[N] : msx[0], sy = atN ? msy[N] : msy[0];
-      if (inter && !far) {   // an in-tile neighbour: its gradient is staged
-        int np0, nst;
+  // a half's flux points: the end face (row RE) and NI interior points from R1
+  // in steps of DR
+  auto fluxes = [&](auto hc) __attribute__((always_inline)) {
+    constexpr int H = decltype(hc)::value;
+    constexpr int RE = H ? N : 0, R1 = H ? N - 1 : 1, DR = H ? -1 : 1;
+    constexpr int NI = H ? N - 1 - N / 2 : N / 2;
+    double Qv[9], t[NI][9], g1[18], sx[NI + 1], sy[NI + 1];
+    if (valid) {
+      double qn[9];
+      if (inter) {
+        const int nt = nb / QT;
+        nci = nb - nt * QT;
         double Lr[N];
-        grad_line(rfp, info, np0, nst, Lr);
-        line_vals<N, double>(qt, np0, nst, nb - tile * QT, [&](int v, const double *vals) {
-          q1[v] = line_trace<N, double>(vals, Lr);
+#pragma unroll
+        for (int s = 0; s < N; ++s) Lr[s] = row(s);
+        if (far)
+          grad_vals<N>(va.gq + (size_t)nt * 2 * QT, np0, nst, nci, [&](int v, const double *x) {
+            grad_trace<N>(x, Lr, g1 + 2 * v);
+          });
+        line_vals<N, double>(va.qin + (size_t)nt * QT, np0, nst, nci, [&](int v, const double *x) {
+          qn[v] = line_trace<N, double>(x, Lr);
         });
-        grad_vals<N>(lds, np0, nst, nb - tile * QT, [&](int v, const double *vals) {
-          grad_trace<N>(vals, Lr, g1 + 2 * v);
-        });
-      } else if (far && !gathered) {
-        far_traces(rfp, nb, info, q1, g1);
       }
-      double t[9], Qv[9], g[18];
-      state_trace(Lo, t);
-      vis_end_state(info, ph, t, q1, sx, sy, Qv);
-      grad_vals<N>(lds, p0, ps, ci, [&](int v, const double *vals) {
-        grad_trace<N>(vals, Lo, g + 2 * v);
+      sx[NI] = ml.x[RE * T];
+      sy[NI] = ml.y[RE * T];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        sx[i] = ml.x[(R1 + DR * i) * T];
+        sy[i] = ml.y[(R1 + DR * i) * T];
+      }
+      double te[9];
+      line_vals<N, double>(qt, p0, ps, ci, [&](int v, const double *x) {
+        te[v] = line_trace<N, double>(x, ops.L[RE]);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) t[i][v] = line_trace<N, double>(x, ops.L[R1 + DR * i]);
+      });
+      vis_end_state(info, ph, te, qn, sx[NI], sy[NI], Qv);
+    }
+    __syncthreads();
+    if (!valid) return;
+    {
+      double g[18], F[7];
+      grad_vals<N>(lds, p0, ps, ci, [&](int v, const double *x) {
+        grad_trace<N>(x, ops.L[RE], g + 2 * v);
       });
       if (inter) {
+        if (!far) {   // an in-tile neighbour: its gradient is staged
+          double Lr[N];
+#pragma unroll
+          for (int s = 0; s < N; ++s) Lr[s] = row(s);
+          grad_vals<N>(lds, np0, nst, nci, [&](int v, const double *x) {
+            grad_trace<N>(x, Lr, g1 + 2 * v);
+          });
+        }
 #pragma unroll
         for (int c = 0; c < 18; ++c) g[c] = 0.5 * g[c] + 0.5 * g1[c];
       } else if (((info >> 3) & 7) == FT_WALL) {
         // d(e)/deta along a xi-line, d(e)/dxi along an eta-line
         const double *de = va.dei + ((size_t)tile * 2 + (1 - fam)) * N2 * T + ci;
-        double dface = 0.0;
+        double dface = 0.0, to[9];
 #pragma unroll
-        for (int s = 0; s < N; ++s) dface = fma(de[(size_t)(p0 + ps * s) * T], Lo[s], dface);
+        for (int s = 0; s < N; ++s) dface = fma(de[(size_t)(p0 + ps * s) * T], ops.L[RE][s], dface);
+        line_vals<N, double>(qt, p0, ps, ci, [&](int v, const double *x) {
+          to[v] = line_trace<N, double>(x, ops.L[RE]);
+        });
         const double *mw = va.metw + (size_t)tile * VisGeo<N>::NW * T + ci;
         double gr4[2];
-        wall_grad_ghost(t, g, dface, mw[VisGeo<N>::slot(fam, atN, 0, line) * T],
-                        mw[VisGeo<N>::slot(fam, atN, 1, line) * T], gr4);
+        wall_grad_ghost(to, g, dface, mw[VisGeo<N>::slot(fam, H, 0, line) * T],
+                        mw[VisGeo<N>::slot(fam, H, 1, line) * T], gr4);
         g[8] = 0.5 * g[8] + 0.5 * gr4[0];
         g[9] = 0.5 * g[9] + 0.5 * gr4[1];
       }
-      vflux_n(Qv, g, va.mu, va.eta0, sx, sy, F);
-    };
-    {
-      double FA[7], FB[7];
-      const bool nfirst = farN && !far0;
-      end_flux(nfirst, true, FA);
-      __builtin_amdgcn_sched_barrier(0);
-      end_flux(!nfirst, false, FB);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int s = 0; s < N; ++s) {
-        const double MA = nfirst ? ops.M[N][s] : ops.M[0][s], MB = nfirst ? ops.M[0][s] : ops.M[N][s];
-#pragma unroll
-        for (int k = 0; k < 7; ++k) D[s][k] = fma(FB[k], MB, FA[k] * MA);
-      }
-    }
-    // interior flux points two at a time (compflux.f90:198-258)
-    auto point = [&](int r, const double *g) {
-      double t[9], F[7];
-      state_trace(ops.L[r], t);
-      vflux_n(t, g, va.mu, va.eta0, msx[r], msy[r], F);
+      vflux_n(Qv, g, va.mu, va.eta0, sx[NI], sy[NI], F);
 #pragma unroll
       for (int s = 0; s < N; ++s)
 #pragma unroll
-        for (int k = 0; k < 7; ++k) D[s][k] = fma(F[k], ops.M[r][s], D[s][k]);
-    };
+        for (int c = 0; c < 7; ++c) D[s][c] = F[c] * ops.M[RE][s];
+    }
+    // interior flux points (compflux.f90:198-258)
 #pragma unroll
-    for (int r = 1; r < N; r += 2) {
-      const bool two = r + 1 < N;
-      double ga[18], gb[18];
-      grad_vals<N>(lds, p0, ps, ci, [&](int v, const double *vals) {
-        grad_trace<N>(vals, ops.L[r], ga + 2 * v);
-        if (two) grad_trace<N>(vals, ops.L[r + 1], gb + 2 * v);
-      });
-      point(r, ga);
-      if (two) point(r + 1, gb);
+    for (int i = 0; i < NI; ++i) {
       __builtin_amdgcn_sched_barrier(0);
+      double g[18], F[7];
+      grad_vals<N>(lds, p0, ps, ci, [&](int v, const double *x) {
+        grad_trace<N>(x, ops.L[R1 + DR * i], g + 2 * v);
+      });
+      vflux_n(t[i], g, va.mu, va.eta0, sx[i], sy[i], F);
+#pragma unroll
+      for (int s = 0; s < N; ++s)
+#pragma unroll
+        for (int c = 0; c < 7; ++c) D[s][c] = fma(F[c], ops.M[R1 + DR * i][s], D[s][c]);
     }
-  }
+  };
+  if (half) fluxes(std::integral_constant<int, 1>{});
+  else fluxes(std::integral_constant<int, 0>{});
+  // half 1's accumulators to half 0, [fam][c][p][ci]
+  double *own = lds + fam * 7 * N2 * T, *other = lds + (1 - fam) * 7 * N2 * T;
+  auto at = [&](int c, int s) { return (c * N2 + p0 + ps * s) * T + ci; };
   __syncthreads();   // every read of the staged gradient is done
-  if (valid) {
+  if (valid && half) {
 #pragma unroll
-    for (int s = 0; s < N; ++s) {
-      const int p = p0 + ps * s;
-      if (fam) {
+    for (int s = 0; s < N; ++s)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) lds[LD::XA + (k * N2 + p) * T + ci] = D[s][k];
-      } else {
-#pragma unroll
-        for (int k = 3; k < 7; ++k) lds[LD::XB + ((k - 3) * N2 + p) * T + ci] = D[s][k];
-      }
-    }
+      for (int c = 0; c < 7; ++c) own[at(c, s)] = D[s][c];
   }
   __syncthreads();
-  if (!valid) return;
+  // the sums of a line; what the other family finishes goes back to where
+  // this thread read it
+  if (valid && !half) {
+#pragma unroll
+    for (int s = 0; s < N; ++s)
+#pragma unroll
+      for (int c = 0; c < 7; ++c) {
+        D[s][c] += own[at(c, s)];
+        if ((c < 3) == (fam == 1)) own[at(c, s)] = D[s][c];
+      }
+  }
+  __syncthreads();
+  if (!valid || half) return;
   double *o = va.visres + (size_t)tile * QT;
 #pragma unroll
   for (int s = 0; s < N; ++s) {
@@ -604,12 +584,12 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void vis_flux_kernel(VisArgs va, 
     double w[4];
     if (fam) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) w[k] = D[s][3 + k] + lds[LD::XB + (k * N2 + p) * T + ci];
+      for (int c = 0; c < 4; ++c) w[c] = D[s][3 + c] + other[at(3 + c, s)];
       store_vars<N, 4, 8>(o, p, ci, w);
     } else {
       w[0] = 0.0;   // rho has no viscous flux
 #pragma unroll
-      for (int k = 0; k < 3; ++k) w[1 + k] = D[s][k] + lds[LD::XA + (k * N2 + p) * T + ci];
+      for (int c = 0; c < 3; ++c) w[1 + c] = D[s][c] + other[at(c, s)];
       store_vars<N, 0, 4>(o, p, ci, w);
     }
   }

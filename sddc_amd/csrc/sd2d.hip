@@ -23,6 +23,7 @@
 #include "sd2d_host.hpp"
 #include "sd2d_stage.hpp"
 #include "sd2d_stage_mx.hpp"
+#include "sd2d_stage_pt.hpp"
 #include "sd2d_visc.hpp"
 #include "sd2d_adj.hpp"
 #include "sd2d_rkseq.hpp"
@@ -330,10 +331,26 @@ static hipError_t launch_stage_mx_t(sd2d_ctx *c, const StageArgs &a) {
   return hipGetLastError();
 }
 
+constexpr int NCU = 256;   // compute units of an MI355X
+
+template <int N, int MODE>
+static hipError_t launch_stage_pt_t(sd2d_ctx *c, const StageArgs &a) {
+  constexpr size_t lds = stage_pt_lds_bytes<N, MODE>();
+  static_assert(lds <= 163840, "a workgroup's LDS above a CU's 160 KiB");
+  hipLaunchKernelGGL((stage_pt_kernel<N, MODE>), dim3(c->ntile), dim3(PT_THREADS<N>), lds,
+                     c->stream, a, c->ops);
+  return hipGetLastError();
+}
+
 template <int N, int MODE>
 static hipError_t launch_stage_t(sd2d_ctx *c, const StageArgs &a) {
   if constexpr ((MODE & (M_COMPAT | M_VIS | M_DIVB | M_TRACE)) == 0) {
     if (c->p.precision == SD2D_MIXED) return launch_stage_mx_t<N, MODE>(c, a);
+  }
+  if constexpr (pt_mode(MODE)) {
+    // one workgroup per CU or fewer: 9 % faster at 128 tiles, 10 at 256, 16 %
+    // slower at 342 (sd2d_stage_pt.hpp)
+    if (c->ntile <= NCU) return launch_stage_pt_t<N, MODE>(c, a);
   }
   constexpr size_t lds = stage_lds_bytes<N, MODE>();
   static_assert(lds <= 65536, "stage kernel LDS above 64 KiB");

@@ -221,6 +221,41 @@ __device__ __forceinline__ void iflux_n(const T *q, T c_h, T sx, T sy, T *Fn, T 
   if (ut > um) um = ut;
 }
 
+// In FP64 the two forms of the stage kernel (sd2d_stage.hpp, sd2d_stage_pt.hpp)
+// form the same bits: "fp contract(on)" fuses a multiply-add by the expression it
+// is written in, not by what the optimiser sees around it.  (The FP32 form keeps
+// the optimiser's choice; it has one kernel.)
+template <>
+__device__ __forceinline__ void iflux_n<double>(const double *q, double c_h, double sx, double sy,
+                                                double *Fn, double &um) {
+#pragma clang fp contract(on)
+  const double rho = q[0], rhou = q[1], rhov = q[2], rhow = q[3], rhoE = q[4];
+  const double Bx = q[5], By = q[6], Bz = q[7], psi = q[8];
+  const double ri = rcp(rho);
+  const double u = rhou * ri, v = rhov * ri, w = rhow * ri;
+  const double B2 = Bx * Bx + By * By + Bz * Bz;
+  // gas and magnetic pressure
+  const double pt =
+      (GAM - 1.0) * (rhoE - 0.5 * (rhou * u + rhov * v + rhow * w) - 0.5 * B2 - 0.5 * psi * psi) +
+      0.5 * B2;
+  const double ub = u * Bx + v * By + w * Bz;
+  const double ef = rhoE - 0.5 * psi * psi + pt;
+  const double un = u * sx + v * sy;
+  const double bn = Bx * sx + By * sy;
+  const double cp = c_h * psi, ez = v * Bx - u * By;
+  Fn[0] = rhou * sx + rhov * sy;
+  Fn[1] = rhou * un + pt * sx - Bx * bn;
+  Fn[2] = rhov * un + pt * sy - By * bn;
+  Fn[3] = rhow * un - Bz * bn;
+  Fn[4] = un * ef - ub * bn + cp * bn;
+  Fn[5] = cp * sx + ez * sy;
+  Fn[6] = cp * sy - ez * sx;
+  Fn[7] = Bz * un - w * bn;
+  Fn[8] = c_h * bn;
+  double ut = fmax(fmax(fabs(u), fabs(v)), fabs(w));
+  if (ut > um) um = ut;
+}
+
 // getrusanovflux (getrusanov.f90:1-125).  Returns the flux stored for the
 // left cell (Fnl) and the factor sign_l*sign_r that gives the right one.
 template <typename T>
@@ -287,6 +322,68 @@ __device__ __forceinline__ void rusanov(const T *QL, const T *QR, T nx, T ny,
   if (ev > eig) eig = ev;
   T ut = fmax(fmax(T(0.5) * fabs(ul + ur), T(0.5) * fabs(vl + vr)),
               T(0.5) * fabs(wl + wr));
+  if (ut > um) um = ut;
+}
+
+// In FP64 as iflux_n<double>; the two sides' fluxes are summed term by term (the
+// energy's apart, whose terms cancel on each side), which saves more multiply-adds
+// than the fusions across statements gave.  Error of the flux against extended
+// precision, rms over random states, relative to its largest component: 6.41e-17
+// (6.44e-17 with the sides formed apart).
+template <>
+__device__ __forceinline__ void rusanov<double>(const double *QL, const double *QR, double nx,
+                                                double ny, int sign_l, double c_h, double *Fn,
+                                                double &eig, double &um) {
+#pragma clang fp contract(on)
+  const double mag = sqrt(nx * nx + ny * ny);
+  const double im = sign_l * rcp(mag);
+  const double ux = nx * im, uy = ny * im;
+  const double ril = rcp(QL[0]), rir = rcp(QR[0]);
+  const double ul = ril * QL[1], vl = ril * QL[2], wl = ril * QL[3];
+  const double ur = rir * QR[1], vr = rir * QR[2], wr = rir * QR[3];
+  const double B2l = QL[5] * QL[5] + QL[6] * QL[6] + QL[7] * QL[7];
+  const double B2r = QR[5] * QR[5] + QR[6] * QR[6] + QR[7] * QR[7];
+  const double al = QL[4] - 0.5 * QL[0] * (ul * ul + vl * vl + wl * wl) - B2l * 0.5 -
+                    0.5 * QL[8] * QL[8];
+  const double pgl = (GAM - 1.0) * al;
+  const double pgr = (GAM - 1.0) * (QR[4] - 0.5 * QR[0] * (ur * ur + vr * vr + wr * wr) -
+                                    B2r * 0.5 - 0.5 * QR[8] * QR[8]);
+  const double ps = fma(GAM - 1.0, al, pgr);   // pgl + pgr
+  const double ptl = pgl + 0.5 * B2l, ptr = pgr + 0.5 * B2r;
+  const double Vnl = ul * ux + vl * uy, Vnr = ur * ux + vr * uy;
+  const double Bnl = QL[5] * ux + QL[6] * uy, Bnr = QR[5] * ux + QR[6] * uy;
+  // the sum of the two sides' normal fluxes
+  const double ez = vl * QL[5] - ul * QL[6] + vr * QR[5] - ur * QR[6];
+  const double cpl = c_h * QL[8], cpr = c_h * QR[8], cps = cpl + cpr;
+  double F[9];
+  F[0] = QL[0] * Vnl + QR[0] * Vnr;
+  F[1] = QL[1] * Vnl + ptl * ux - QL[5] * Bnl + QR[1] * Vnr + ptr * ux - QR[5] * Bnr;
+  F[2] = QL[2] * Vnl + ptl * uy - QL[6] * Bnl + QR[2] * Vnr + ptr * uy - QR[6] * Bnr;
+  F[3] = QL[3] * Vnl - QL[7] * Bnl + QR[3] * Vnr - QR[7] * Bnr;
+  F[4] = ((QL[4] - 0.5 * QL[8] * QL[8] + ptl) * Vnl -
+          Bnl * (ul * QL[5] + vl * QL[6] + wl * QL[7]) + cpl * Bnl) +
+         ((QR[4] - 0.5 * QR[8] * QR[8] + ptr) * Vnr -
+          Bnr * (ur * QR[5] + vr * QR[6] + wr * QR[7]) + cpr * Bnr);
+  F[5] = ez * uy + cps * ux;
+  F[6] = cps * uy - ez * ux;
+  F[7] = QL[7] * Vnl - wl * Bnl + QR[7] * Vnr - wr * Bnr;
+  F[8] = c_h * Bnl + c_h * Bnr;
+  // fast magneto-acoustic speed from averaged B and rho (:92-105)
+  const double bx = 0.5 * (QL[5] + QR[5]), by = 0.5 * (QL[6] + QR[6]), bz = 0.5 * (QL[7] + QR[7]);
+  const double irs = rcp(QL[0] + QR[0]);
+  const double ca = GAM * ps * irs;
+  const double bn = bx * ux + by * uy;
+  const double cn = 2 * bn * bn * irs;
+  const double cad = fma(2 * (bx * bx + by * by + bz * bz), irs, ca);
+  const double ct = sqrt(cad * cad - 4 * ca * cn);
+  const double cf = sqrt(0.5 * (cad + ct));
+  const double ev = 0.5 * fabs(Vnl + Vnr) + cf;
+  const double sc = 0.5 * mag * sign_l;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) Fn[k] = sc * (F[k] - ev * (QR[k] - QL[k]));
+  if (ev > eig) eig = ev;
+  const double ut = fmax(fmax(0.5 * fabs(fma(ril, QL[1], ur)), 0.5 * fabs(fma(ril, QL[2], vr))),
+                         0.5 * fabs(fma(ril, QL[3], wr)));
   if (ut > um) um = ut;
 }
 

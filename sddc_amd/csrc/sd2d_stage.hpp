@@ -540,6 +540,7 @@ __device__ __forceinline__ void face_flux(int info, int fam, int rfp, const Phys
 
 template <int N, int MODE>
 __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Ops ops) {
+#pragma clang fp contract(on)   // as iflux_n<double>
   using G = Geo<N>;
   using LD = StageLds<N, MODE>;
   constexpr int T = G::CPW, N2 = G::N2, NF = N + 1;

@@ -16,8 +16,9 @@
 // and split the solution points' work by variable: each xi-line thread
 // (fam 0) finishes variables 0-3, each eta-line thread (fam 1) variables
 // 4-8 at the N points of its line: residual, Powell and GLM sources, the RK
-// combination, norm partials.  The running maxima and norms are reduced
-// per workgroup; the AV smoothness sensor runs per cell on the last stage.
+// combination, norm partials.  The norms are reduced per workgroup, a line that
+// raises a running maximum does so by itself; the AV smoothness sensor runs per
+// cell on the last stage.  (Meshes of at most one tile per CU: sd2d_stage_pt.hpp.)
 //
 // Register budget: the neighbour traces of a line's two end faces are
 // gathered first, while nothing else is live; the tile's state is staged

@@ -21,8 +21,8 @@
 //                     the residual before the Jacobian scaling
 //                     (compresid.f90:43-46).
 //
-// Both use the stage kernel's thread layout: one 128-thread workgroup per
-// tile of cells, one thread per grid line, one family per wavefront.  The
+// Both use the stage kernel's thread layout: one workgroup per tile of cells, one
+// family per wavefront, one thread per grid line (vis_flux_kernel: two).  The
 // gradient (18 values per point) lives in HBM between the two kernels in
 // tiles of twice the size of a state.
 //

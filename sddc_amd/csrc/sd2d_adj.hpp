@@ -42,7 +42,7 @@ struct AdjArgs {
   const int *ftab;
   const int *tinfo;        // per tile: member << 6 | TI_FIRST | valid cells
   const Phys *phm;         // free stream
-  const double *gm;        // eigvmax_g, umax_g that the evaluation's c_h came from
+  const unsigned long long *gm;   // the maxima that the evaluation's c_h came from (a set)
   double *qbar, *abar;     // cotangents of Qin and Qaux (abar may be null)
   int qadd, aadd;          // add to what they hold (else overwrite it)
   double *part;            // per tile: c_hbar, pbar[6] (rinf pinf uinf vinf bx by)
@@ -451,7 +451,8 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void adj_stage_kernel(AdjArgs a, 
       msy[r] = ml.y[r * T];
     }
   }
-  const double ge = a.gm[0], gu = a.gm[1];
+  double ge, gu;
+  set_pair(a.gm, ge, gu);
   const double c_h = sqrt(ge * (ge - gu));   // as the forward forms it (compflux.f90:6)
   const Phys &ph = a.phm[0];
   double chb = 0.0, pb[6] = {0, 0, 0, 0, 0, 0};
@@ -824,11 +825,10 @@ __device__ __forceinline__ void adj_speed_apply(const AdjArgs &a, const Ops &ops
 }
 
 // What the reverse pass carries from one evaluation to the next, on the
-// device: the pending cotangents of the running maxima, the free stream's,
-// the c_h cotangent of a single evaluation, and whether a maximum's flux point
-// was not found.
+// device: the pending cotangents of the running maxima, the free stream's, and
+// whether a maximum's flux point was not found.
 struct AdjCarry {
-  double PE, PU, p[6], ch;
+  double PE, PU, p[6];
   int missed;
 };
 
@@ -845,8 +845,8 @@ template <int N>
 __global__ __launch_bounds__(ADJ_TAIL_THREADS) void adj_tail_kernel(AdjArgs a, Ops ops_arg,
                                                                     const double *tmax,
                                                                     const int *tloc,
-                                                                    const double *g1, AdjCarry *cy,
-                                                                    double *chbar) {
+                                                                    const unsigned long long *m1,
+                                                                    AdjCarry *cy, double *chbar) {
   constexpr int NT = ADJ_TAIL_THREADS;
   __shared__ double so[sizeof(Ops) / sizeof(double)];
   __shared__ double sum[ADJ_NPART][NT / 64], mv[2][NT / 64];
@@ -854,7 +854,9 @@ __global__ __launch_bounds__(ADJ_TAIL_THREADS) void adj_tail_kernel(AdjArgs a, O
   const Ops &ops = ops_to_lds<0>(so, ops_arg);
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
   const int none = 0x7fffffff;
-  const double E = a.gm[0], U = a.gm[1];
+  double E, U, g1[2];
+  set_pair(a.gm, E, U);
+  set_pair(m1, g1[0], g1[1]);
   const double PE = cy->PE, PU = cy->PU;
   const bool raised[2] = {g1[0] > E, g1[1] > U};
   double x[ADJ_NPART] = {0, 0, 0, 0, 0, 0, 0}, best[2] = {0.0, 0.0};
@@ -911,7 +913,7 @@ __global__ __launch_bounds__(ADJ_TAIL_THREADS) void adj_tail_kernel(AdjArgs a, O
       }
       cy->PE = pe;
       cy->PU = pu;
-      if (chbar) *chbar = s;
+      *chbar = s;
     }
   }
 }

@@ -33,7 +33,7 @@ struct AdjState {
   double *b[6] = {};          // cotangents of Q0..Q5
   double *divb = nullptr;     // divB per point of the five evaluations of a step
   double *part = nullptr;     // per tile partial sums
-  double *gm = nullptr;       // gmax before each of the 5 stages and after (device)
+  unsigned long long *gm = nullptr;   // the maxima read by each of the 5 stages (sets)
   double *tmax = nullptr;     // per evaluation and tile: largest speeds and where
   int *tloc = nullptr;
   AdjCarry *carry = nullptr;  // what goes from one reversed evaluation to the next
@@ -69,23 +69,18 @@ static void adj_free(AdjState *A) {
 static size_t state_len(const sd2d_ctx *c) { return (size_t)c->ntile * 9 * c->N * c->N * c->cpw; }
 
 // The running maxima of one run (a set) to and from four doubles on the device:
-// eigvmax, umax, eigvmax_g, umax_g; `only_g` the last two alone.
-__global__ void k_save_max(const unsigned long long *set, double *m, bool only_g) {
-  const bool apart = set[2] != MAX_NONE;
-  double *g = only_g ? m : m + 2;
-  if (!only_g) {
-    m[0] = __longlong_as_double((long long)set[0]);
-    m[1] = __longlong_as_double((long long)set[1]);
-  }
-  g[0] = __longlong_as_double((long long)set[apart ? 2 : 0]);
-  g[1] = __longlong_as_double((long long)set[apart ? 3 : 1]);
+// eigvmax, umax, eigvmax_g, umax_g.
+__global__ void k_save_max(const unsigned long long *set, double *m) {
+  m[0] = __longlong_as_double((long long)set[0]);
+  m[1] = __longlong_as_double((long long)set[1]);
+  set_pair(set, m[2], m[3]);
 }
 __global__ void k_load_max(const double *m, unsigned long long *set) {
   set[threadIdx.x] = as_bits(m[threadIdx.x]);
 }
 
-static int save_max(sd2d_ctx *c, double *m, bool only_g) {
-  hipLaunchKernelGGL(k_save_max, dim3(1), dim3(1), 0, c->stream, max_set(c, c->mset), m, only_g);
+static int save_max(sd2d_ctx *c, double *m) {
+  hipLaunchKernelGGL(k_save_max, dim3(1), dim3(1), 0, c->stream, max_set(c, c->mset), m);
   HIPCHK(c, hipGetLastError());
   return SD2D_OK;
 }
@@ -137,9 +132,9 @@ static int adj_alloc(sd2d_ctx *c, AdjState *A, int nck, bool steps) {
   for (int i = 0; i < (steps ? 6 : 2); ++i) ADJGET(A->b[i], n);
   ADJGET(A->divb, 5 * np);
   ADJGET(A->part, (size_t)c->ntile * ADJ_NPART);
-  ADJGET(A->carry, 1);
-  ADJGET(A->gm, 12);
   if (!steps) return SD2D_OK;
+  ADJGET(A->carry, 1);
+  ADJGET(A->gm, 5 * MSTRIDE);
   for (auto &p : A->t) ADJGET(p, n);
   ADJGET(A->tmax, 10 * (size_t)c->ntile);
   ADJGET(A->tloc, 10 * (size_t)c->ntile);
@@ -202,8 +197,8 @@ static const AdjStage kS5P3[5] = {
 
 // The five stages of one step from qs[0] (the forward's launches), its states
 // into qs[1..5]; with trace, what the reverse sweep needs of each evaluation
-// is recorded as well (divB, the maxima before every stage and after the last,
-// and where each tile's largest speeds are attained).
+// is recorded as well (divB, the maxima before it, and where each tile's largest
+// speeds are attained).
 static int adj_stages(sd2d_ctx *c, double *const *qs, bool trace) {
   AdjState *A = c->adj;
   const int av = (c->p.artiv == 1 && c->p.vismode == 1) ? M_AV : 0;
@@ -223,37 +218,38 @@ static int adj_stages(sd2d_ctx *c, double *const *qs, bool trace) {
     if (trace) {
       mode |= M_TRACE;
       a.divb = A->divb + s * np;
-      a.gmrec = A->gm + 2 * s;
+      a.gmrec = A->gm + MSTRIDE * s;
       a.tmax = A->tmax + 2 * (size_t)c->ntile * s;
       a.tloc = A->tloc + 2 * (size_t)c->ntile * s;
     }
     HIPCHK(c, launch_stage(c, a, mode));
     rotate_maxima(c);
   }
-  return trace ? save_max(c, A->gm + 10, true) : SD2D_OK;
+  return SD2D_OK;
 }
 
-// One evaluation backwards: adj_stage_kernel, then adj_tail_kernel with the
-// maxima g1 after the evaluation.
+// One evaluation backwards: adj_stage_kernel and, within a pass over steps (m1
+// set), adj_tail_kernel with the maxima m1 after the evaluation.
 template <int N>
 static hipError_t adj_launch_n(sd2d_ctx *c, const AdjArgs &a, const double *tmax, const int *tloc,
-                               const double *g1, double *chbar) {
+                               const unsigned long long *m1, double *chbar) {
   AdjState *A = c->adj;
   static_assert(adj_lds_bytes<N>() <= 65536, "adjoint kernel LDS above 64 KiB");
   hipLaunchKernelGGL(adj_stage_kernel<N>, dim3(c->ntile), dim3(STAGE_THREADS), adj_lds_bytes<N>(),
                      c->stream, a, c->ops);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || !m1) return e;
   hipLaunchKernelGGL(adj_tail_kernel<N>, dim3(1), dim3(ADJ_TAIL_THREADS), 0, c->stream, a, c->ops,
-                     tmax, tloc, g1, A->carry, chbar);
+                     tmax, tloc, m1, A->carry, chbar);
   return hipGetLastError();
 }
-static int adj_launch(sd2d_ctx *c, const AdjArgs &a, const double *tmax, const int *tloc,
-                      const double *g1, double *chbar) {
+static int adj_launch(sd2d_ctx *c, const AdjArgs &a, const double *tmax = nullptr,
+                      const int *tloc = nullptr, const unsigned long long *m1 = nullptr,
+                      double *chbar = nullptr) {
   switch (c->N) {
-    case 3: HIPCHK(c, adj_launch_n<3>(c, a, tmax, tloc, g1, chbar)); break;
-    case 4: HIPCHK(c, adj_launch_n<4>(c, a, tmax, tloc, g1, chbar)); break;
-    default: HIPCHK(c, adj_launch_n<5>(c, a, tmax, tloc, g1, chbar)); break;
+    case 3: HIPCHK(c, adj_launch_n<3>(c, a, tmax, tloc, m1, chbar)); break;
+    case 4: HIPCHK(c, adj_launch_n<4>(c, a, tmax, tloc, m1, chbar)); break;
+    default: HIPCHK(c, adj_launch_n<5>(c, a, tmax, tloc, m1, chbar)); break;
   }
   return SD2D_OK;
 }
@@ -268,7 +264,8 @@ static AdjArgs adj_args(sd2d_ctx *c) {
 
 // Reverse one RK_S5P3 step: A->b[5] holds the cotangent of the step's
 // output (Q5), on return A->b[0] that of its input (Q0).  qs[0..4] are the
-// recomputed stage inputs (adj_stages with trace).
+// recomputed stage inputs (adj_stages with trace; the maxima after the last
+// stage are still the context's).
 static int adj_step_vjp(sd2d_ctx *c, double *const *qs, double *chbar5) {
   AdjState *A = c->adj;
   double **B = A->b;
@@ -284,7 +281,7 @@ static int adj_step_vjp(sd2d_ctx *c, double *const *qs, double *chbar5) {
     a.cin = st.cin;
     a.ca = st.ca;
     a.divb = A->divb + s * np;
-    a.gm = A->gm + 2 * s;
+    a.gm = A->gm + MSTRIDE * s;
     a.qbar = B[st.in];
     a.qadd = have[st.in];
     have[st.in] = true;
@@ -293,8 +290,9 @@ static int adj_step_vjp(sd2d_ctx *c, double *const *qs, double *chbar5) {
       a.aadd = have[st.aux];
       have[st.aux] = true;
     }
+    const unsigned long long *m1 = s == 4 ? max_set(c, c->mset) : A->gm + MSTRIDE * (s + 1);
     const int r = adj_launch(c, a, A->tmax + 2 * (size_t)c->ntile * s,
-                             A->tloc + 2 * (size_t)c->ntile * s, A->gm + 2 * (s + 1), chbar5 + s);
+                             A->tloc + 2 * (size_t)c->ntile * s, m1, chbar5 + s);
     if (r) return r;
   }
   return SD2D_OK;
@@ -391,7 +389,7 @@ int sd2d_vjp(sd2d_ctx *c, const double *qbar_final, double jbar, double *qbar_in
     };
     double *qs[6];
     for (int i = 0; i < len; ++i) {
-      if ((r = save_max(c, A->segm + 4 * i, false))) return r;
+      if ((r = save_max(c, A->segm + 4 * i))) return r;
       if (i + 1 == len) break;   // the last step runs once, below
       step_states(i, qs);
       if ((r = adj_stages(c, qs, false))) return r;
@@ -546,34 +544,42 @@ int sd2d_compresid_vjp(sd2d_ctx *c, const double *rbar, double *qbar, double *ch
   int r = adj_alloc(c, A, 0, false);
   if (r) return r;
   const size_t n = (size_t)c->ncell * 9 * c->N * c->N;
+  const size_t np = (size_t)c->ntile * ADJ_NPART;
+  const std::unique_ptr<double[]> part(new (std::nothrow) double[np]);
+  if (!part) return fail(c, SD2D_ENOMEM, "host allocation failed");
   HIPCHK(c, to_device(c, c->stagef, rbar, n));
   if ((r = f2t(c, c->stagef, A->b[1]))) return r;
   // divB of the state as the stepping kernel forms it for the Powell source
   const double *q = c->q[c->cur];
-  if ((r = save_max(c, A->gm, true))) return r;
+  const unsigned long long *set = max_set(c, c->mset);
   StageArgs s = base_args(c);
   s.qin = q;
   s.mread = nullptr;
-  s.gmax = A->gm;
+  s.gmax = reinterpret_cast<const double *>(set);   // (divB does not depend on c_h)
   s.divb = A->divb;
   HIPCHK(c, launch_stage(c, s, M_DIVB));
   AdjArgs a = adj_args(c);
   a.q = q;
   a.rbar = A->b[1];
   a.divb = A->divb;
-  a.gm = A->gm;
+  a.gm = set;
   a.qbar = A->b[0];
-  HIPCHK(c, hipMemsetAsync(A->carry, 0, sizeof(AdjCarry), c->stream));
-  if ((r = adj_launch(c, a, nullptr, nullptr, A->gm, &A->carry->ch))) return r;   // raises nothing
+  if ((r = adj_launch(c, a))) return r;
   if (qbar) {
     if ((r = t2f(c, A->b[0], c->stagef))) return r;
     HIPCHK(c, to_host(c, qbar, c->stagef, n));
   }
-  AdjCarry cy{};
-  HIPCHK(c, hipMemcpyAsync(&cy, A->carry, sizeof(cy), hipMemcpyDeviceToHost, c->stream));
+  // The tiles' partial sums are added up here, 56 bytes a tile: a launch for the
+  // sum and two to prepare it cost more than they save (7 x 5 cells, N = 3: 118 us
+  // a pullback with them, 93 without; 97 x 163, N = 5: 2.05 ms either way).
+  HIPCHK(c, hipMemcpyAsync(part.get(), A->part, np * sizeof(double), hipMemcpyDeviceToHost,
+                           c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (chbar) *chbar = cy.ch;
-  if (pbar) for (int j = 0; j < 6; ++j) pbar[j] = cy.p[j];
+  double acc[ADJ_NPART] = {};
+  for (int t = 0; t < c->ntile; ++t)
+    for (int j = 0; j < ADJ_NPART; ++j) acc[j] += part[(size_t)t * ADJ_NPART + j];
+  if (chbar) *chbar = acc[0];
+  if (pbar) for (int j = 0; j < 6; ++j) pbar[j] = acc[1 + j];
   return SD2D_OK;
 }
 

@@ -69,10 +69,11 @@ struct StageArgs {
   double avf[NMAX * NMAX];
   const double *visres;     // viscous divergence dFv + dGv (tile layout), M_VIS
   double *divb;             // divB per solution point [tile][p][ci], M_DIVB and M_TRACE
-  // M_TRACE, for the adjoint: the maxima c_h was formed from (2), and per tile
+  // M_TRACE, for the adjoint: a copy of the maxima that were read, and per tile
   // the largest wave speed and velocity bound of this evaluation and the
   // smallest location code that attains each
-  double *gmrec, *tmax;     // tmax[2*tile]: eig, um
+  unsigned long long *gmrec;   // MSTRIDE
+  double *tmax;             // tmax[2*tile]: eig, um
   int *tloc;                // tloc[2*tile]
   const int *s2c;           // slot -> mesh cell, for the cell-indexed outputs
   // per tile (member << 6 | TI_FIRST | valid cells), member 0 for one run; an
@@ -172,6 +173,13 @@ __device__ __forceinline__ double wave_sum(double x) {
 
 __device__ __forceinline__ unsigned long long as_bits(double x) {
   return (unsigned long long)__double_as_longlong(x);
+}
+
+// The pair (eigvmax_g, umax_g) that the c_h formed from a set of maxima takes.
+__device__ __forceinline__ void set_pair(const unsigned long long *m, double &ge, double &gu) {
+  const bool apart = m[2] != MAX_NONE;
+  ge = __longlong_as_double((long long)m[apart ? 2 : 0]);
+  gu = __longlong_as_double((long long)m[apart ? 3 : 1]);
 }
 
 // eigvmax_g and umax_g (ge, gu) that this evaluation's c_h is formed from, and
@@ -631,8 +639,7 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void stage_kernel(StageArgs a, Op
   const double c_h = sqrt(ge * (ge - gu));   // lagged GLM speed, compflux.f90:6
   double eig = 0.0, um = 0.0, nres = 0.0, ndiv = 0.0;
   if (TRACE && blockIdx.x == 0 && tid == 0) {
-    a.gmrec[0] = ge;
-    a.gmrec[1] = gu;
+    for (int i = 0; i < MSTRIDE; ++i) a.gmrec[i] = a.mread[i];
   }
   // M_TRACE: the flux point of the line that attains eig and um (the smaller
   // number on a tie; the points come in the order 0, N, 1, ..., N-1)

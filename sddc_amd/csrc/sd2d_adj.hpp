@@ -833,10 +833,14 @@ struct AdjCarry {
 };
 
 // After adj_stage_kernel of one evaluation (one block): the tiles' partial
-// sums in a fixed order; where this evaluation raised a maximum (g0 -> g1) the
-// pending cotangent of the later evaluations' c_h goes to the flux point that
-// attained it (the smallest location code on a tie); and this evaluation's own
-// c_h = sqrt(E (E - U)) is passed on to the maxima before it.
+// sums in a fixed order; where a flux point of this evaluation exceeded a
+// running maximum the pending cotangent of the later evaluations' c_h goes to
+// the point that attained the new one (the smallest location code on a tie); and
+// this evaluation's own c_h = sqrt(E (E - U)) is passed on to the maxima before
+// it.  Where no point exceeded it, the pending cotangent goes on to the earlier
+// evaluations, unless the maximum is another value than the one this c_h was
+// formed from: then it is the caller's (sd2d_set_state with eigvmax apart from
+// eigvmax_g), a constant, and the cotangent ends here.
 // 128 x 256 cells, N = 4: 13 us; it replaces two searches over all flux points
 // (71 us each), a single-thread evaluation of the 18 directions (106 us) and
 // the copy of the partial sums to the host, which waited for every stage.
@@ -858,7 +862,8 @@ __global__ __launch_bounds__(ADJ_TAIL_THREADS) void adj_tail_kernel(AdjArgs a, O
   set_pair(a.gm, E, U);
   set_pair(m1, g1[0], g1[1]);
   const double PE = cy->PE, PU = cy->PU;
-  const bool raised[2] = {g1[0] > E, g1[1] > U};
+  const bool raised[2] = {g1[0] > __longlong_as_double((long long)a.gm[0]),
+                          g1[1] > __longlong_as_double((long long)a.gm[1])};
   double x[ADJ_NPART] = {0, 0, 0, 0, 0, 0, 0}, best[2] = {0.0, 0.0};
   int loc[2] = {none, none};
   for (int i = t; i < a.ntile; i += NT) {
@@ -906,7 +911,7 @@ __global__ __launch_bounds__(ADJ_TAIL_THREADS) void adj_tail_kernel(AdjArgs a, O
     if (t > 0) cy->p[t - 1] += s;
     else {
       const double ch = sqrt(E * (E - U));
-      double pe = raised[0] ? 0.0 : PE, pu = raised[1] ? 0.0 : PU;
+      double pe = raised[0] || g1[0] != E ? 0.0 : PE, pu = raised[1] || g1[1] != U ? 0.0 : PU;
       if (ch > 0.0) {
         pe += s * (2.0 * E - U) / (2.0 * ch);
         pu += s * (-E) / (2.0 * ch);

@@ -419,14 +419,14 @@ int sd2d_vjp(sd2d_ctx *c, const double *qbar_final, double jbar, double *qbar_in
                              c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (pbar) for (int j = 0; j < 6; ++j) pbar[j] = cy.p[j];
-  if (cy.missed)
-    return fail(c, SD2D_EINVAL, "adjoint: the flux point of a running maximum was not found");
   // the context returns to the final state of sd2d_fwd
   HIPCHK(c, hipMemcpyAsync(c->q[c->cur], A->ck[nck - 1], nb, hipMemcpyDeviceToDevice, c->stream));
   if ((r = adj_maxima_set(c, A->ckm[nck - 1]))) return r;
   c->ctime = A->fin_ctime;
   c->iter = A->fin_iter;
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (cy.missed)
+    return fail(c, SD2D_EINVAL, "adjoint: the flux point of a running maximum was not found");
   return SD2D_OK;
 }
 

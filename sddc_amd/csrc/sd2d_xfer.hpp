@@ -40,12 +40,15 @@ class HostRing {
     static HostRing r;
     return r;
   }
+  // A context comes and goes without waiting for another's copy: the lock is held
+  // only to take the ring and to give it back.  (A copy belongs to a context that
+  // lives, so the ring has a user as long as it is taken.)
   void add_user() {
-    std::lock_guard<std::mutex> lk(use_);
+    std::lock_guard<std::mutex> lk(m_);
     ++users_;
   }
   void drop_user() {
-    std::lock_guard<std::mutex> lk(use_);
+    std::lock_guard<std::mutex> lk(m_);
     if (--users_ > 0) return;
     if (buf_) (void)hipHostFree(buf_);
     buf_ = nullptr;
@@ -54,8 +57,15 @@ class HostRing {
   // Copy `bytes` from the device to the host (out) or back, in stream order;
   // done only when the caller has synchronised the stream.
   hipError_t copy(hipStream_t st, void *host, void *dev, size_t bytes, bool out) {
-    std::unique_lock<std::mutex> own(use_, std::defer_lock);
-    if (bytes < (out ? MIN_OUT : MIN_IN) || !own.try_lock() || !ready()) return plain(st, host, dev, bytes, out);
+    if (bytes < (out ? MIN_OUT : MIN_IN) || !take()) return plain(st, host, dev, bytes, out);
+    const hipError_t e = ring_copy(st, host, dev, bytes, out);
+    std::lock_guard<std::mutex> lk(m_);
+    busy_ = false;
+    return e;
+  }
+
+ private:
+  hipError_t ring_copy(hipStream_t st, void *host, void *dev, size_t bytes, bool out) {
     Job j;
     j.host = static_cast<char *>(host);
     j.ring = buf_;
@@ -93,7 +103,6 @@ class HostRing {
     return e;
   }
 
- private:
   struct Job {
     char *host, *ring;
     size_t bytes, chunk;
@@ -187,19 +196,25 @@ class HostRing {
     return out ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st)
                : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
   }
-  bool ready() {
-    if (buf_) return true;
-    void *p = nullptr;
-    if (hipHostMalloc(&p, NSLOT_ * SLOT, hipHostMallocPortable) != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
+  // The ring for one copy, allocated by the first; false where another copy has it
+  // or there is no memory for it.
+  bool take() {
+    std::lock_guard<std::mutex> lk(m_);
+    if (busy_) return false;
+    if (!buf_) {
+      void *p = nullptr;
+      if (hipHostMalloc(&p, NSLOT_ * SLOT, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
+      buf_ = static_cast<char *>(p);
     }
-    buf_ = static_cast<char *>(p);
-    return true;
+    return busy_ = true;
   }
 
-  std::mutex use_;
+  std::mutex m_;          // users_, buf_, busy_
   int users_ = 0;
+  bool busy_ = false;     // a copy has the ring
   char *buf_ = nullptr;
 };
 

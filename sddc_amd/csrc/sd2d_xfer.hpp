@@ -57,7 +57,7 @@ class HostRing {
   // Copy `bytes` from the device to the host (out) or back, in stream order;
   // done only when the caller has synchronised the stream.
   hipError_t copy(hipStream_t st, void *host, void *dev, size_t bytes, bool out) {
-    if (bytes < (out ? MIN_OUT : MIN_IN) || !take()) return plain(st, host, dev, bytes, out);
+    if (!pays(host, bytes, out) || !take()) return plain(st, host, dev, bytes, out);
     const hipError_t e = ring_copy(st, host, dev, bytes, out);
     std::lock_guard<std::mutex> lk(m_);
     busy_ = false;
@@ -196,6 +196,18 @@ class HostRing {
     return out ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st)
                : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
   }
+  // Whether the ring moves these bytes faster than the runtime's copy.  The copy
+  // engine reaches registered memory by itself: into pinned memory 472 MB take
+  // 8.9 ms, through the ring 12.2 ms (8.1 MB: 0.20 and 0.38 ms).
+  static bool pays(const void *host, size_t bytes, bool out) {
+    if (bytes < (out ? MIN_OUT : MIN_IN)) return false;
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, host) == hipSuccess)
+      return at.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();   // (some runtimes refuse pageable memory)
+    return true;
+  }
+
   // The ring for one copy, allocated by the first; false where another copy has it
   // or there is no memory for it.
   bool take() {

@@ -2,7 +2,7 @@
 // the CPU stand-ins of hip/hip_runtime.h, built with ThreadSanitizer by
 // tests/test_emu_xfer.py.  Test infrastructure only.
 //
-//   xfer_emu data | contexts
+//   xfer_emu data | contexts | pinned
 #include "sd2d_xfer.hpp"
 
 #include <chrono>
@@ -90,10 +90,30 @@ static void contexts() {
   CHECK(fake::pinned_bytes == 0);
 }
 
+// an array the copy engine reaches by itself is copied in one piece
+static void pinned() {
+  fake::Stream st;
+  RingUser u;
+  const size_t n = size_t(70) << 20;
+  std::vector<char> dev = pattern(n, 5);
+  void *p = nullptr;
+  CHECK(hipHostMalloc(&p, n, 0) == hipSuccess);
+  for (bool out : {true, false}) {
+    fake::ring_copies = 0;   // (counts every copy whose host side is pinned)
+    CHECK(HostRing::get().copy(&st, p, dev.data(), n, out) == hipSuccess);
+    CHECK(hipStreamSynchronize(&st) == hipSuccess);
+    CHECK(fake::ring_copies == 1 && fake::direct_copies == 0);
+    CHECK(std::memcmp(p, dev.data(), n) == 0);
+  }
+  CHECK(fake::pinned_bytes == n);
+  CHECK(hipHostFree(p) == hipSuccess);
+}
+
 int main(int argc, char **argv) {
   const std::string job = argc > 1 ? argv[1] : "";
   if (job == "data") data();
   else if (job == "contexts") contexts();
+  else if (job == "pinned") pinned();
   else return 2;
   return 0;
 }

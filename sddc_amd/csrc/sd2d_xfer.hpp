@@ -6,8 +6,8 @@
 // output array.  Here the copy engine writes into (reads from) a ring of
 // pinned slots while a few host threads move earlier (later) slots to (from)
 // the caller's array.  To the host, 472 MB: 45 -> 12.5 ms (10.4 -> 37.7 GB/s;
-// the link takes 57 GB/s into pinned memory), 29 MB: 1.75 -> 0.98 ms, 2.3 MB:
-// 0.20 ms either way; to the device, 472 MB: 16.4 -> 12.3 ms.
+// the link takes 57 GB/s into pinned memory), 29 MB: 1.75 -> 0.98 ms; to the
+// device, 472 MB: 16.4 -> 12.3 ms.
 //
 // The ring (32 MiB) is one per process, allocated by the first large copy and
 // freed with the last context.  A copy holds it alone: one that finds it
@@ -29,12 +29,12 @@ class HostRing {
  public:
   static constexpr int NSLOT_ = 16, LEAD = NSLOT_ / 2, MAXW = 8;
   static constexpr size_t SLOT = size_t(2) << 20;
-  // To the host below 1 MiB the runtime's copy costs as little as the ring's
-  // events; one host thread more per 2 MiB.  To the device the runtime's copy
-  // is the faster one up to some tens of MB (29 MB: 35 against 29 GB/s, 118 MB:
-  // 28 against 35).
-  static constexpr size_t MIN_OUT = size_t(1) << 20, MIN_IN = size_t(64) << 20;
-  static constexpr size_t MT_BYTES = size_t(3) << 20;
+  // To the host the runtime's copy is the faster one below 2.5 MiB (a state of 1.2
+  // MiB: 127 against 147 us, 1.9 MiB: 160 against 202) and as fast up to 4 MiB (3.2:
+  // 250 / 257, 4.0: 283 / 277, 4.8: 340 / 304, 7.8: 514 / 388); one host thread
+  // more per 2 MiB.  To the device it is the faster one up to some tens of MB
+  // (29 MB: 35 against 29 GB/s, 118 MB: 28 against 35).
+  static constexpr size_t MIN_OUT = size_t(4) << 20, MIN_IN = size_t(64) << 20;
 
   static HostRing &get() {
     static HostRing r;
@@ -80,15 +80,15 @@ class HostRing {
       e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
     std::thread th[MAXW];
     int nw = 0;
-    if (e == hipSuccess && bytes >= MT_BYTES) {
+    if (e == hipSuccess) {
       const int want = std::min({MAXW, (int)std::max(1u, std::thread::hardware_concurrency() / 2),
                                  1 + (int)std::min<size_t>(MAXW, bytes / SLOT)});
       try {
         for (; nw < want; ++nw) th[nw] = std::thread([&j] { j.work(); });
       } catch (...) {   // no thread to be had: go on with those that started
       }
+      e = nw ? drive(j, st, static_cast<char *>(dev), ev) : plain(st, host, dev, bytes, out);
     }
-    if (e == hipSuccess) e = drive(j, st, static_cast<char *>(dev), ev, nw);
     {
       std::lock_guard<std::mutex> lk(j.m);
       j.stop = true;
@@ -147,9 +147,8 @@ class HostRing {
     }
   };
 
-  // The copy engine's side of a job; with nw == 0 this thread moves the chunks
-  // as well.
-  static hipError_t drive(Job &j, hipStream_t st, char *dev, hipEvent_t *ev, int nw) {
+  // The copy engine's side of a job.
+  static hipError_t drive(Job &j, hipStream_t st, char *dev, hipEvent_t *ev) {
     hipError_t e = hipSuccess;
     auto dma = [&](int k) {
       char *r = j.ring + (size_t)(k % NSLOT_) * SLOT, *d = dev + (size_t)k * j.chunk;
@@ -157,33 +156,26 @@ class HostRing {
                            : hipMemcpyAsync(d, r, j.len(k), hipMemcpyHostToDevice, st);
       return x != hipSuccess ? x : hipEventRecord(ev[k % NSLOT_], st);
     };
-    auto moved = [&](int k) {   // the host's part of chunk k, done
-      if (nw) j.wait_moved(k);
-      else j.move(k);
-    };
     if (j.out) {
       for (int k = 0; k < std::min(LEAD, j.n); ++k)
         if ((e = dma(k)) != hipSuccess) return e;
       for (int k = 0; k < j.n; ++k) {
         if ((e = hipEventSynchronize(ev[k % NSLOT_])) != hipSuccess) return e;
-        if (nw) j.let(k + 1);
-        else j.move(k);
+        j.let(k + 1);
         const int a = k + LEAD;   // its slot's last chunk was LEAD chunks ago
         if (a < j.n) {
-          if (nw && a >= NSLOT_) j.wait_moved(a - NSLOT_);
+          if (a >= NSLOT_) j.wait_moved(a - NSLOT_);
           if ((e = dma(a)) != hipSuccess) return e;
         }
       }
-      if (nw)
-        for (int k = std::max(0, j.n - NSLOT_); k < j.n; ++k) j.wait_moved(k);
+      for (int k = std::max(0, j.n - NSLOT_); k < j.n; ++k) j.wait_moved(k);
     } else {
-      if (nw) j.let(std::min(LEAD, j.n));
+      j.let(std::min(LEAD, j.n));
       for (int k = 0; k < j.n; ++k) {
-        if (!nw && k >= NSLOT_ && (e = hipEventSynchronize(ev[k % NSLOT_])) != hipSuccess) return e;
-        moved(k);
+        j.wait_moved(k);
         if ((e = dma(k)) != hipSuccess) return e;
         const int a = k + LEAD;   // chunk a's slot was last read by chunk a - NSLOT_
-        if (nw && a < j.n) {
+        if (a < j.n) {
           if (a >= NSLOT_ && (e = hipEventSynchronize(ev[a % NSLOT_])) != hipSuccess) return e;
           j.let(a + 1);
         }

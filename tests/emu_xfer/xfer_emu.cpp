@@ -2,7 +2,7 @@
 // the CPU stand-ins of hip/hip_runtime.h, built with ThreadSanitizer by
 // tests/test_emu_xfer.py.  Test infrastructure only.
 //
-//   xfer_emu data | contexts | pinned
+//   xfer_emu data | contexts | pinned | small
 #include "sd2d_xfer.hpp"
 
 #include <chrono>
@@ -40,8 +40,8 @@ static std::vector<char> pattern(size_t n, unsigned seed) {
 static void data() {
   fake::Stream st;
   const size_t M = size_t(1) << 20;
-  for (size_t n : {size_t(1000), M - 8, M, M + 8, 3 * M - 8, 3 * M, 5 * M + 24, 17 * M + 8, 33 * M,
-                   64 * M, 67 * M + 40}) {
+  for (size_t n : {size_t(1000), M - 8, M, M + 8, 3 * M - 8, 3 * M, 4 * M - 8, 4 * M, 5 * M + 24,
+                   17 * M + 8, 33 * M, 64 * M, 67 * M + 40}) {
     RingUser u;
     std::vector<char> dev = pattern(n, 1), host(n);
     CHECK(HostRing::get().copy(&st, host.data(), dev.data(), n, true) == hipSuccess);
@@ -109,11 +109,29 @@ static void pinned() {
   CHECK(hipHostFree(p) == hipSuccess);
 }
 
+// below the sizes where the ring is the faster way, a copy is one of the runtime's
+static void small() {
+  fake::Stream st;
+  RingUser u;
+  const size_t M = size_t(1) << 20;
+  for (size_t n : {M, 2 * M, 3 * M + 8, 4 * M - 8}) {
+    std::vector<char> dev = pattern(n, 6), host(n);
+    for (bool out : {true, false}) {
+      fake::direct_copies = 0;
+      CHECK(HostRing::get().copy(&st, host.data(), dev.data(), n, out) == hipSuccess);
+      CHECK(hipStreamSynchronize(&st) == hipSuccess);
+      CHECK(fake::direct_copies == 1 && fake::ring_copies == 0);
+    }
+  }
+  CHECK(fake::pinned_bytes == 0);
+}
+
 int main(int argc, char **argv) {
   const std::string job = argc > 1 ? argv[1] : "";
   if (job == "data") data();
   else if (job == "contexts") contexts();
   else if (job == "pinned") pinned();
+  else if (job == "small") small();
   else return 2;
   return 0;
 }

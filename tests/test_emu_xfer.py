@@ -3,8 +3,8 @@
 tests/emu_xfer/xfer_emu.cpp compiles the header unchanged against stand-ins of
 the HIP calls it makes (a stream is a host thread that runs its operations in
 order) under ThreadSanitizer: whole copies at the sizes where the path changes,
-contexts that come and go while another thread's copy is under way, and pinned
-arrays of the caller's."""
+contexts that come and go while another thread's copy is under way, pinned arrays
+of the caller's, and copies too small for the ring."""
 import hashlib
 import os
 import shutil
@@ -35,7 +35,7 @@ def xfer_exe():
     return exe
 
 
-@pytest.mark.parametrize("job", ["data", "contexts", "pinned"])
+@pytest.mark.parametrize("job", ["data", "contexts", "pinned", "small"])
 def test_ring(xfer_exe, job):
     r = subprocess.run([xfer_exe, job], capture_output=True, text=True, timeout=300,
                        env=dict(os.environ, TSAN_OPTIONS="halt_on_error=1"))

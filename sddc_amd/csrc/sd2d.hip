@@ -49,6 +49,8 @@ struct sd2d_ctx {
   double *fsr[4] = {nullptr, nullptr, nullptr, nullptr};  // FiveStageRk registers
   double *met = nullptr;
   int mcomp = 0;                                // met (and metf) in the compact form
+  int ncu = 0;                                  // compute units of the device
+  bool pt = false;                              // stages by stage_pt_kernel (small meshes)
   int *ftab = nullptr;
   int *c2s = nullptr, *s2c = nullptr;          // cell <-> slot maps of the tile shape
   double avf[NMAX * NMAX] = {};               // AV smoothing filter (kernel arguments)
@@ -332,8 +334,6 @@ static hipError_t launch_stage_mx_t(sd2d_ctx *c, const StageArgs &a) {
   return hipGetLastError();
 }
 
-constexpr int NCU = 256;   // compute units of an MI355X
-
 template <int N, int MODE>
 static hipError_t launch_stage_pt_t(sd2d_ctx *c, const StageArgs &a) {
   constexpr size_t lds = stage_pt_lds_bytes<N, MODE>();
@@ -349,9 +349,7 @@ static hipError_t launch_stage_t(sd2d_ctx *c, const StageArgs &a) {
     if (c->p.precision == SD2D_MIXED) return launch_stage_mx_t<N, MODE>(c, a);
   }
   if constexpr (pt_mode(MODE)) {
-    // one workgroup per CU or fewer: 9 % faster at 128 tiles, 10 at 256, 16 %
-    // slower at 342 (sd2d_stage_pt.hpp)
-    if (c->ntile <= NCU) return launch_stage_pt_t<N, MODE>(c, a);
+    if (c->pt) return launch_stage_pt_t<N, MODE>(c, a);
   }
   constexpr size_t lds = stage_lds_bytes<N, MODE>();
   static_assert(lds <= 65536, "stage kernel LDS above 64 KiB");
@@ -564,6 +562,11 @@ static int ctx_upload(sd2d_ctx *c, const HostTables &tb, int nwall, int nmem,
     c->sfam = cross[0] < cross[1] ? 0 : 1;
   }
   CK(hipGetDevice(&c->device));
+  CK(hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, c->device));
+  // one workgroup per CU or fewer, us a stage with the line kernel and with the
+  // point one: 128 tiles, N = 3, 4, 5: 8.3 / 9.5 / 11.3 and 7.2 / 8.2 / 9.7; 256: 8.6 /
+  // 10.2 / 12.0 and 7.6 / 8.9 / 10.6; 288: 10.6 / 12.7 / 15.4 and 10.3 / 14.3 / 17.6
+  c->pt = nt <= c->ncu;
   scratch_init(c->device);
   CK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   const size_t qn = (size_t)nt * 9 * N2 * CPW;

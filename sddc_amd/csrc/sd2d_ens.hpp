@@ -74,6 +74,27 @@ static void ens_free_group(sd2d_ens *e, int g) {
 // between steps, whether a graph or direct launches ran the step.
 static void ens_sync_cur(const sd2d_ens *e, sd2d_ctx *c) { c->cur = c->mset = e->cur; }
 
+// The stage kernel of each group.  The groups of a step share the chip, so a group
+// of at most one tile per CU takes the form of small meshes (sd2d_stage_pt.hpp,
+// a third to half of a CU's LDS per tile) only where all groups together have 7/4
+// tiles per CU or fewer, or where such groups leave the others half the CUs.  us
+// a stage, all groups with the line kernel against the small ones with the point
+// kernel (256 CUs; tiles of N = 3 + 4 + 5): 128 + 128 + 128 22.3 / 20.7, 0 + 192 + 192
+// 19.7 / 19.2, 224 + 224 + 0 17.8 / 17.0, 0 + 224 + 224 20.0 / 20.3, 176 + 176 + 176
+// 22.7 / 23.1, 0 + 256 + 256 20.3 / 21.5, 256 + 256 + 256 22.3 / 28.6; beside a larger
+// group 0 + 1024 + 128 26.6 / 25.4, 64 + 1024 + 0 25.5 / 24.8, 96 + 96 + 640 26.0 / 27.1,
+// 192 + 640 + 256 25.6 / 30.1.
+static void ens_choose_kernels(sd2d_ens *e) {
+  int all = 0, small = 0;
+  for (const sd2d_ctx *c : e->grp) {
+    if (!c) continue;
+    all += c->ntile;
+    if (c->ntile <= c->ncu) small += c->ntile;
+  }
+  for (sd2d_ctx *c : e->grp)
+    if (c) c->pt = c->ntile <= c->ncu && (4 * all <= 7 * c->ncu || 2 * small <= c->ncu);
+}
+
 // (Re)build group g with tile shape `shape`: host tables of every member,
 // concatenated, uploaded into a fresh context.  Member states are not kept.
 static int ens_build_group(sd2d_ens *e, int g, int shape, bool full_metrics = false) {
@@ -162,6 +183,7 @@ static int ens_build_group(sd2d_ens *e, int g, int shape, bool full_metrics = fa
     ++k;
   }
   ens_sync_cur(e, c);
+  ens_choose_kernels(e);
   e->grp_shape[g] = shape;
   return SD2D_OK;
 }

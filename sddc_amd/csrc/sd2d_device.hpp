@@ -170,6 +170,13 @@ __device__ __forceinline__ double rcp(double x) {
 }
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
+// a / x with ri = rcp(x) and one correction, as accurate as the division (the
+// plain product a * ri has twice its error).
+__device__ __forceinline__ double quot(double a, double x, double ri) {
+  const double q = a * ri;
+  return fma(fma(-x, q, a), ri, q);
+}
+
 // Gas pressure (gamma-1)*(E - |m|^2/(2 rho) - |B|^2/2 - psi^2/2), the
 // recovery that cancels at low plasma beta.  The FP64 path keeps the
 // operation order of each caller (iflux_n, rusanov); the mixed path

@@ -114,9 +114,9 @@ __device__ __forceinline__ void vis_end_state(int info, const Phys &ph, const do
 // it (compflux.f90:275-280).
 __device__ __forceinline__ double enei_of(const double *q) {
   const double ri = rcp(q[0]);
-  const double u = q[1] * ri, v = q[2] * ri, w = q[3] * ri;
-  return (((q[4] * ri - 0.5 * (u * u)) - 0.5 * (v * v)) - 0.5 * (w * w)) -
-         0.5 * (((q[5] * q[5] + q[6] * q[6]) + q[7] * q[7]) + q[8] * q[8]) * ri;
+  const double u = quot(q[1], q[0], ri), v = quot(q[2], q[0], ri), w = quot(q[3], q[0], ri);
+  return (((quot(q[4], q[0], ri) - 0.5 * (u * u)) - 0.5 * (v * v)) - 0.5 * (w * w)) -
+         quot(0.5 * (((q[5] * q[5] + q[6] * q[6]) + q[7] * q[7]) + q[8] * q[8]), q[0], ri);
 }
 
 // nablaQsp (compflux.f90:107-157) and, on tiles with walls,
@@ -304,20 +304,20 @@ __device__ __forceinline__ void vflux_n(const double *Qv, const double *g, doubl
   const double rho = Qv[0], rhoE = Qv[4];
   const double Bx = Qv[5], By = Qv[6], Bz = Qv[7], psi = Qv[8];
   const double ri = rcp(rho);
-  const double u = Qv[1] * ri, v = Qv[2] * ri, w = Qv[3] * ri;
+  const double u = quot(Qv[1], rho, ri), v = quot(Qv[2], rho, ri), w = quot(Qv[3], rho, ri);
   const double nu = u * u + v * v + w * w;
   const double nb = Bx * Bx + By * By + Bz * Bz;
-  const double inte = (rhoE - 0.5 * nu * rho - 0.5 * nb - 0.5 * (psi * psi)) * ri;
+  const double inte = quot(rhoE - 0.5 * nu * rho - 0.5 * nb - 0.5 * (psi * psi), rho, ri);
   double du[2], dv[2], dw[2], de[2];
 #pragma unroll
   for (int d = 0; d < 2; ++d) {
     const double dr = g[d];
-    du[d] = (g[2 + d] - dr * u) * ri;
-    dv[d] = (g[4 + d] - dr * v) * ri;
-    dw[d] = (g[6 + d] - dr * w) * ri;
+    du[d] = quot(g[2 + d] - dr * u, rho, ri);
+    dv[d] = quot(g[4 + d] - dr * v, rho, ri);
+    dw[d] = quot(g[6 + d] - dr * w, rho, ri);
     const double dke = 0.5 * nu * dr + rho * (u * du[d] + v * dv[d] + w * dw[d]);
     const double dpb = Bx * g[10 + d] + By * g[12 + d] + Bz * g[14 + d];
-    de[d] = (g[8 + d] - dke - dpb - dr * inte - psi * g[16 + d]) * ri;
+    de[d] = quot(g[8 + d] - dke - dpb - dr * inte - psi * g[16 + d], rho, ri);
   }
   const double ux = du[0], uy = du[1], vx = dv[0], vy = dv[1], wx = dw[0], wy = dw[1];
   constexpr double KP = GAM / PRANDTL;
@@ -347,14 +347,15 @@ __device__ __forceinline__ void vflux_n(const double *Qv, const double *g, doubl
 __device__ __forceinline__ void wall_grad_ghost(const double *Qo, const double *gl, double dface,
                                                 double ox, double oy, double *gr4) {
   const double ri = rcp(Qo[0]);
-  const double ur = Qo[1] * ri, vr = Qo[2] * ri, wr = Qo[3] * ri;
+  const double ur = quot(Qo[1], Qo[0], ri), vr = quot(Qo[2], Qo[0], ri),
+               wr = quot(Qo[3], Qo[0], ri);
   const double inte = enei_of(Qo);
   const double dBp = ((Qo[5] * gl[10] + Qo[6] * gl[12]) + Qo[7] * gl[14]) + Qo[8] * gl[16];
 #pragma unroll
   for (int d = 0; d < 2; ++d) {
-    const double dur = (gl[2 + d] - ur * gl[d]) * ri;
-    const double dvr = (gl[4 + d] - vr * gl[d]) * ri;
-    const double dwr = (gl[6 + d] - wr * gl[d]) * ri;
+    const double dur = quot(gl[2 + d] - ur * gl[d], Qo[0], ri);
+    const double dvr = quot(gl[4 + d] - vr * gl[d], Qo[0], ri);
+    const double dwr = quot(gl[6 + d] - wr * gl[d], Qo[0], ri);
     const double dKE = 0.5 * ((ur * ur + vr * vr) + wr * wr) * gl[d] +
                        Qo[0] * ((ur * dur + vr * dvr) + wr * dwr);
     gr4[d] = (((-gl[8 + d] + 2.0 * inte * gl[d]) + 2.0 * dKE) + dBp) +

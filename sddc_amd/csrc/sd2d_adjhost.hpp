@@ -6,9 +6,9 @@
 // keeps a checkpoint (state and running maxima) every `ckpt` steps.
 // sd2d_vjp runs backwards over the checkpoint segments: a segment's step
 // inputs are recomputed from its checkpoint, then each step's five stage
-// inputs and the GLM maxima before each stage are recomputed with the very
-// kernels of the forward run (bitwise the same states), and the step is
-// reversed stage by stage:
+// inputs and the GLM maxima before each stage are recomputed by the line kernel
+// with M_TRACE (the forward's states bit for bit, whichever form of the stage
+// kernel it took), and the step is reversed stage by stage:
 //   Q1 = Q0 + b10 dt R(Q0)            Q0bar += Q1bar + (dR/dQ0)^T b10 dt Q1bar
 //   Q2 = Q1 + b21 dt R(Q1)            ...
 //   Q3 = a30 Q0 + a32 Q2 + b32 dt R(Q2)

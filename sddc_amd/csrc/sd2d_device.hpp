@@ -404,6 +404,7 @@ __device__ __forceinline__ void rusanov<double>(const double *QL, const double *
 template <typename T>
 __device__ __forceinline__ void bc_ghost_p(int bc, const T *Ql, T nx, T ny, T rinf, T pinf,
                                            T ui, T vi, T bxi, T byi, int vismode, T *Qr) {
+#pragma clang fp contract(on)   // as iflux_n<double>: the same bits in every kernel
   const T g1 = T(GAM - 1.0);
   const T ri = rcp(Ql[0]);
   const T uw = Ql[1] * ri, vw = Ql[2] * ri, ww = Ql[3] * ri;

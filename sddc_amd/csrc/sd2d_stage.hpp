@@ -257,6 +257,7 @@ __device__ __forceinline__ void av_sensor_lines(const StageArgs &a, const double
                                                 const double *jz2, double *lineb,
                                                 const double (&rs)[N], const double (&js2)[N],
                                                 int line, int ci, int cell, bool valid) {
+#pragma clang fp contract(on)   // as iflux_n<double>
   wave_lds_sync();   // the cell's Jz^2 (and rho) of the other lines are in LDS
   double e1 = 0.0, e2 = 0.0;
   if (valid) {

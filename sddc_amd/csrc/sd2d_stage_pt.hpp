@@ -1,7 +1,8 @@
 // sd2d_stage_pt.hpp - the stage kernel of meshes too small to fill the chip.
 //
-// The same tiles, arithmetic and results as stage_kernel (bit for bit: a run
-// made alone and as a member of a large ensemble agree), split finer: one
+// The same tiles and arithmetic as stage_kernel, and the same state, maxima and
+// sensor bit for bit (a run made alone and as a member of a large ensemble agree;
+// the norms are summed in another order), split finer: one
 // wavefront per (line family, flux-point number), so a thread forms the flux of
 // one flux point of one line, then one thread per solution point and half of
 // its variables.  With less than one tile per CU the line

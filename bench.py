@@ -390,7 +390,8 @@ def main() -> int:
     ms, nlaunch = g.get_profile()
     g.set_profiling(False)
     avg_s = ms / 1e3 / max(nlaunch, 1)
-    balg = cases.alg_bytes_per_dof_stage(N, case.params.k_stage, lines_share=True)
+    share = cases.lines_share_metrics(case)
+    balg = cases.alg_bytes_per_dof_stage(N, case.params.k_stage, lines_share=share)
     achieved = ndof * balg / avg_s / 1e9
     d = g.diag()
     nsteps_done = args.warmup + 2 * args.steps
@@ -449,7 +450,7 @@ def main() -> int:
         l2 = np.sqrt(((a - b) ** 2).sum(axis=1)) / den
         avg_m = ms_m / 1e3 / max(n_m, 1)
         balg_m = cases.alg_bytes_per_dof_stage(N, case.params.k_stage, metric_bytes=4,
-                                                lines_share=True)
+                                                lines_share=share)
         vm = ndof * 5 * args.steps / wall_m
         res["mixed"] = {
             "value": vm, "unit": "DOF-stage/s", "ms_per_step": wall_m / args.steps * 1e3,

@@ -152,13 +152,21 @@ def dof(case: M.Case) -> int:
     return case.ncell * case.N * case.N
 
 
+def lines_share_metrics(case: M.Case) -> bool:
+    """Whether the face-normal metric vectors are, bit for bit, the same on
+    every line of a family in every cell, as on 4-node cells: the library
+    then keeps (and a stage reads) one vector per flux-point position."""
+    s1, s2 = case.s1[0].view(np.int64), case.s2[1].view(np.int64)
+    return bool((s1[:, :, 1:] == s1[:, :, :1]).all() and (s2[:, 1:] == s2[:, :1]).all())
+
+
 def alg_bytes_per_dof_stage(N: int, k_stage: int = 3, metric_bytes: int = 8,
                             lines_share: bool = False) -> float:
     """Compulsory HBM bytes per DOF-stage of a fused stage: the RK state
     traffic (RK_S5P3: 13 state passes of 72 B over 5 stages; FiveStageRk:
     18 + the stored residual) plus Jac and the face-normal metric vectors
-    S1(1,:), S2(2,:) read once per stage; with lines_share (4-node cells)
-    the N+1 vectors that the N lines of a family share."""
+    S1(1,:), S2(2,:) read once per stage; with lines_share (see
+    lines_share_metrics) the N+1 vectors that the N lines of a family share."""
     state = 13 * 72 / 5 if k_stage == 3 else 18 * 72 / 5
     metrics = metric_bytes * (N * N + 4 * (1 if lines_share else N) * (N + 1)) / (N * N)
     return state + metrics

@@ -333,14 +333,14 @@ __device__ __forceinline__ double adj_divb_cot(const double *q, const double *rb
            rb[4] * (ux * q[5] + uy * q[6] + uz * q[7]) + rb[5] * ux + rb[6] * uy + rb[7] * uz);
 }
 
-// From the line of another cell through a shared face point (points p0 + ps*s
-// of slot ci, state q and cotangent r in qo layout, 1/J at ji): the state's
-// trace t with row Lr, and the cotangents of that cell's flux and divB weight
-// there, Mr^T Dbar and Mr^T wbar.
 // (is, js) of a solution point
 template <int N> __device__ __forceinline__ int pt_is(int p) { return p % N; }
 template <int N> __device__ __forceinline__ int pt_js(int p) { return p / N; }
 
+// From the line of another cell through a shared face point (points p0 + ps*s
+// of slot ci, state q and cotangent r in qo layout, 1/J at ji): the state's
+// trace t with row Lr, and the cotangents of that cell's flux and divB weight
+// there, Mr^T Dbar and Mr^T wbar.
 template <int N>
 __device__ __forceinline__ void adj_far_line(const double *q, const double *r, const double *ji,
                                              int p0, int ps, int ci, const double *Lr,
@@ -486,13 +486,12 @@ __global__ __launch_bounds__(STAGE_THREADS, 1) void adj_stage_kernel(AdjArgs a, 
       });
     };
     auto end_point = [&](bool atN, bool gathered, double *Qt) __attribute__((always_inline)) {
-      const int rfp = atN ? N : 0, info = atN ? infoN : info0;
+      const int info = atN ? infoN : info0;
       const int k = fam == 0 ? (atN ? 1 : 3) : (atN ? 2 : 0);
       const bool inter = atN ? iN : i0, far = atN ? farN : far0;
       const double sx = atN ? msx[N] : msx[0], sy = atN ? msy[N] : msy[0];
       if (inter && !far) other_side(atN, true);
       else if (far && !gathered) other_side(atN, false);
-      (void)rfp;
       double Lo[N], Mo[N], t[9], Fb[9], Wb;
 #pragma unroll
       for (int s = 0; s < N; ++s) {

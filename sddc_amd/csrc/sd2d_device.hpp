@@ -94,9 +94,9 @@ inline int qo_rt(int N, int v, int p, int ci) {
 // table).  A cell then has 49 metric values instead of 145 at N = 5, 16 % of
 // the bytes of a stage without an RK register, and the lanes of one load touch
 // one run of cells instead of N.
-// Stages of 512 x 1024 cells, N = 5: 691 / 791 / 826 -> 673 / 750 / 795 us
-// (none, one RK register, with the sensor); 512 x 512, N = 4, mixed: 189 / 228 /
-// 236 -> 184 / 222 / 230 us.
+// Stages of 512 x 1024 cells, N = 5: 671 / 764 / 810 -> 655 / 725 / 777 us (none, one
+// RK register, with the sensor); 512 x 512, N = 4, mixed: 194 / 232 / 235 ->
+// 188 / 226 / 229 us.
 template <int N, typename R> struct MetLine {
   static constexpr int T = cpw_of(N), NF = N + 1;
   const R *x, *y;   // the line's metric vector at flux point r: x[r*T], y[r*T]

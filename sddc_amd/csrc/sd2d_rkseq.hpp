@@ -1,6 +1,6 @@
 // sd2d_rkseq.hpp - the stage sequences of the two Runge-Kutta schemes
-// (host side; `launch(args, mode)` runs one stage kernel and the
-// running-maximum update).  The state rotates through three buffers so no
+// (host side; `launch(args, mode)` runs one stage kernel and moves on to the next
+// set of running maxima).  The state rotates through three buffers so no
 // copy is made; FiveStageRk keeps its registers qj2, qj3, resid0 in three
 // more.
 #pragma once

@@ -51,8 +51,9 @@ struct StageArgs {
   int mcomp;                // met is the compact table (MetLine)
   const int *ftab;          // per-cell face table (tile layout)
   // the running maxima before this evaluation, to raise and to clear (MSTRIDE
-  // per member); or, mread null (an evaluation outside the sequence), the pair
-  // to form c_h from and NSLOT x 2 slots to raise (none by M_DIVB)
+  // per member); or, mread null (an evaluation outside the sequence, in the
+  // library M_DIVB, which raises none), the pair to form c_h from and NSLOT x 2
+  // slots to raise
   const unsigned long long *mread;
   unsigned long long *mwrite, *mclear;
   const double *gmax;
@@ -221,8 +222,9 @@ __device__ __forceinline__ void lagged_maxima(const StageArgs &a, int ti, int ti
 // their wait at the end of every workgroup are gone.
 // 512 x 1024 cells, N = 5, stages without and with an RK register: one atomic
 // per tile and value on 256 addresses 720 / 824 us, on 64 addresses 831 / 920,
-// only where a tile raises a maximum 701 / 801; and without the reduction over
-// the workgroup (compact metrics on both sides) 703 / 776 -> 687 / 746.
+// only where a tile raises a maximum 701 / 801.  The reduction over the workgroup
+// cost 2 to 4 % (703 / 776 -> 687 / 746, compact metrics on both sides, one device;
+// devices differ by as much).
 __device__ __forceinline__ void raise_maxima(const StageArgs &a, int mem, double e, double u,
                                              double me, double mu) {
   if (!a.mread) {
@@ -428,12 +430,6 @@ __device__ __forceinline__ void neighbour_line(int kn, int nfp, int &p0, int &st
   endN = (kn == 1 || kn == 2);
 }
 
-// Gather for an end face: the face-table info word and, for an interior or
-// periodic face, the neighbour's trace Qn at the shared face point (its
-// line through that point, interpolated with the same arithmetic as the
-// own trace: interfaceflux_all.f90:59-76).  When the neighbour cell is in
-// the same tile, nothing is read here: lci returns its index in the tile
-// and the trace is formed from the staged tile by face_trace_lds.
 // The face-table words (neighbour base, info) of end face `rfp` of a line.
 // (A is StageArgs, or another kernel's arguments with the same ftab and, for
 // the gathers, qin.)
@@ -454,7 +450,11 @@ __device__ __forceinline__ void face_words(const A &a, int tile, int ci, int fam
 // lanes that need both.  In a wave whose lanes need at most one gather each
 // (a line family whose neighbours are mostly in the tile: only the lanes of
 // the strip's end cells gather) pass 2 is skipped, which halves its gather
-// loads.  Each face's trace is formed exactly as by face_gather_w.
+// loads.  A gathered trace Qn is the neighbour's at the shared face point: its
+// line through that point, interpolated with the arithmetic of the own trace
+// (interfaceflux_all.f90:59-76).  When the neighbour cell is in the same tile,
+// nothing is read here: lci returns its index in the tile and face_trace_lds
+// forms the trace from the staged tile.
 template <int N, typename R, typename A, typename OP>
 __device__ __forceinline__ void face_gather_pair(const A &a, const OP &ops, int tile,
                                                  int fam, int line, int nb0, int info0, int nbN,
@@ -491,7 +491,7 @@ __device__ __forceinline__ void face_gather_pair(const A &a, const OP &ops, int 
 }
 
 // The neighbour's trace for a neighbour in the same tile, from the staged
-// tile (the same values and arithmetic as face_gather).
+// tile (the same values and arithmetic as face_gather_pair).
 template <int N, typename R, typename OP>
 __device__ __forceinline__ void face_trace_lds(const R *qs, const OP &ops, int info, int fam,
                                                int line, int rfp, int lci, R *Qn) {

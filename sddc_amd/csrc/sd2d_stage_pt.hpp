@@ -22,7 +22,7 @@
 // more than one tile per CU it loses: 342 tiles, N = 5: 19.0 against 16.3; 512
 // tiles, N = 4: 16.7 against 14.8; 8192 tiles, N = 4: 236 against 127.
 // 20 steps of 32 x 64 cells, N = 4, with the state's download: 1384 -> 1276 us; a
-// step of 13 x 9 cells, N = 3, by host stages: 191 -> 172 us.
+// step of 13 x 9 cells, N = 3, by host stages and downloads: 140 us.
 #pragma once
 #include "sd2d_stage.hpp"
 

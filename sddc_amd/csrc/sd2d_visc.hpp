@@ -131,9 +131,9 @@ __device__ __forceinline__ double enei_of(const double *q) {
 // after the barrier adds the two, scales by 1/J and stores both components
 // as one 16-byte word.  The xi-lines finish variables 0-3 and d(psi)/dx, the
 // eta-lines 4-7 and d(psi)/dy, so both waves store half.
-// Bound by the L2 and the loads in flight (2 waves per SIMD: 182-210 VGPRs,
-// 31-41 KB of LDS).  128 x 256 cells, N = 5: 63 us, 3.0 TB/s of its compulsory
-// 232 bytes a point; N = 4: 33 us.  The form before it, which read every
+// Bound by the L2 and the loads in flight (2 waves per SIMD, 3 at N = 3: 158-210
+// VGPRs, 31-41 KB of LDS).  128 x 256 cells, N = 5: 62 us, 3.1 TB/s of its compulsory
+// 232 bytes a point; N = 4: 33 us, N = 3: 21 us.  The form before it, which read every
 // flux point's line and neighbour from memory (12 reads of the tile, one
 // 8-byte word at a time) and let one family store everything: 259 and 115 us.
 template <int N>
@@ -299,6 +299,9 @@ __global__ __launch_bounds__(STAGE_THREADS, 2) void vis_grad_kernel(VisArgs va, 
 // vector (sx, sy): Fn[k] = Fv[k+1]*sx + Gv[k+1]*sy for variables 1-7 (the
 // fluxes of rho and psi are zero; compflux.f90:215-216,243-244).
 // g[2v] is d(q_v)/dx, g[2v+1] is d(q_v)/dy.
+// The quotients by rho share one reciprocal and are corrected (quot): plain
+// products with it put the momentum components 8-11 % further from the exact flux
+// than divisions do (rms over random states) and saved at most 1 % of a step.
 __device__ __forceinline__ void vflux_n(const double *Qv, const double *g, double mu,
                                         double eta, double sx, double sy, double *Fn) {
   const double rho = Qv[0], rhoE = Qv[4];
@@ -408,10 +411,11 @@ __device__ __forceinline__ void grad_trace(const double *vals, const double *Lr,
 // families exchange: the xi-lines finish variables 1-3, the eta-lines 4-7.
 // Two waves per SIMD (193-254 VGPRs, 26-43 KB of LDS); bound by the vector
 // memory and LDS pipes together (95 16-byte loads and 180 LDS reads a thread
-// at N = 5), then by FP64 issue.  128 x 256 cells, N = 5: 111 us; with one
+// at N = 5), then by FP64 issue.  128 x 256 cells, N = 5: 109 us; with one
 // thread per line (both ends and all interior points: 376 registers, one wave
 // per SIMD) 133 us; when every flux point read its lines from memory, 406 us.
-// N = 4 (151 x 90): 34 / 35 / 108 us, N = 3 (128 x 256): 46 / 44 / 153 us.
+// N = 4 (151 x 90): 35 / 35 / 108 us, N = 3 (128 x 256): 47 / 44 / 153 us
+// (this form with uncorrected quotients: 111, 34 and 46 us).
 // All flux points' gradient traces in one pass over LDS spill (660 bytes a
 // lane at N = 5).
 constexpr int VIS_FLUX_THREADS = 256;

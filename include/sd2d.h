@@ -388,7 +388,9 @@ int sd2d_ens_nonfinite(sd2d_ens *ens, int32_t *flags);
  *               the boundary ghosts read, or NULL).  The lagged GLM speed
  *               c_h of every evaluation is differentiated through the
  *               running maxima it comes from, back to the flux point that
- *               attained each maximum; chbar (5*nsteps entries, or NULL)
+ *               attained each maximum (one that the caller set apart with
+ *               sd2d_set_state is a constant); chbar (5*nsteps entries, or
+ *               NULL)
  *               returns the cotangent of each evaluation's c_h.  The
  *               context returns to the final state of sd2d_fwd.
  * sd2d_compresid_vjp  for the residual of the current state with the
